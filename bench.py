@@ -68,6 +68,14 @@ def log(msg):
     print(f"[bench {time.strftime('%H:%M:%S')}] {msg}", file=sys.stderr, flush=True)
 
 
+def transform_len(info):
+    """Length the FFT passes run at: compiled passes take half of the planned
+    length unless it is the spectrum's own period (2 N_v)."""
+    L, n1, n2 = int(info.fft_len), int(info.n1), int(info.n2)
+    half = info.compiled_fft and L != 2 * int(info.n_v) and (n1 >= 512 or n2 >= 128)
+    return L // 2 if half else L
+
+
 def stage_bytes(n_lines, info, db):
     """Algorithmic HBM bytes per launch of each kernel of one request.
 
@@ -81,10 +89,11 @@ def stage_bytes(n_lines, info, db):
     fft_a       : 4*M*(N_v+1) LDM read + 8*P*L packed-row spectra write
     fft_b       : 8*P*L read + 8*L write
     fft_c       : 8*L read + 4*N_v abscoeff write
+    with L the length the passes run at (transform_len).
     """
     M = int(info.n_g * info.n_l)
     P = (M + 1) // 2
-    L = int(info.fft_len)
+    L = transform_len(info)
     V = int(info.n_v) + 1
     ns = 4 if db.has_nself else 0
     per_fill = 28 + ns + (4 if db.has_delta else 0) + (1 if db.has_iso else 0)

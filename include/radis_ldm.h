@@ -130,7 +130,9 @@ typedef struct {
  * L = 2*N_v (radis/lbl/broadening.py:1900-1902, 2340-2346).  Without this
  * flag a transform longer than 2*N_v has its circular images corrected
  * (image-correction items in the fill launch), so the output is the L = 2*N_v
- * result whatever fft_len is; an
+ * result whatever fft_len is.  The compiled passes then run at fft_len / 2,
+ * a period just above N_v, and its images are corrected from a coarse
+ * description (the result is the same L = 2*N_v one to FP32 rounding); an
  * explicit fft_len must then be 2*N_v itself or leave a gap the correction
  * can span (about 0.5 % of L). */
 #define RADIS_LDM_PERIOD_L 64

@@ -14,6 +14,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "radis_ldm.h"
@@ -170,6 +171,7 @@ struct LaunchGroup {
   int cls, first, count;
   int rows;  // pass B: the rows' coefficients staged in LDS (the largest m_cap of the group, at most FC_B_ROWS_LDS)
   int wh;    // pass B: L-axis nodes of the image-correction values staged in LDS (largest wrap_rows, 0: none)
+  int img_first, img_count;  // pass B: half-length transforms' correction cells (image items)
 };
 
 struct radis_ldm_batch {
@@ -196,13 +198,14 @@ struct radis_ldm_batch {
   size_t tw_bytes = 0;
   int4* items_d = nullptr;
   size_t items_bytes = 0;
-  int n_axis = 0, n_wrap = 0, n_fill = 0, n_a = 0, n_b = 0, n_c = 0;
+  int n_axis = 0, n_wrap = 0, n_fill = 0, n_a = 0, n_b = 0, n_c = 0, n_img = 0;
   // launches of the FFT passes (see LaunchGroup)
   using Group = LaunchGroup;
   std::vector<Group> grp_a, grp_b, grp_c;
   bool tiles_valid = false;  // fill tile bounds computed for the current layout
   size_t fill_lds = 0;
   bool fill_grouped = false;  // some request fills its tiles in row groups
+  bool fill_half = false;     // some request runs half-length transforms
   std::vector<float*> outs;        // outputs of the last eager run
   std::vector<float*> graph_outs;  // outputs bound to the captured graph
   hipEvent_t ev_done[2] = {nullptr, nullptr};
@@ -223,6 +226,9 @@ struct radis_ldm_batch {
 
 namespace {
 
+// LDS behind a fill tile for its moments
+size_t fill_moment_bytes(const Req& R) { return R.half ? (size_t)tile_moment_lds(R.m_cap, R.tile_w) : 0; }
+
 void free_layout(radis_ldm_batch* b) {
   if (b->gexec) { (void)hipGraphExecDestroy(b->gexec); b->gexec = nullptr; }
   if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
@@ -239,13 +245,14 @@ int build_layout(radis_ldm_batch* b) {
   // --- workspace
   size_t total = 0;
   size_t fill_lds = 0;
-  bool fill_grouped = false;
+  bool fill_grouped = false, fill_half = false;
   choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu);
   for (Req& R : b->reqs) {
     int rc = layout_request(R, total);
     if (rc) return rc;
-    fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w));
+    fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R));
     fill_grouped = fill_grouped || R.fill_groups > 1;
+    fill_half = fill_half || R.half;
   }
   // --- twiddle tables, deduplicated by size
   std::map<int, size_t> sub_off;
@@ -254,11 +261,11 @@ int build_layout(radis_ldm_batch* b) {
   sub_off[LDM_WRAP_LC] = twsz;  // the image correction's transform
   twsz = align_up(twsz + (size_t)LDM_WRAP_LC * 8, 256);
   for (Req& R : b->reqs) {
-    for (int N : {R.plan.n1, R.plan.n2})
+    for (int N : {R.tn1, R.tn2})
       if (!sub_off.count(N)) { sub_off[N] = twsz; twsz = align_up(twsz + (size_t)N * 8, 256); }
-    if (!l_off.count(R.plan.L)) {
-      l_off[R.plan.L] = twsz;
-      const size_t nhi = (size_t)((R.plan.L + 1023) >> LDM_TW_LO_BITS);
+    if (!l_off.count(R.tL)) {
+      l_off[R.tL] = twsz;
+      const size_t nhi = (size_t)((R.tL + 1023) >> LDM_TW_LO_BITS);
       twsz = align_up(twsz + (nhi + 1024) * 8, 256);
     }
   }
@@ -287,24 +294,25 @@ int build_layout(radis_ldm_batch* b) {
   HIPCHK(hipGetLastError());
   for (Req& R : b->reqs) {
     char* base = (char*)b->twmem;
-    R.tw1 = (const float2*)(base + sub_off[R.plan.n1]);
-    R.tw2 = (const float2*)(base + sub_off[R.plan.n2]);
-    R.twl_hi = (const float2*)(base + l_off[R.plan.L]);
-    R.twl_lo = R.twl_hi + (size_t)((R.plan.L + 1023) >> LDM_TW_LO_BITS);
+    R.tw1 = (const float2*)(base + sub_off[R.tn1]);
+    R.tw2 = (const float2*)(base + sub_off[R.tn2]);
+    R.twl_hi = (const float2*)(base + l_off[R.tL]);
+    R.twl_lo = R.twl_hi + (size_t)((R.tL + 1023) >> LDM_TW_LO_BITS);
     R.tw_wrap = (const float2*)(base + sub_off[LDM_WRAP_LC]);
   }
   // --- work items (FFT passes grouped by kernel variant), per request in
   // the order plan_item gives them
   std::vector<int4> ax, fi, wr;
-  std::map<int, std::vector<int4>> ma, mb, mc;
+  std::map<int, std::vector<int4>> ma, mb, mc, mi;
   std::map<int, int> mb_rows, mb_wh;  // pass B class -> largest m_cap, largest wrap_rows
   for (int j = 0; j < b->n; ++j) {
     Req& R = b->reqs[j];
     const LdmItemPlan P = item_plan(*b->db, R);
     const int nax = P.n_lo + P.n_g + P.n_hi, bw = nax, bf = bw + P.n_wrap, ba = bf + P.n_fill;
     const int bb = ba + P.pcap * P.n_colA, bc = bb + P.n_rowB, be = bc + P.n_colC;
-    const int ca_ = R.plan.fc ? R.plan.n1 : 0;
-    const int cb_ = R.plan.fc ? R.plan.n2 : (R.plan.n2 <= LDM_CAP_B ? 0 : -1);
+    const int ca_ = R.plan.fc ? R.tn1 | (R.narrow_a ? FC_NARROW : 0) : 0;
+    const int cc_ = (R.plan.fc ? R.tn1 | (R.narrow_c ? FC_NARROW : 0) : 0) | (R.n_share > 1 ? FC_C_SUM : 0);
+    const int cb_ = R.plan.fc ? R.tn2 : (R.plan.n2 <= LDM_CAP_B ? 0 : -1);
     auto put = [&](std::vector<int4>& v, int a, int e) {
       for (int i = a; i < e; ++i) {
         int4 t = plan_item(P, i);
@@ -318,21 +326,26 @@ int build_layout(radis_ldm_batch* b) {
     put(ma[ca_], ba, bb);
     put(mb[cb_], bb, bc);
     mb_rows[cb_] = std::max(mb_rows[cb_], R.m_cap);
-    mb_wh[cb_] = std::max(mb_wh[cb_], R.wrap_rows);
-    put(mc[ca_ | (R.split_b > 1 ? FC_C_SUM : 0)], bc, be);  // split pass B: pass C adds two shares
+    mb_wh[cb_] = std::max(mb_wh[cb_], R.half ? 0 : R.wrap_rows);
+    put(mc[cc_], bc, be);  // split pass B: pass C adds the shares
+    put(mi[cb_], be, be + P.n_img);
   }
   std::vector<int4> fa, fb, fc;
   auto flatten = [](std::map<int, std::vector<int4>>& m, std::vector<int4>& v,
                     std::vector<radis_ldm_batch::Group>& g) {
     g.clear();
     for (auto& kv : m) {
-      g.push_back({kv.first, (int)v.size(), (int)kv.second.size(), 0, 0});
+      g.push_back({kv.first, (int)v.size(), (int)kv.second.size(), 0, 0, 0, 0});
       v.insert(v.end(), kv.second.begin(), kv.second.end());
     }
   };
   flatten(ma, fa, b->grp_a);
   flatten(mb, fb, b->grp_b);
+  std::vector<int4> im;
   for (auto& G : b->grp_b) {
+    G.img_first = (int)im.size();
+    G.img_count = (int)mi[G.cls].size();
+    im.insert(im.end(), mi[G.cls].begin(), mi[G.cls].end());
     G.rows = std::min(mb_rows[G.cls], FC_B_ROWS_LDS);
     G.wh = mb_wh[G.cls];
   }
@@ -343,13 +356,14 @@ int build_layout(radis_ldm_batch* b) {
   b->n_a = (int)fa.size();
   b->n_b = (int)fb.size();
   b->n_c = (int)fc.size();
+  b->n_img = (int)im.size();
   for (const Req& R : b->reqs) {
     const int rc = check_layout(R, total);
     if (rc) return rc;
   }
   std::vector<int4> all;
-  for (auto* v : {&ax, &wr, &fi, &fa, &fb, &fc}) all.insert(all.end(), v->begin(), v->end());
-  if (all.size() != (size_t)(b->n_axis + b->n_wrap + b->n_fill + b->n_a + b->n_b + b->n_c) || all.size() > INT32_MAX)
+  for (auto* v : {&ax, &wr, &fi, &fa, &fb, &fc, &im}) all.insert(all.end(), v->begin(), v->end());
+  if (all.size() != (size_t)(b->n_axis + b->n_wrap + b->n_fill + b->n_a + b->n_b + b->n_c + b->n_img) || all.size() > INT32_MAX)
     return fail(RADIS_LDM_EINVAL, "internal: %zu work items for the launch counts", all.size());
   if (all.empty()) all.push_back(make_int4(0, 0, 0, 0));
   b->items_bytes = all.size() * sizeof(int4);
@@ -361,6 +375,7 @@ int build_layout(radis_ldm_batch* b) {
   HIPCHK(hipStreamSynchronize(b->ctx->side));
   b->fill_lds = std::max<size_t>(fill_lds, 4);
   b->fill_grouped = fill_grouped;
+  b->fill_half = fill_half;
   return 0;
 }
 
@@ -424,13 +439,14 @@ struct LaunchSet {
   LdmJob* jobs;
   LdmAxes* axes;
   LdmResult* res;
-  int4* items;  // axis, image-correction, fill, pass A, pass B, pass C items in this order
+  int4* items;  // axis, image-correction, fill, pass A, pass B, pass C, cell items in this order
   int n_req;
   int n_axis, n_wrap, n_fill, n_a, n_b, n_c;
   const LaunchGroup *ga, *gb, *gc;
   int nga, ngb, ngc;
   size_t fill_lds;
   bool fill_grouped;  // the fill kernel with row groups (some request's LDM is taller than a tile)
+  bool fill_half;     // the fill kernel with tile moments (some request runs half-length transforms)
   bool tile_bounds;  // run k_tile_bounds (else the items hold valid tile line ranges)
   int n_cu;
 };
@@ -457,16 +473,20 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
     const size_t lds = X.n_wrap ? std::max(X.fill_lds, (size_t)LDM_WRAP_LDS * sizeof(float2)) : X.fill_lds;
     const dim3 grid(X.n_wrap + X.n_fill);
     const bool plain = !dbd.iso && !dbd.delta && !dbd.n_self;
-    if (X.fill_grouped) {
-      if (plain)
-        launch(b, timed, slot, 3, k_fill<true, true>, grid, dim3(LDM_FILL_T), lds, s, cj, ca, wrap_fill, X.n_wrap, dbd);
-      else
-        launch(b, timed, slot, 3, k_fill<false, true>, grid, dim3(LDM_FILL_T), lds, s, cj, ca, wrap_fill, X.n_wrap, dbd);
-    } else if (plain) {
-      launch(b, timed, slot, 3, k_fill<true, false>, grid, dim3(LDM_FILL_T), lds, s, cj, ca, wrap_fill, X.n_wrap, dbd);
-    } else {
-      launch(b, timed, slot, 3, k_fill<false, false>, grid, dim3(LDM_FILL_T), lds, s, cj, ca, wrap_fill, X.n_wrap, dbd);
-    }
+    auto fill = [&](auto P, auto G, auto H) {
+      launch(b, timed, slot, 3, k_fill<decltype(P)::value, decltype(G)::value, decltype(H)::value>, grid, dim3(LDM_FILL_T),
+             lds, s, cj, ca, wrap_fill, X.n_wrap, dbd);
+    };
+    auto by_half = [&](auto P, auto G) {
+      if (X.fill_half) fill(P, G, std::true_type{});
+      else fill(P, G, std::false_type{});
+    };
+    auto by_group = [&](auto P) {
+      if (X.fill_grouped) by_half(P, std::true_type{});
+      else by_half(P, std::false_type{});
+    };
+    if (plain) by_group(std::true_type{});
+    else by_group(std::false_type{});
   }
   items += X.n_fill;
   for (int g = 0; g < X.nga; ++g) {
@@ -474,27 +494,38 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
     const int4* it = items + G.first;
     const bool f = g == 0, l = g == X.nga - 1;
     const dim3 grid(G.count);
-    // compiled pass A is persistent: one workgroup per CU loops over the column blocks
-    const dim3 grid_p(std::min(G.count, X.n_cu));
-#define FC_A(N) \
-  case N: launch_part(b, timed, slot, 4, f, l, k_fft_a_c<N>, grid_p, dim3(FC_T_A), 0, s, cj, ca, it, G.count); break;
+    // compiled pass A is persistent: one workgroup per CU loops over the column
+    // blocks (narrow tiles: four per CU)
+    const dim3 grid_p(std::min(G.count, (G.cls & FC_NARROW) ? 4 * X.n_cu : X.n_cu));
+#define FC_A(N)                                                                                                       \
+  case N:                                                                                                             \
+    launch_part(b, timed, slot, 4, f, l, k_fft_a_c<N, fc_cols_a(N), FC_T_A>, grid_p, dim3(FC_T_A), 0, s, cj, ca, it,  \
+                G.count);                                                                                             \
+    break;
+#define FC_AN(N)                                                                                                      \
+  case N | FC_NARROW:                                                                                                 \
+    launch_part(b, timed, slot, 4, f, l, k_fft_a_c<N, FC_COLS_A_NARROW, N>, grid_p, dim3(N), 0, s, cj, ca, it, G.count); \
+    break;
     switch (G.cls) {
       FC_A(256) FC_A(320) FC_A(384) FC_A(512) FC_A(640) FC_A(768) FC_A(1024)
+      FC_AN(256)
       default: launch_part(b, timed, slot, 4, f, l, k_fft_a, grid, dim3(LDM_FFT_T), 0, s, cj, ca, it, G.count);
     }
 #undef FC_A
+#undef FC_AN
   }
   items += X.n_a;
   for (int g = 0; g < X.ngb; ++g) {
     const auto& G = X.gb[g];
     const int4* it = items + G.first;
+    const int4* img = items + X.n_b + X.n_c + G.img_first;
     const bool f = g == 0, l = g == X.ngb - 1;
-    const dim3 grid(G.count);
+    const dim3 grid(G.img_count + G.count);
 #define FC_B(N) \
   case N:                                                                                                    \
     launch_part(b, timed, slot, 5, f, l, k_fft_b_c<N>, grid, dim3(FC_T_B),                                   \
                 (size_t)G.rows * sizeof(float4) + (size_t)2 * fc_rows_b(N) * G.wh * sizeof(float), s, cj, ca, it,  \
-                G.rows, G.wh);                                                                                 \
+                G.rows, G.wh, img, G.img_count);                                                                      \
     break;
     switch (G.cls) {
       FC_B(64) FC_B(128) FC_B(256) FC_B(512) FC_B(1024) FC_B(2048)
@@ -513,16 +544,22 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
     const int4* it = items + G.first;
     const bool f = g == 0, l = g == X.ngc - 1;
     const dim3 grid(G.count);
-#define FC_C(N)                                                                                                \
-  case N: launch_part(b, timed, slot, 6, f, l, k_fft_c_c<N, false>, grid, dim3(FC_T), 0, s, cj, it, G.count); break; \
-  case N | FC_C_SUM:                                                                                                  \
-    launch_part(b, timed, slot, 6, f, l, k_fft_c_c<N, true>, grid, dim3(FC_T), 0, s, cj, it, G.count);               \
+#define FC_C1(N, F, SUM, B, T)                                                                             \
+  case (N) | (F):                                                                                        \
+    launch_part(b, timed, slot, 6, f, l, k_fft_c_c<N, SUM, B, T>, grid, dim3(T), 0, s, cj, it, G.count); \
     break;
+#define FC_C(N) FC_C1(N, 0, false, fc_cols_c(N), FC_T) FC_C1(N, FC_C_SUM, true, fc_cols_c(N), FC_T)
+#define FC_CN(N)                                              \
+  FC_C1(N, FC_NARROW, false, FC_COLS_C_NARROW, (N) / 2)       \
+  FC_C1(N, FC_NARROW | FC_C_SUM, true, FC_COLS_C_NARROW, (N) / 2)
     switch (G.cls) {
       FC_C(256) FC_C(320) FC_C(384) FC_C(512) FC_C(640) FC_C(768) FC_C(1024)
+      FC_CN(256)
       default: launch_part(b, timed, slot, 6, f, l, k_fft_c, grid, dim3(LDM_FFT_T), 0, s, cj, it, G.count);
     }
 #undef FC_C
+#undef FC_CN
+#undef FC_C1
   }
   HIPCHK(hipGetLastError());
   return 0;
@@ -552,6 +589,7 @@ int launch_kernels(radis_ldm_batch* b, hipStream_t s, bool timed, int slot, bool
   X.ngc = (int)b->grp_c.size();
   X.fill_lds = b->fill_lds;
   X.fill_grouped = b->fill_grouped;
+  X.fill_half = b->fill_half;
   // Tile line bounds depend on the grid and, through the pressure-shift
   // margin, on p; without a shift column they are fixed per layout.
   X.tile_bounds = db.has_delta || !b->tiles_valid;
@@ -915,9 +953,12 @@ int radis_ldm_batch_set_request(radis_ldm_batch* b, int i, const radis_ldm_reque
   rc = bound_request(*b->db, T);
   if (rc) return rc;
   const bool grow = T.m_need > R.m_cap;
+  // conditions the half-length transform does not take (a Gaussian beyond
+  // IMG_TMAX kelvin's, min-RMS weights)
+  const bool whole = R.half && !half_ok(T, R.tile_w);
   R = T;
-  if (grow) {
-    R.m_cap = std::max(T.m_need, (int)std::ceil(1.5 * R.m_cap));  // vulkan_compute_lib.py:1308-1313
+  if (grow || whole) {
+    if (grow) R.m_cap = std::max(T.m_need, (int)std::ceil(1.5 * R.m_cap));  // vulkan_compute_lib.py:1308-1313
     rc = build_layout(b);
     if (rc) return rc;
   }
@@ -1126,7 +1167,7 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   rc = layout_request(R, work);
   if (rc) return rc;
   const LdmItemPlan P = item_plan(*db, R);
-  const int n_items = plan_items(P);
+  const int n_items = plan_items(P) + P.n_img;
   rc = check_layout(R, work);
   if (rc) return rc;
   // scratch layout
@@ -1137,8 +1178,12 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
     return o;
   };
   const size_t o_job = take(sizeof(LdmJob)), o_axes = take(sizeof(LdmAxes)), o_res = take(sizeof(LdmResult));
-  const size_t o_items = take((size_t)n_items * sizeof(int4));
-  const long long nhi = (R.plan.L + 1023) >> LDM_TW_LO_BITS;
+  // (a half-length transform's items lie in the part of its workspace that it
+  // leaves unused)
+  const size_t items_bytes = (size_t)n_items * sizeof(int4);
+  const bool items_in_work = R.half && R.off_free + items_bytes <= R.off_y + (size_t)P.pcap * R.plan.L * 8;
+  const size_t o_items_ = items_in_work ? 0 : take(items_bytes);
+  const long long nhi = (R.tL + 1023) >> LDM_TW_LO_BITS;
   const size_t o_tw1 = take((size_t)R.plan.n1 * 8), o_tw2 = take((size_t)R.plan.n2 * 8);
   const size_t o_twl = take((size_t)(nhi + 1024) * 8);
   const size_t o_twc = take((size_t)LDM_WRAP_LC * 8);
@@ -1146,6 +1191,7 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   if (off > (size_t)RADIS_LDM_NOALLOC_BYTES)
     return fail(RADIS_LDM_ERANGE, "request needs %zu bytes of scratch, above the %lld of radis_ldm_run_noalloc "
                                   "(use a batch)", off, (long long)RADIS_LDM_NOALLOC_BYTES);
+  const size_t o_items = items_in_work ? o_work + R.off_free : o_items_;
   char* const base = ctx->scratch;
   float2* tw1 = (float2*)(base + o_tw1);
   float2* tw2 = (float2*)(base + o_tw2);
@@ -1159,18 +1205,19 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   fill_job(*db, R, base + o_work, out_dev, J);
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_put_job, dim3(1), dim3(64), 0, s, J, (LdmJob*)(base + o_job));
-  const long long n_tw = R.plan.n1 + R.plan.n2 + nhi + 1024;
+  const long long n_tw = R.tn1 + R.tn2 + nhi + 1024;
   hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((n_tw + 255) / 256, 4096)), dim3(256), 0, s, tw1,
-                     R.plan.n1, tw2, R.plan.n2, twl, (long long)R.plan.L);
+                     R.tn1, tw2, R.tn2, twl, (long long)R.tL);
   hipLaunchKernelGGL(k_twiddles, dim3(LDM_WRAP_LC / 256), dim3(256), 0, s, (float2*)(base + o_twc), LDM_WRAP_LC,
                      (float2*)nullptr, 0, (float2*)nullptr, 0ll);
   hipLaunchKernelGGL(k_make_items, dim3((n_items + 255) / 256), dim3(256), 0, s, (int4*)(base + o_items), P, n_items);
   HIPCHK(hipGetLastError());
-  const int cls_ac = R.plan.fc ? R.plan.n1 : 0;
-  const int cls_b = R.plan.fc ? R.plan.n2 : (R.plan.n2 <= LDM_CAP_B ? 0 : -1);
-  const LaunchGroup ga{cls_ac, 0, P.pcap * P.n_colA, 0, 0},
-      gb{cls_b, 0, P.n_rowB, std::min(R.m_cap, FC_B_ROWS_LDS), R.wrap_rows},
-      gc{cls_ac | (R.split_b > 1 ? FC_C_SUM : 0), 0, P.n_colC, 0, 0};
+  const int cls_a = R.plan.fc ? R.tn1 | (R.narrow_a ? FC_NARROW : 0) : 0;
+  const int cls_c = (R.plan.fc ? R.tn1 | (R.narrow_c ? FC_NARROW : 0) : 0) | (R.n_share > 1 ? FC_C_SUM : 0);
+  const int cls_b = R.plan.fc ? R.tn2 : (R.plan.n2 <= LDM_CAP_B ? 0 : -1);
+  const LaunchGroup ga{cls_a, 0, P.pcap * P.n_colA, 0, 0, 0, 0},
+      gb{cls_b, 0, P.n_rowB, std::min(R.m_cap, FC_B_ROWS_LDS), R.half ? 0 : R.wrap_rows, 0, P.n_img},
+      gc{cls_c, 0, P.n_colC, 0, 0, 0, 0};
   LaunchSet X{};
   X.jobs = (LdmJob*)(base + o_job);
   X.axes = (LdmAxes*)(base + o_axes);
@@ -1189,8 +1236,9 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   X.ngb = 1;
   X.gc = &gc;
   X.ngc = 1;
-  X.fill_lds = std::max<size_t>(fill_tile_bytes(R.fill_rows, R.tile_w), 4);
+  X.fill_lds = std::max<size_t>(fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R), 4);
   X.fill_grouped = R.fill_groups > 1;
+  X.fill_half = R.half;
   X.tile_bounds = true;
   X.n_cu = ctx->n_cu;
   rc = launch_set(X, db->dev, nullptr, s, false, 0);

@@ -14,6 +14,7 @@
 // LDS slot pad_idx(i*B + b) (the same layout as the generic transform).
 #pragma once
 #include "ldm_fft.h"
+#include "ldm_image.h"
 
 constexpr int fc_odd(int n) { return n % 3 == 0 ? 3 : (n % 5 == 0 ? 5 : 1); }
 constexpr int fc_log2(int n) { return n <= 1 ? 0 : 1 + fc_log2(n >> 1); }
@@ -270,8 +271,9 @@ __device__ __forceinline__ void fc_load_tw_stages(float2* __restrict__ s_tw, con
 // Twiddles W_L^(m * (j0 + s*DS + q*DQ)) of one thread's last-stage outputs
 // (s < IT thread passes, q < R legs; m fixed per thread) as
 // base * A^s * C^q from three table values, so an output costs one complex
-// product instead of two table gathers.  The longest product chain has
-// IT + R - 2 factors (~1e-7 rounding each).  Every exponent is below L.
+// product instead of two table gathers.  The powers of C are products at most
+// log2(R) deep (a chain of R - 1 took as many operations and 15 roundings at
+// R = 16).  Every exponent is below L.
 template <int IT, int R>
 struct TwProg {
   float2 ws[IT], wq[R];
@@ -285,7 +287,7 @@ struct TwProg {
     for (int s = 1; s < IT; ++s) ws[s] = cmul(ws[s - 1], A);
     wq[0] = make_float2(1.0f, 0.0f);
 #pragma unroll
-    for (int q = 1; q < R; ++q) wq[q] = cmul(wq[q - 1], C);
+    for (int q = 1; q < R; ++q) wq[q] = q == 1 ? C : cmul(wq[q / 2], wq[q - q / 2]);
   }
   __device__ __forceinline__ float2 operator()(int s, int q) const { return cmul(ws[s], wq[q]); }
 };
@@ -302,11 +304,11 @@ struct TwProg {
 // (tile sizes FC_CAP_A, FC_CAP, FC_CAP_B and fc_cols_a / fc_cols_c /
 // fc_rows_b are in ldm_job.h: the host planner sizes the work items with them)
 
-template <int N1>
-__global__ __launch_bounds__(FC_T_A) void k_fft_a_c(const LdmJob* __restrict__ jobs, const LdmAxes* __restrict__ axes,
+template <int N1, int B, int T>
+__global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob* __restrict__ jobs, const LdmAxes* __restrict__ axes,
                                                    const int4* __restrict__ items, int n_items) {
-  constexpr int B = fc_cols_a(N1), LB = fc_log2(B), CAPE = N1 * B, T = FC_T_A;
-  static_assert(CAPE % T == 0, "tile is a whole number of thread passes");
+  constexpr int LB = fc_log2(B), CAPE = N1 * B;
+  static_assert(CAPE % T == 0 && T % B == 0, "tile is a whole number of thread passes");
   using SH = FcShape<N1, B, T>;
   constexpr int NR0 = N1 / SH::R0;
   constexpr int NSL = fc_ns(N1, fc_nstages(N1) - 1);
@@ -331,14 +333,14 @@ __global__ __launch_bounds__(FC_T_A) void k_fft_a_c(const LdmJob* __restrict__ j
     const LdmJob& J = jobs[it.x];
     const int p = it.y;
     if (J.status || p >= axes[it.x].p) return false;
-    const int N2 = J.n2, n2_0 = it.z * B, V = (int)J.v;
+    const int N2 = J.tn2, n2_0 = it.z * B, V = (int)J.v;
     // pair p's rows, interleaved: z = (x_2p, x_2p+1) is one float2
     const float2* rz = reinterpret_cast<const float2*>(J.ldm) + (long long)p * J.ldm_stride;
     const bool has_b = (2 * p + 1) < axes[it.x].m;
     // L >= 2 N_v, so V = N_v + 1 <= L/2 unless L = 2 N_v exactly: then the
     // upper half of every column (n1 >= N1/2, n >= L/2) is zero and its
     // loads are skipped
-    const bool upper_zero = (long long)V <= J.L / 2;
+    const bool upper_zero = (long long)V <= J.tL / 2;
     // the two LDM rows, zero beyond V (and row b zero when the pair is odd)
 #pragma unroll
     for (int s = 0; s < SH::IT0; ++s) {
@@ -371,8 +373,8 @@ __global__ __launch_bounds__(FC_T_A) void k_fft_a_c(const LdmJob* __restrict__ j
     }
     const int4 it = items[idx];
     const LdmJob& J = jobs[it.x];
-    const int N2 = J.n2, n2_0 = it.z * B;
-    float2* Y = J.ybuf + (long long)it.y * J.L;
+    const int N2 = J.tn2, n2_0 = it.z * B;
+    float2* Y = J.ybuf + (long long)it.y * J.tL;
     // output k1 of this thread's last-stage element (s, q): j0 + s*(T/B) + q*NS;
     // the table halves of the progression's three factors load now and are
     // multiplied out just before the last stage
@@ -412,9 +414,10 @@ __global__ __launch_bounds__(FC_T_A) void k_fft_a_c(const LdmJob* __restrict__ j
 // registers (fetched during the previous pair) and its last stage multiplies
 // by the lineshape FTs and accumulates in registers; only the accumulated
 // spectrum goes through LDS into the inverse transform, whose last stage
-// writes B with the W_L twiddle.  Item (job, row block, share): with
-// J.bbuf2 set, share 0 takes the first ceil(P/2) pairs into B and share 1
-// the rest into bbuf2 (pass C adds the two).  The dynamic LDS (sized per
+// writes B with the W_L twiddle.  Item (job, y, z): number
+// y * split_b + z, row block number / n_share, share number % n_share of its
+// pairs, whose partial spectrum goes to bbuf + share * share_stride (pass C
+// adds them).  The dynamic LDS (sized per
 // launch) holds the rows' lineshape coefficients (n_rows_lds float4), then
 // the image-correction values of the block's rows at its two corrected bins
 // (2 x B x n_wh floats, n_wh >= N_L of every request with a correction).
@@ -422,7 +425,8 @@ __global__ __launch_bounds__(FC_T_A) void k_fft_a_c(const LdmJob* __restrict__ j
 template <int N2>
 __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_fft_b_c(const LdmJob* __restrict__ jobs,
                                                       const LdmAxes* __restrict__ axes,
-                                                      const int4* __restrict__ items, int n_rows_lds, int n_wh) {
+                                                      const int4* __restrict__ items, int n_rows_lds, int n_wh,
+                                                      const int4* __restrict__ img, int n_img) {
   constexpr int CAP = FC_CAP_B, T = FC_T_B;
   constexpr int B = fc_rows_b(N2), LB = fc_log2(B);
   static_assert(fc_pow2(N2), "pass B rows are powers of two");
@@ -439,15 +443,21 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
   __shared__ float2 bufs[2][LdsSize<CAP>::value];
   constexpr bool SWAP = fc_nstages(N2, PV) % 2 == 0;
   __shared__ float2 s_tw[fc_tw_off(N2, fc_nstages(N2, PV), PV)];  // per-stage twiddle tables
-  const int4 it = items[blockIdx.x];
+  if ((int)blockIdx.x < n_img) {  // the cells' image corrections (half-length transforms)
+    static_assert(sizeof(bufs) >= IMG_LDS, "an image item's LDS");
+    const int4 c = img[blockIdx.x];
+    image_item(jobs[c.x], axes[c.x], c.y, c.z, reinterpret_cast<char*>(bufs));
+    return;
+  }
+  const int4 it = items[blockIdx.x - n_img];
   const LdmJob& J = jobs[it.x];
   if (J.status) return;
-  const int N1 = J.n1;
-  const int k1_0 = it.y * B;
-  const long long L = J.L;
+  const int N1 = J.tn1;
+  const int item = it.y * J.split_b + it.z, share = item % J.n_share;
+  const int k1_0 = (item / J.n_share) * B;
+  const long long L = J.tL;
   const int P = axes[it.x].p, M = axes[it.x].m;
-  const int p_mid = J.bbuf2 ? (P + 1) / 2 : P;
-  const int p0 = it.z ? p_mid : 0, p1 = it.z ? P : p_mid;  // this workgroup's pairs
+  const int p0 = P * share / J.n_share, p1 = P * (share + 1) / J.n_share;  // this workgroup's pairs
   fc_load_tw_stages<N2, T, PV>(s_tw, J.tw2);
   // The rows' lineshape coefficients (a_l, b_m, 1/F(0), fold count) staged
   // in LDS.  Read from global memory they are scalar loads, and the LDS
@@ -529,7 +539,7 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
   // w_lo / w_hi hold the row b of those bins (-1: none), w_s the second's s.
   float* const s_wh = reinterpret_cast<float*>(s_row + n_rows_lds);  // [2][B][n_wh]
   auto wh = [&](int c, int b, int m) -> float& { return s_wh[(c * B + b) * n_wh + m]; };
-  const int WK = J.wrap_k;
+  const int WK = J.half ? 0 : J.wrap_k;
   int w_lo = -1, w_hi = -1, w_s = 0;
   if (WK) {
     const int NLw = axes[it.x].nl;
@@ -647,7 +657,7 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
     }
   }
   __syncthreads();
-  float2* Bo = (it.z ? J.bbuf2 : J.bbuf) + (long long)k1_0 * N2;
+  float2* Bo = J.bbuf + share * J.share_stride + (long long)k1_0 * N2;
   // output n2 of this thread's last-stage element (s, q): j0 + s*(T/B) + q*NS, row k1 fixed
   TwProg<SH::ITL, SH::RL> tw;
   tw.init(J, k1_0 + (threadIdx.x & (B - 1)), threadIdx.x >> LB, T >> LB, NSL);
@@ -663,54 +673,71 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
 
 // ---------------------------------------------------------------------------
 // Pass C with N1 fixed (see k_fft_c): first stage straight from B, last
-// stage straight to the output.  SUM: B is J.bbuf + J.bbuf2 (pass B split
-// its pairs over two workgroups per row block).
+// stage straight to the output.  SUM: B is the sum of pass B's shares.  After a
+// half-length transform the image correction is added.
 // ---------------------------------------------------------------------------
-template <int N1, bool SUM>
-__global__ __launch_bounds__(FC_T, 4) void k_fft_c_c(const LdmJob* __restrict__ jobs, const int4* __restrict__ items,
+template <int N1, bool SUM, int B, int T>
+__global__ __launch_bounds__(T, 4) void k_fft_c_c(const LdmJob* __restrict__ jobs, const int4* __restrict__ items,
                                                      int n_items) {
-  constexpr int B = fc_cols_c(N1), LB = fc_log2(B), CAPE = N1 * B;
-  static_assert(CAPE % FC_T == 0, "tile is a whole number of thread passes");
+  constexpr int LB = fc_log2(B), CAPE = N1 * B;
+  static_assert(CAPE % T == 0, "tile is a whole number of thread passes");
   __shared__ float2 buf[LdsSize<CAPE>::value];
   __shared__ float2 s_tw[N1];
+  __shared__ float s_cf[IMG_MAX_CELLS * IMG_NODES];
   const int4 it = items[xcd_block(blockIdx.x, n_items)];
   const LdmJob& J = jobs[it.x];
-  const int N2 = J.n2;
+  const int N2 = J.tn2;
   const int n2_0 = it.z * B;
   const int nv = (int)J.nv;
   if (J.status) {
 #pragma unroll
-    for (int s = 0; s < CAPE / FC_T; ++s) {
-      const int e = threadIdx.x + s * FC_T;
+    for (int s = 0; s < CAPE / T; ++s) {
+      const int e = threadIdx.x + s * T;
       const int n = n2_0 + (e & (B - 1)) + N2 * (e >> LB);
       if (n < nv) gst(J.out, 4u * (unsigned)n, 0.0f);
     }
     return;
   }
-  fc_load_tw<N1, FC_T>(s_tw, J.tw1);
+  fc_load_tw<N1, T>(s_tw, J.tw1);
   const float sc = J.out_scale;
   auto nop = [] {};
   auto off = [&](int e) { return 8u * (unsigned)((e >> LB) * N2 + n2_0 + (e & (B - 1))); };  // < 8 L <= 2^24
-  auto ld = [&](int, int, int e) -> float2 {
-    float2 z = gld(J.bbuf, off(e));
-    if constexpr (SUM) {
-      const float2 w = gld(J.bbuf2, off(e));
-      z.x += w.x;
-      z.y += w.y;
+  // the first stage's inputs, a share at a time (a share's loads in flight
+  // together)
+  using SH = FcShape<N1, B, T>;
+  float2 v[SH::IT0][SH::R0];
+  auto fetch = [&](const float2* b, bool add) {
+#pragma unroll
+    for (int s = 0; s < SH::IT0; ++s) {
+      const int t = threadIdx.x + s * T;
+      if (SH::ITEMS0 % T == 0 || t < SH::ITEMS0) {
+#pragma unroll
+        for (int q = 0; q < SH::R0; ++q) {
+          const float2 z = gld(b, off(t + q * (N1 / SH::R0) * B));
+          v[s][q] = add ? cadd(v[s][q], z) : z;
+        }
+      }
     }
-    return z;
   };
+  fetch(J.bbuf, false);
+  if constexpr (SUM) {
+    for (int s = 1; s < J.n_share; ++s) fetch(J.bbuf + s * J.share_stride, true);
+  }
+  auto ld = [&](int s, int q, int) -> float2 { return v[s][q]; };
+  ImageEval img{};
+  const bool half = J.half != 0;
+  if (half) img.load(J, s_cf, T);  // the transform's barriers lie between this and its use
   if (J.derived) {  // uniform per workgroup: the plain store path stays as lean as without the epilogue
     auto st = [&](int, int, int e, float2 z) {
       const int n = n2_0 + (e & (B - 1)) + N2 * (e >> LB);
-      if (n < nv) store_derived(J, n, z.x * sc);
+      if (n < nv) store_derived(J, n, half ? z.x * sc + img(n) : z.x * sc);
     };
-    fc_fft_io<N1, B, FC_T, false, true, true>(buf, s_tw, ld, st, nop);
+    fc_fft_io<N1, B, T, false, true, true>(buf, s_tw, ld, st, nop);
   } else {
     auto st = [&](int, int, int e, float2 z) {
       const int n = n2_0 + (e & (B - 1)) + N2 * (e >> LB);
-      if (n < nv) gst(J.out, 4u * (unsigned)n, z.x * sc);
+      if (n < nv) gst(J.out, 4u * (unsigned)n, half ? z.x * sc + img(n) : z.x * sc);
     };
-    fc_fft_io<N1, B, FC_T, false, true, true>(buf, s_tw, ld, st, nop);
+    fc_fft_io<N1, B, T, false, true, true>(buf, s_tw, ld, st, nop);
   }
 }

@@ -57,11 +57,42 @@ static_assert(LDM_AX_CHUNK == LDM_SKY_BLOCK, "a partial block is one scan chunk"
 #define FC_T_B 256
 #define FC_C_SUM (1 << 20)  // pass C launch-class flag: B is the sum of two pass B shares
 #define FC_B_ROWS_LDS 512  // rows whose lineshape coefficients pass B stages in LDS (more: read from global memory)
+// Half-length transforms (ldm_image.h): the compiled passes run at half the
+// planned length L, and the circular images that a period of L/2 < 2 N_v
+// brings onto the grid are corrected from a coarse description.  With the gap
+// D = L/2 - N_v (the distance of the nearest image from any output) the grid
+// is cut into cells of at most 2 D / 5 points with IMG_NODES Chebyshev nodes
+// each: an image's Lorentzian is analytic around a cell out to D (to 3 D / 5
+// from a last cell that reaches past the grid), so the interpolation error is
+// (6 + sqrt(35))^-8 ~ 2e-9 ((4 + sqrt(15))^-8 ~ 7e-8) of the image.  A fill tile
+// is described by four moments, so it must be short against D
+// (IMG_TILES_PER_GAP: 5 (1/64)^4 ~ 3e-7 of the image), and so must the Gaussian
+// part (IMG_SIGMAS_PER_GAP standard deviations, at IMG_TMAX kelvin or the
+// request's temperature: the image's Gaussian enters to second order, the
+// fourth is 15 / 64^4 of the image).
+#define IMG_NODES 8
+#define IMG_TARGETS 128  // nodes per image item: its source part costs about as much as so many
+#define IMG_TILES_PER_GAP 32
+#define IMG_SIGMAS_PER_GAP 64.0
+#define IMG_TMAX 1e4
+#define IMG_MAX_CELLS 128  // D >= 0.025 L/2: at most 2.5 N_v / D + a few
+// LDS behind a fill tile (M rows of W columns) for its moments: a float2 per
+// row, then a float4 per row and part of 128 columns (TileMoments)
+constexpr int tile_parts(int W) { return W > 128 ? W / 128 : 1; }
+constexpr int tile_moment_lds(int M, int W) { return 16 + ((8 * M + 15) & ~15) + 16 * (M + 1) * tile_parts(W); }
 constexpr int fc_pow2_floor(int n) { return n < 2 ? 1 : 2 * fc_pow2_floor(n >> 1); }
 // columns per workgroup of pass A and of pass C for N1, and rows per
 // workgroup of pass B for N2
 constexpr int fc_cols_a(int n1) { return fc_pow2_floor(FC_CAP_A / n1); }
 constexpr int fc_cols_c(int n1) { return fc_pow2_floor(FC_CAP / n1); }
+// narrow pass A and C tiles, for launches whose wide ones would leave CUs
+// idle: 16 and 8 columns, 16 elements per thread.  At n1 = 256 a 72-block pass A
+// took 9.2 -> 6.9 us and an 8-block pass C 8.1 -> 6.8 us; with an odd factor
+// (n1 = 320: a first stage of 3.2 passes) pass C took 8.2 -> 15.5 us.
+constexpr bool fc_narrow(int n1) { return n1 == 256; }
+#define FC_COLS_A_NARROW 16
+#define FC_COLS_C_NARROW 8
+#define FC_NARROW (1 << 21)  // pass A and C launch-class flag
 constexpr int fc_rows_b(int n2) { return FC_CAP_B / n2; }
 
 // device status codes (LdmJob::status)
@@ -185,26 +216,40 @@ struct LdmJob {
   float inv_Lws;                 // 1/(L*wstep) (frequency step of the FT grid)
   float half_inv_ws;             // 1/(2*wstep)
   int single_iso;                // 1: every line is iso slot 1 and the G axis comes from the window ends
-  int n1, n2;                    // four-step split
+  int n1, n2;                    // four-step split of L
+  // the transform the passes run: L itself, or half of it (half, compiled
+  // passes only: image correction of ldm_image.h)
+  long long tL;
+  int tn1, tn2;
+  // pass B's partial spectra: share s of a row block's pairs goes to
+  // bbuf + s * share_stride (n_share of them, added by pass C); a pass B item
+  // (y, z) is number y * split_b + z, row block number / n_share
+  int n_share, split_b;
+  long long share_stride;
+  // half-length transforms: per cell IMG_NODES values of the correction
+  double* img_u;                 // [n_cell][IMG_NODES]
+  int cell_tiles, n_cell;        // fill tiles per cell, cells
   int nrad1, nrad2;
   int rad1[LDM_MAX_RAD], rad2[LDM_MAX_RAD];
   int bA, bB;                    // columns per workgroup in passes A/C and pass B
   int m_cap, tile_w, n_tiles;
   int fill_rows, fill_groups;    // LDM rows per fill row group, groups per tile (1: the tile holds every row)
   long long ldm_stride;          // elements per LDM row
+  int half;                      // 1: half-length transforms (the transform fields above)
+  float* mom;                    // then per fill tile and L-axis node four moments, [n_tiles][N_L][4]
+  float* row_a;                  // [m_cap] (pi*wG_l)^2/(4 ln2)
+  float* row_inv_f0;             // [m_cap] 1/F_lm(0)
   float* ldm;                    // [ceil(m_cap/2)][ldm_stride] float2: rows 2p, 2p+1 interleaved
   float2* ybuf;                  // [(m_cap+1)/2][L]
-  float2* bbuf;                  // [L]
-  float2* bbuf2;                 // [L] pass B's second share of the pairs (null: not split); pass C adds it
+  float2* bbuf;                  // [n_share][share_stride] pass B's partial spectra
+  float2* bbuf2;                 // null: pass B not split
   float* out;                    // [nv]
   // derived outputs (null = not wanted): absorbance, transmittance, emissivity, radiance
   float *d_abs, *d_trans, *d_emis, *d_rad;
   double path_length, Tgas;
   int derived, scale_log2;
   int* nfold;                    // [m_cap]
-  float* row_a;                  // [m_cap] (pi*wG_l)^2/(4 ln2)
   float* row_b;                  // [m_cap] pi*wL_m
-  float* row_inv_f0;             // [m_cap] 1/F_lm(0)
   const float2* tw1;             // exp(-2 pi i e/n1), e < n1
   const float2* tw2;             // exp(-2 pi i e/n2), e < n2
   const float2* twl_hi;          // W_L^(h*1024)

@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include "ldm_fft.h"
+#include "ldm_image.h"
 #include "ldm_job.h"
 
 #define LDM_C_CGS 2.99792458e10       /* radis/phys/constants.py:78 */
@@ -354,6 +355,8 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
   float* const row_b = J.row_b;
   float* const row_inv_f0 = J.row_inv_f0;
   const bool ends = threadIdx.x == 0 && single && i1 > i0;
+  if (J.half)  // the image correction is accumulated by the pass B launch
+    for (int e = threadIdx.x; e < J.n_cell * IMG_NODES; e += blockDim.x) J.img_u[e] = 0.0;
   const double nu_a = ends ? db.nu0[i0] : 0.0, nu_b = ends ? db.nu0[i1 - 1] : 0.0;
   // Q(Tref)/Q(T) of the slots with a partition-function spline (the fill
   // reads these after this kernel): calc_linestrength_eq's Qref/Q,
@@ -846,8 +849,8 @@ __device__ __forceinline__ void line_terms(const LineConst& C, const LineRaw& r,
 // request of the launch); item y = tile * fill_groups + g, and the workgroup
 // keeps rows [g * fill_rows, g * fill_rows + MR) only: each of its 8 atomics
 // checks its corner's row.  A request with fill_groups = 1 has one group of
-// every row.
-template <bool NONEQ, bool PLAIN, bool GROUPED>
+// every row.  HALF: some request of the launch runs half-length transforms.
+template <bool NONEQ, bool PLAIN, bool GROUPED, bool HALF>
 __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, const int4 it, const LdmDb& db,
                                           double* acc) {
   const int M = A.m;
@@ -882,6 +885,11 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
     const unsigned l1 = first + LDM_FILL_T;
     cols.load<NONEQ, PLAIN>(l1 < hlast ? l1 : hlast, n2);
   }
+  // half-length transforms: the rows' values for the tile's moments, in flight
+  // during the line loop (a taller LDM's remaining rows after it)
+  const bool half = HALF && J.half != 0;
+  float2 row_v = make_float2(0.0f, 0.0f);
+  if (half && (int)threadIdx.x < M) row_v = tile_row(J, threadIdx.x);
   {
     // whole 16-byte pairs, and the last cell alone when MR * Wp is odd
     const int n = MR * Wp, n2 = n >> 1;
@@ -889,7 +897,7 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
     for (int e = threadIdx.x; e < n2; e += blockDim.x) a2[e] = make_double2(0.0, 0.0);
     if ((n & 1) && threadIdx.x == 0) acc[n - 1] = 0.0;
   }
-  __syncthreads();
+  lds_barrier();
   const int wlen = (int)(k_hi - k_lo);
   const int sg = nl * Wp;
   // Corner order per lane.  The 8 atomics of a line go to its stencil's
@@ -950,7 +958,12 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
       if (q11) atomicAdd(b1 + s_g + s_l, (double)(v * w11));
     }
   }
-  __syncthreads();
+  TileMoments mom(acc + MR * Wp, M, W);  // half: one row group, MR = M
+  if (half) {
+    if ((int)threadIdx.x < M) mom.rows[threadIdx.x] = row_v;
+    for (int r = threadIdx.x + LDM_FILL_T; r < M; r += LDM_FILL_T) mom.rows[r] = tile_row(J, r);
+  }
+  lds_barrier();
   // flush: the LDM interleaves rows 2p and 2p+1 (element n of row 2p+h at
   // float 2n+h of pair p).  A lane writes 2 columns of one pair (16 bytes)
   // per step: (2p, c), (2p+1, c), (2p, c+1), (2p+1, c+1); the second row of
@@ -962,16 +975,21 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
   float* const out = J.ldm + 2 * k_lo + (long long)(r0 >> 1) * pstride;  // column k_lo of the group's first pair
   for (int w = threadIdx.x; w < (P2 << sh2); w += LDM_FILL_T) {
     const int p = w >> sh2, c = 2 * (w & (W2 - 1));
-    if (c >= wlen) continue;
     const double* src = acc + (2 * p) * Wp + c;
     const double2 a = *reinterpret_cast<const double2*>(src);
     // row 2p starts on an even cell (16-byte aligned), row 2p+1 on an odd one when Wp is odd
     const double2 b = (2 * p + 1 < MR) ? ((Wp & 1) ? make_double2(src[Wp], src[Wp + 1])
                                                    : *reinterpret_cast<const double2*>(src + Wp))
                                       : make_double2(0.0, 0.0);
+    const float a0 = (float)a.x, a1 = (float)a.y, b0 = (float)b.x, b1 = (float)b.y;
     float* dst = out + p * pstride + 2 * c;
-    if (c + 2 <= wlen) *reinterpret_cast<float4*>(dst) = make_float4((float)a.x, (float)b.x, (float)a.y, (float)b.y);
-    else *reinterpret_cast<float2*>(dst) = make_float2((float)a.x, (float)b.x);
+    if (c + 2 <= wlen) *reinterpret_cast<float4*>(dst) = make_float4(a0, b0, a1, b1);
+    else if (c < wlen) *reinterpret_cast<float2*>(dst) = make_float2(a0, b0);
+    if (half) mom.pair(p, c, a0, a1, b0, b1);  // (cells past the grid hold zeros)
+  }
+  if (half) {
+    lds_barrier();
+    mom.nodes(J, ng, nl, tile);
   }
 }
 

@@ -131,10 +131,19 @@ struct Req {
   int64_t stride = 0;
   int scale_log2 = 0;
   int bA = 0, bB = 0, bC = 0;  // log2 of the pass A / C column blocks and pass B row blocks
-  int split_b = 1;     // workgroups per pass B row block, each taking a share of the pairs
+  // what the passes run (plan_exec): the planned split, or for half the planned
+  // length (half) one of its halves; bX: log2 of the columns / rows per workgroup
+  bool half = false, may_half = false, narrow_a = false, narrow_c = false;
+  int64_t tL = 0;
+  int tn1 = 0, tn2 = 0, bX[3] = {0, 0, 0};
+  int cell_tiles = 0, n_cell = 0;  // half: fill tiles per cell of the image correction, cells
+  double wg_hi = 0;    // bound of the Gaussian FWHM (cm-1)
+  int split_b = 1;     // 2: pass B's pairs are split over several workgroups per row block
+  int n_share = 1;     // workgroups per pass B row block, each taking a share of the pairs
   int n_axp = 0;       // axis partials (items of k_axis)
   bool sky_whole = false;  // width extremes from the whole list's Pareto sets in k_finalize (no k_axis items)
   size_t off_ldm = 0, off_y = 0, off_b = 0, off_b2 = 0, off_rows = 0, off_axp = 0, off_wrap = 0;
+  size_t off_share = 0, off_img = 0, off_mom = 0, off_free = 0;  // partial spectra; half: correction values, tile moments, unused from here
   const float2 *tw1 = nullptr, *tw2 = nullptr, *twl_hi = nullptr, *twl_lo = nullptr, *tw_wrap = nullptr;
 };
 
@@ -545,6 +554,7 @@ int bound_request(const radis_ldm_db& db, Req& R) {
   if (R.i1 <= R.i0) {
     R.m_need = 1;
     R.scale_log2 = 0;
+    R.wg_hi = 0;
     return 0;
   }
   const int b0 = (int)(R.i0 / STAT_BLOCK), b1 = (int)((R.i1 - 1) / STAT_BLOCK);
@@ -590,6 +600,7 @@ int bound_request(const radis_ldm_db& db, Req& R) {
   }
   const double wg_lo = 2 * (db.h_nu0[R.i0] / 2.99792458e10) * dmin * (1 - 1e-9);
   const double wg_hi = 2 * (db.h_nu0[R.i1 - 1] / 2.99792458e10) * dmax * (1 + 1e-9);
+  R.wg_hi = wg_hi;
   if (!(wg_lo > 0)) return fail(RADIS_LDM_EINVAL, "non-positive Gaussian width (nu0 <= 0 in window)");
   // k_axis takes N = ceil((log(w_max + 1e-4) - log(w_min)) / dx) + 1 from the
   // exact extremes; the bounds above enclose them with a 1e-9 relative
@@ -721,12 +732,18 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   }
   J.c_stim_T = (float)(-HC_K / r.Tgas);
   J.c_stim_R = (float)(-HC_K / r.Tref);
-  J.out_scale = (float)(1.0 / ((double)R.plan.L * r.wstep));
-  J.inv_Lws = (float)(1.0 / ((double)R.plan.L * r.wstep));
+  J.out_scale = (float)(1.0 / ((double)R.tL * r.wstep));
+  J.inv_Lws = (float)(1.0 / ((double)R.tL * r.wstep));
   J.half_inv_ws = (float)(0.5 / r.wstep);
   J.single_iso = db.has_iso ? 0 : 1;
   J.n1 = R.plan.n1;
   J.n2 = R.plan.n2;
+  J.tL = R.tL;
+  J.tn1 = R.tn1;
+  J.tn2 = R.tn2;
+  J.half = R.half ? 1 : 0;
+  J.n_share = R.n_share;
+  J.split_b = R.split_b;
   J.nrad1 = R.plan.nr1;
   J.nrad2 = R.plan.nr2;
   for (int i = 0; i < J.nrad1; ++i) J.rad1[i] = R.plan.r1[i];
@@ -741,7 +758,12 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.ldm_stride = R.stride;
   J.ldm = (float*)(work + R.off_ldm);
   J.ybuf = (float2*)(work + R.off_y);
-  J.bbuf = (float2*)(work + R.off_b);
+  J.bbuf = (float2*)(work + R.off_share);
+  J.share_stride = R.half ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
+  J.mom = R.half ? (float*)(work + R.off_mom) : nullptr;
+  J.img_u = R.half ? (double*)(work + R.off_img) : nullptr;
+  J.cell_tiles = R.cell_tiles;
+  J.n_cell = R.n_cell;
   J.bbuf2 = R.split_b > 1 ? (float2*)(work + R.off_b2) : nullptr;
   J.out = out;
   J.d_abs = R.derived.absorbance;
@@ -775,35 +797,24 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.status = 0;
 }
 
-// Workgroups per pass B row block (Req::split_b) for requests reqs[0..n)
-// that run together.  A compiled pass B workgroup walks every pair of its
-// row block; when a launch has few row blocks (a 500,001-point grid at
-// L = 512 x 2048: 512 workgroups, two per CU) the device runs them at two
-// waves per SIMD, latency-bound.  Splitting the pairs over two workgroups
-// (pass C adds the two partial spectra) doubles the waves when the doubled
-// launch still fits FC_B_SPLIT_WGS_PER_CU workgroups per CU at once; it
-// costs an inverse transform per share and L*8 bytes written and read.
-// Measured on that grid: pass B 44.2 -> 37.7 us; on L = 640 x 2048 with 72
-// pairs (1280 workgroups, more than fit at once) the split was slower.
-constexpr int FC_B_SPLIT_WGS_PER_CU = 4;
-constexpr int FC_B_SPLIT_MIN_PAIRS = 4;
-void choose_split_b(Req* reqs, int n, int n_cu) {
-  std::map<int, long long> blocks;  // compiled pass B class (N2) -> row blocks of the launch
-  for (int i = 0; i < n; ++i)
-    if (reqs[i].plan.fc) blocks[reqs[i].plan.n2] += reqs[i].plan.n1 / fc_rows_b(reqs[i].plan.n2);
-  for (int i = 0; i < n; ++i) {
-    Req& R = reqs[i];
-    R.split_b = 1;
-    if (R.plan.fc && (R.m_cap + 1) / 2 >= FC_B_SPLIT_MIN_PAIRS &&
-        2 * blocks[R.plan.n2] <= (long long)FC_B_SPLIT_WGS_PER_CU * n_cu)
-      R.split_b = 2;
-  }
+// Whether the passes of a request with tiles of `tile_w` points may run at
+// half the planned length (ldm_image.h): the images of the shorter period stay
+// IMG_SIGMAS_PER_GAP Gaussian standard deviations and IMG_TILES_PER_GAP tiles
+// away from every output.  Not with min-RMS weights: neighbouring G rows then
+// hold (wL / wG)^2 / 20 times a line with opposite signs, so the FP32 rounding
+// of the transforms shows, and per output it is sqrt 2 larger at half the
+// length (the same noise over half as many points, of which the grid is more;
+// 50,001 points, 2.5 bar: 2.6e-6 -> 3.1e-6 to 5e-6 of the norm).
+bool half_ok(const Req& R, int tile_w) {
+  if (R.r.flags & RADIS_LDM_MIN_RMS) return false;
+  const double gap = (double)(R.plan.L / 2 - R.nv);
+  const double sigma = R.wg_hi * std::sqrt(std::max(1.0, IMG_TMAX / R.r.Tgas)) / (2.3548 * R.delta_w);
+  return gap >= (double)IMG_TILES_PER_GAP * tile_w && gap >= IMG_SIGMAS_PER_GAP * sigma;
 }
 
-// Workspace of one request (tile width, pass splits and the offsets of its
-// buffers from `total`, which it advances); shared by the batch layout and
-// radis_ldm_request_bytes.
-int layout_request(Req& R, size_t& total) {
+// Tile width, row groups and the transform a request runs (Req::half, tL,
+// tn1, tn2), from its plan, its row capacity and its conditions.
+int plan_exec(Req& R) {
   R.tile_w = R.r.tile_w ? R.r.tile_w : choose_tile(R.m_cap);
   R.fill_rows = R.m_cap;
   R.fill_groups = 1;
@@ -820,26 +831,142 @@ int layout_request(Req& R, size_t& total) {
     R.fill_groups = (R.m_cap + rows - 1) / rows;
   }
   const int64_t V = R.nv + 1;
-  R.n_tiles = (int)((V + R.tile_w - 1) / R.tile_w);
-  R.stride = (int64_t)align_up((size_t)V, 64);
-  const int n1 = R.plan.n1, n2 = R.plan.n2;
-  if (R.plan.fc) {
-    R.bA = floor_log2(fc_cols_a(n1));
-    R.bB = floor_log2(fc_rows_b(n2));
-    R.bC = floor_log2(fc_cols_c(n1));
-  } else {
-    R.bA = std::min({6, floor_log2(LDM_CAP / n1), ctz(n2)});
-    R.bB = std::min(floor_log2((n2 <= LDM_CAP_B ? LDM_CAP_B : LDM_CAP) / n2), ctz(n1));
-    R.bC = R.bA;
+  // The passes' bytes and operations go with the transform length, and half of
+  // the planned one still holds the grid: compiled passes run at L / 2 (half
+  // of n1 down to 256, else half of n2) wherever the correction of its images
+  // holds.  Not for a length that is the spectrum's period by request
+  // (wrap_k = 0), nor with row groups (a tile's moments need all its rows).
+  R.half = false;
+  R.tL = R.plan.L;
+  R.tn1 = R.plan.n1;
+  R.tn2 = R.plan.n2;
+  R.cell_tiles = R.n_cell = 0;
+  const bool halves = R.plan.n1 >= 512 || R.plan.n2 >= 128;
+  if (R.may_half && R.plan.fc && R.plan.wrap_k > 0 && R.fill_groups == 1 && halves) {
+    int w = R.tile_w;
+    if (!R.r.tile_w)
+      while (w > MIN_TILE_W && !half_ok(R, w)) w >>= 1;
+    const int64_t gap = R.plan.L / 2 - R.nv;
+    const int64_t tiles = (V + w - 1) / w, per = gap * 2 / 5 / w;
+    if (half_ok(R, w) && (tiles + per - 1) / per <= IMG_MAX_CELLS &&
+        fill_tile_bytes(R.m_cap, w) + (size_t)tile_moment_lds(R.m_cap, w) <= (size_t)FILL_LDS_MAX) {
+      R.half = true;
+      R.tile_w = w;
+      R.tL = R.plan.L / 2;
+      if (R.plan.n1 >= 512) R.tn1 = R.plan.n1 / 2;
+      else R.tn2 = R.plan.n2 / 2;
+      R.cell_tiles = (int)per;
+      R.n_cell = (int)((tiles + per - 1) / per);
+    }
   }
+  R.n_tiles = (int)((V + R.tile_w - 1) / R.tile_w);
+  if (R.plan.fc) {
+    R.bX[0] = floor_log2(R.narrow_a ? FC_COLS_A_NARROW : fc_cols_a(R.tn1));
+    R.bX[1] = floor_log2(fc_rows_b(R.tn2));
+    R.bX[2] = floor_log2(R.narrow_c ? FC_COLS_C_NARROW : fc_cols_c(R.tn1));
+  } else {
+    R.bX[0] = std::min({6, floor_log2(LDM_CAP / R.tn1), ctz(R.tn2)});
+    R.bX[1] = std::min(floor_log2((R.tn2 <= LDM_CAP_B ? LDM_CAP_B : LDM_CAP) / R.tn2), ctz(R.tn1));
+    R.bX[2] = R.bX[0];
+  }
+  return 0;
+}
+
+// Image items of a request with n_cell cells: (cell, part of the nodes).
+int image_parts(int n_cell) { return std::max(1, (n_cell * IMG_NODES + IMG_TARGETS - 1) / IMG_TARGETS); }
+int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
+
+// Workgroups per pass B row block (Req::n_share) for requests reqs[0..n)
+// that run together.  A compiled pass B workgroup walks every pair of its
+// row block; when a launch has few row blocks (a 500,001-point grid at
+// 512 x 2048: 512 workgroups, two per CU) the device runs them at two waves
+// per SIMD or fewer, latency-bound.  The pairs then go to several workgroups
+// (pass C adds their partial spectra): as many as fit FC_B_SPLIT_WGS_PER_CU
+// workgroups per CU at once, with FC_B_SPLIT_MIN_PAIRS pairs each; every
+// share costs an inverse transform and 8 tL bytes written and read.
+constexpr int FC_B_SPLIT_WGS_PER_CU = 4;
+constexpr int FC_B_SPLIT_MIN_PAIRS = 2;
+constexpr int FC_B_SPLIT_MAX = 4;
+constexpr double HALF_MIN_POINTS = 1 << 19;
+constexpr int FC_A_NARROW_PER_CU = 1, FC_C_NARROW_PER_CU = 1;
+void choose_split_b(Req* reqs, int n, int n_cu) {
+  // Half-length transforms pay where the launch's passes are more than a chain
+  // of latencies: below HALF_MIN_POINTS (pairs times planned length) the
+  // shorter passes take as long as the whole ones and the correction is extra.
+  double points = 0;
+  for (int i = 0; i < n; ++i) points += (double)((reqs[i].m_cap + 1) / 2) * (double)reqs[i].plan.L;
+  for (int i = 0; i < n; ++i) reqs[i].may_half = points >= HALF_MIN_POINTS;
+  std::map<int, long long> cols_a, cols_c;  // compiled n1 -> wide column blocks of passes A and C
+  std::map<int, long long> blocks, images;  // compiled pass B class (N2) -> row blocks, image items of the launch
+  for (int i = 0; i < n; ++i) {
+    Req& R = reqs[i];
+    R.narrow_a = R.narrow_c = false;
+    if (plan_exec(R)) continue;  // reported by layout_request
+    if (!R.plan.fc) continue;
+    cols_a[R.tn1] += (long long)((R.m_cap + 1) / 2) * (R.tn2 >> R.bX[0]);
+    cols_c[R.tn1] += R.tn2 >> R.bX[2];
+    blocks[R.tn2] += R.tn1 >> R.bX[1];
+    images[R.tn2] += image_items(R.n_cell);
+  }
+  for (int i = 0; i < n; ++i) {
+    Req& R = reqs[i];
+    R.split_b = R.n_share = 1;
+    if (!R.plan.fc) continue;
+    if (fc_narrow(R.tn1)) {
+      R.narrow_a = cols_a[R.tn1] < (long long)FC_A_NARROW_PER_CU * n_cu;
+      R.narrow_c = cols_c[R.tn1] < (long long)FC_C_NARROW_PER_CU * n_cu;
+    }
+    const int pairs = (R.m_cap + 1) / 2, rb = R.tn1 >> R.bX[1];
+    // whole length: two shares at most (the workspace holds two)
+    const long long room = std::max<long long>(0, (long long)FC_B_SPLIT_WGS_PER_CU * n_cu - images[R.tn2]);
+    int ns = (int)std::min<long long>(room / blocks[R.tn2], pairs / FC_B_SPLIT_MIN_PAIRS);
+    ns = std::min(ns, R.half ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);
+    if (R.half && ns > 2) ns = std::min(ns, pairs - 1 - pairs / 8);  // they share Y's unused half with the moments
+    if (ns > 1) {
+      R.n_share = ns;
+      R.split_b = 2;
+    }
+  }
+}
+
+// Workspace of one request (tile width, pass splits and the offsets of its
+// buffers from `total`, which it advances); shared by the batch layout and
+// radis_ldm_request_bytes.
+int layout_request(Req& R, size_t& total) {
+  const int rc = plan_exec(R);
+  if (rc) return rc;
+  const int64_t V = R.nv + 1;
+  R.stride = (int64_t)align_up((size_t)V, 64);
+  R.bA = R.bX[0];
+  R.bB = R.half ? 0 : R.bX[1];  // (the run-time-sized pass B's; the item numbers of a half-length one go past n1 >> bX)
+  R.bC = R.bX[2];
   const int pcap = (R.m_cap + 1) / 2;
   // LDM: pcap pairs of rows, rows 2p and 2p+1 interleaved (element n of row
   // 2p+h at float 2n+h of pair p): pass A reads each element pair as one float2
   R.off_ldm = total; total = align_up(total + (size_t)pcap * 2 * R.stride * 4, 256);
-  R.off_y = total;   total = align_up(total + (size_t)pcap * R.plan.L * 8, 256);
+  // one partial spectrum of length L (two of L / 2)
   R.off_b = total;   total = align_up(total + (size_t)R.plan.L * 8, 256);
-  // pass B's second share of the pairs (split pass B)
-  R.off_b2 = total;  if (R.split_b > 1) total = align_up(total + (size_t)R.plan.L * 8, 256);
+  // Y, for the whole length whatever runs (a request's workspace does not
+  // depend on its conditions); half-length transforms use its first half, and
+  // their correction and further partial spectra lie in the second
+  R.off_y = total;   total = align_up(total + (size_t)pcap * R.plan.L * 8, 256);
+  R.off_share = R.off_b;
+  if (R.half) {
+    size_t o = align_up(R.off_y + (size_t)pcap * R.tL * 8, 256);
+    R.off_img = o; o = align_up(o + (size_t)R.n_cell * IMG_NODES * 8, 256);
+    // N_L <= M/2, as N_G >= 2
+    R.off_mom = o; o = align_up(o + (size_t)R.n_tiles * std::max(1, std::min(R.m_cap / 2, LDM_MAX_AX)) * 16, 256);
+    if (R.n_share > 2) {
+      R.off_share = o;
+      o += (size_t)R.n_share * R.tL * 8;
+    }
+    R.off_free = align_up(o, 256);
+    if (o > total) return fail(RADIS_LDM_EINVAL, "internal: half-length buffers exceed the workspace");
+    R.off_b2 = R.off_y;
+  } else {
+    // pass B's second share of the pairs
+    R.off_b2 = total; if (R.split_b > 1) total = align_up(total + (size_t)R.plan.L * 8, 256);
+  }
   R.off_rows = total; total = align_up(total + (size_t)R.m_cap * 16, 256);
   // axis partials: at most one per chunk, plus the two partial blocks at the window edges
   R.off_axp = total; total = align_up(total + (size_t)((R.i1 - R.i0 + LDM_AX_CHUNK - 1) / LDM_AX_CHUNK + 2) * 32, 256);
@@ -860,7 +987,13 @@ int check_layout(const Req& R, size_t total) {
                   R.off_b + (size_t)R.plan.L * 8 <= total &&
                   (R.split_b == 1 || R.off_b2 + (size_t)R.plan.L * 8 <= total) && R.off_rows + (size_t)R.m_cap * 16 <= total &&
                   R.off_axp + parts * 32 <= total && (size_t)R.n_axp <= parts &&
-                  R.off_wrap + (size_t)R.wrap_rows * R.plan.wrap_k * 4 <= total;
+                  R.off_wrap + (size_t)R.wrap_rows * R.plan.wrap_k * 4 <= total &&
+                  R.off_share + (size_t)(R.n_share - 1) * (R.half ? (size_t)R.tL * 8 : R.off_b2 - R.off_b) + (size_t)R.tL * 8 <= total &&
+                  (!R.half || (R.tL * 2 == R.plan.L && (size_t)R.tL >= V && (long long)R.n_cell * R.cell_tiles >= R.n_tiles &&
+                               R.off_y + (size_t)((R.m_cap + 1) / 2) * R.tL * 8 <= R.off_img &&
+                               R.off_img + (size_t)R.n_cell * IMG_NODES * 8 <= R.off_mom &&
+                               R.off_mom + (size_t)R.n_tiles * std::max(1, std::min(R.m_cap / 2, LDM_MAX_AX)) * 16 <=
+                                   (R.n_share > 2 ? R.off_share : total)));
   return ok ? 0 : fail(RADIS_LDM_EINVAL, "internal: request workspace layout exceeds its %zu bytes", total);
 }
 
@@ -877,7 +1010,8 @@ struct LdmItemPlan {
   long long hi_a, hi_e;         // lines [hi_a, hi_e) scanned in chunks
   int n_lo, n_g, n_hi;          // items of the three axis parts
   int n_wrap, n_fill, pcap, n_colA, n_rowB, n_colC;
-  int split_b;                  // pass B items per row block (n_rowB counts them all)
+  int split_b;                  // pass B's item numbers are y * split_b + z
+  int n_img, img_parts;         // image items (half-length transforms), parts per cell
 };
 
 // Item i of the request (job field 0), i < plan_items(P).
@@ -906,8 +1040,10 @@ __host__ __device__ inline int4 plan_item(const LdmItemPlan& P, int i) {
   if (k < P.n_wrap) return make_int4(0, k, 0, 0);                 // L-axis node pair
   if ((k -= P.n_wrap) < P.n_fill) return make_int4(0, k, 0, 0);  // fill tile
   if ((k -= P.n_fill) < P.pcap * P.n_colA) return make_int4(0, k / P.n_colA, k % P.n_colA, 0);  // (pair, column block)
-  if ((k -= P.pcap * P.n_colA) < P.n_rowB) return make_int4(0, k / P.split_b, k % P.split_b, 0);  // pass B (row block, share)
-  return make_int4(0, 0, k - P.n_rowB, 0);                        // pass C column block
+  if ((k -= P.pcap * P.n_colA) < P.n_rowB) return make_int4(0, k / P.split_b, k % P.split_b, 0);  // pass B, number k = y * split_b + z
+  if ((k -= P.n_rowB) < P.n_colC) return make_int4(0, 0, k, 0);   // pass C column block
+  k -= P.n_colC;
+  return make_int4(0, k / P.img_parts, k % P.img_parts, 0);       // image item (cell, part of the nodes), after plan_items
 }
 
 namespace {
@@ -945,13 +1081,15 @@ LdmItemPlan item_plan(const radis_ldm_db& db, Req& R) {
     P.n_lo = chunks(R.i0, R.i1);
   }
   R.n_axp = P.n_lo + P.n_g + P.n_hi;
-  P.n_wrap = (R.wrap_rows + 1) / 2;
+  P.n_wrap = R.half ? 0 : (R.wrap_rows + 1) / 2;
   P.n_fill = R.n_tiles * R.fill_groups;  // item y = tile * fill_groups + group
   P.pcap = (R.m_cap + 1) / 2;
-  P.n_colA = R.plan.n2 >> R.bA;
+  P.n_colA = R.tn2 >> R.bX[0];
   P.split_b = R.split_b;
-  P.n_rowB = (R.plan.n1 >> R.bB) * R.split_b;
-  P.n_colC = R.plan.n2 >> R.bC;
+  P.n_rowB = (R.tn1 >> R.bX[1]) * R.n_share;
+  P.n_colC = R.tn2 >> R.bX[2];
+  P.img_parts = image_parts(R.n_cell);
+  P.n_img = image_items(R.n_cell);
   return P;
 }
 

@@ -31,20 +31,8 @@
 // B, two launches later, is the first reader of the table.
 #pragma once
 #include "ldm_fftc.h"
+#include "ldm_image.h"
 #include "ldm_kernels.h"
-
-struct WrapNode {
-  double omE, omE2, E;  // 1 - e^-a, 1 - e^-2a, e^-a for the period's a = 2 pi gamma / period
-};
-
-__device__ __forceinline__ WrapNode wrap_node(double gamma, double period) {
-  const double a = 6.283185307179586 * gamma / period;
-  WrapNode w;
-  w.omE = -expm1(-a);
-  w.omE2 = -expm1(-2.0 * a);
-  w.E = exp(-a);
-  return w;
-}
 
 // P(d) of one period in the overflow-free form (1/L)(1 - E^2) / ((1 - E)^2 +
 // 4 E sin^2(pi d / L)) (sinh and cosh multiplied by 2 e^-a); s2 = sin^2(pi d / L)
@@ -131,10 +119,10 @@ __device__ __forceinline__ void wrap_item(const LdmJob* __restrict__ jobs, const
 // (items[0, n_wrap)), the others the fill tiles that follow them in the
 // item list.  One kernel per line-list variant (PLAIN: no isotopologue,
 // shift or n_self column; the host picks), so each gets its own register
-// allocation: the plain kernel needs the fewest; GROUPED (fill_tile) only
-// when some request's LDM is taller than a tile.  The dynamic LDS holds the
+// allocation: the plain kernel needs the fewest; GROUPED and HALF (fill_tile)
+// only when some request needs them.  The dynamic LDS holds the
 // larger of a fill tile (or row group) and an image-correction item.
-template <bool PLAIN, bool GROUPED>
+template <bool PLAIN, bool GROUPED, bool HALF>
 __global__ __launch_bounds__(LDM_FILL_T, 4) void k_fill(const LdmJob* __restrict__ jobs,
                                                      const LdmAxes* __restrict__ axes,
                                                      const int4* __restrict__ items, int n_wrap, LdmDb db) {
@@ -147,6 +135,6 @@ __global__ __launch_bounds__(LDM_FILL_T, 4) void k_fill(const LdmJob* __restrict
   const LdmJob& J = jobs[it.x];
   const LdmAxes& A = axes[it.x];
   if (A.m == 0 || J.status) return;
-  if (J.noneq) fill_tile<true, PLAIN, GROUPED>(J, A, it, db, acc);
-  else fill_tile<false, PLAIN, GROUPED>(J, A, it, db, acc);
+  if (J.noneq) fill_tile<true, PLAIN, GROUPED, HALF>(J, A, it, db, acc);
+  else fill_tile<false, PLAIN, GROUPED, HALF>(J, A, it, db, acc);
 }
