@@ -1267,10 +1267,21 @@ int radis_ldm_slit_convolve(const float* in, int64_t n, const float* slit, int32
   const char *a0 = (const char*)in, *a1 = a0 + n * 4, *b0 = (const char*)out, *b1 = b0 + n * 4;
   const char *s0 = (const char*)slit, *s1 = s0 + (int64_t)k * 4;
   if ((a0 < b1 && b0 < a1) || (s0 < b1 && b0 < s1)) return fail(RADIS_LDM_EINVAL, "output overlaps the input or the slit");
-  const int64_t grid = (n + SLIT_OUT - 1) / SLIT_OUT;
-  if (grid > INT32_MAX) return fail(RADIS_LDM_ERANGE, "grid too long");
-  hipLaunchKernelGGL(k_slit_conv, dim3((unsigned)grid), dim3(SLIT_T), 0, (hipStream_t)stream, in, (long long)n, slit, k,
-                     scale, out);
+  // outputs per lane: the more the fewer LDS reads per product, but a workgroup
+  // for every CU comes first
+  const auto launch_slit = [&](auto tile, auto kernel) -> int {
+    using Tile = decltype(tile);
+    const int64_t grid = (n + Tile::OUT - 1) / Tile::OUT;
+    if (grid > INT32_MAX) return fail(RADIS_LDM_ERANGE, "grid too long");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(Tile::T), 0, (hipStream_t)stream, in, (long long)n, slit, k,
+                       scale, out);
+    return 0;
+  };
+  int rc;
+  if (n >= 256 * SlitTile<16, 4>::OUT) rc = launch_slit(SlitTile<16, 4>{}, k_slit_conv<16, 4>);
+  else if (n >= 256 * SlitTile<8, 4>::OUT) rc = launch_slit(SlitTile<8, 4>{}, k_slit_conv<8, 4>);
+  else rc = launch_slit(SlitTile<4, 8>{}, k_slit_conv<4, 8>);
+  if (rc) return rc;
   HIPCHK(hipGetLastError());
   return 0;
 }

@@ -3,54 +3,109 @@
 // (radis/tools/slit.py:477-757, scipy.signal.oaconvolve(I, slit, 'same') *
 // wstep).  Here the sum is direct:
 //   out[i] = scale * sum_j slit[j] * in[i + c - j],  c = (k - 1) / 2,
-// with in[] outside [0, n) read as zero.  A workgroup takes SLIT_OUT
-// consecutive outputs; the slit is consumed in LDS chunks of SLIT_KCH taps
-// together with the input window those taps reach.  Lanes read consecutive
-// input words and the same slit word (a broadcast), so the LDS reads are
-// conflict-free.  Slit widths are a few hundred to a few thousand grid
-// points against grids of 10^5-10^6, so this is a small kernel next to the
-// synthesis.  Products are FP32 and the running sums FP64, so the error is
-// that of one FP32 product per tap, whatever the slit length.
+// with in[] outside [0, n) read as zero: k products and additions per point in
+// FP64 (the product of two FP32 values is exact there), so every output is the
+// exact sum rounded to FP32, whatever the slit length and the range of the
+// spectrum, and a value that is not finite reaches the outputs within the
+// slit's reach only.
+//
+// Bound by FP64 multiply-adds (about 56 TFLOP/s here; the FP64 matrix products
+// of a Toeplitz form ran at 43).  With the taps reversed,
+//   out[i] = sum_m h[m] x[i + m],  x[q] = in[q + c - k + 1],
+// a lane takes R consecutive outputs and walks the taps in groups of R: 2 R
+// inputs in registers give R^2 products, and the next group needs R new ones
+// (an earlier form with a tap and an input read from LDS for every product
+// spent more on the reads and conversions than on the sums).  The inputs lie
+// transposed in LDS (element e at row e % R, column e / R), so the lanes'
+// reads are consecutive; the taps are read as broadcasts.  The waves of a
+// workgroup take the same 64 R outputs and a share of the taps each, and add
+// their sums at the end.
 #pragma once
 
-#define SLIT_T 256
-#define SLIT_PER 4                    // outputs per thread
-#define SLIT_OUT (SLIT_T * SLIT_PER)  // outputs per workgroup
-#define SLIT_KCH 2048                 // slit taps per LDS chunk
+#define SLIT_KCH 2048  // slit taps per LDS chunk
 
-__global__ __launch_bounds__(SLIT_T) void k_slit_conv(const float* __restrict__ in, long long n,
-                                                    const float* __restrict__ slit, int k, double scale,
-                                                    float* __restrict__ out) {
-  __shared__ float s_in[SLIT_OUT + SLIT_KCH];
-  __shared__ float s_k[SLIT_KCH];
-  const long long o0 = (long long)blockIdx.x * SLIT_OUT;
-  const int c = (k - 1) / 2;
-  double acc[SLIT_PER];
+template <int R, int NW>
+struct SlitTile {
+  static constexpr int T = 64 * NW, OUT = 64 * R;
+  static constexpr int COLS = 64 + SLIT_KCH / R + 1;          // columns of the input window
+  static constexpr int S = COLS + (COLS % 2 == 0 ? 5 : 4);     // odd row stride
+  static constexpr int RED = NW * R * 65 * 8, STAGE = SLIT_KCH * 8 + R * S * 4;
+  static constexpr int LDS = RED > STAGE ? RED : STAGE;
+};
+
+template <int R, int NW>
+__global__ __launch_bounds__(64 * NW) void k_slit_conv(const float* __restrict__ in, long long n,
+                                                       const float* __restrict__ slit, int k, double scale,
+                                                       float* __restrict__ out) {
+  using Tile = SlitTile<R, NW>;
+  constexpr int S = Tile::S, T = Tile::T;
+  __shared__ __align__(16) char lds[Tile::LDS];
+  double* const s_h = reinterpret_cast<double*>(lds);               // [SLIT_KCH]
+  float* const s_x = reinterpret_cast<float*>(lds + SLIT_KCH * 8);  // [R][S]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long o0 = (long long)blockIdx.x * Tile::OUT;
+  const long long x0 = o0 + (k - 1) / 2 - (k - 1);  // in[] index of x[o0]
+  double acc[R];
 #pragma unroll
-  for (int q = 0; q < SLIT_PER; ++q) acc[q] = 0.0;
-  for (int j0 = 0; j0 < k; j0 += SLIT_KCH) {
-    const int kc = (k - j0 < SLIT_KCH) ? k - j0 : SLIT_KCH;
-    __syncthreads();  // the previous chunk has been consumed
-    for (int e = threadIdx.x; e < kc; e += SLIT_T) s_k[e] = slit[j0 + e];
-    // taps j0..j0+kc-1 of outputs o0..o0+SLIT_OUT-1 read in[base .. base+SLIT_OUT+kc-2]
-    const long long base = o0 + c - j0 - kc + 1;
-    for (int e = threadIdx.x; e < SLIT_OUT + kc - 1; e += SLIT_T) {
-      const long long x = base + e;
-      s_in[e] = (x >= 0 && x < n) ? in[x] : 0.0f;
+  for (int r = 0; r < R; ++r) acc[r] = 0.0;
+  for (int m0 = 0; m0 < k; m0 += SLIT_KCH) {
+    const int kc = k - m0 < SLIT_KCH ? k - m0 : SLIT_KCH;
+    if (m0) __syncthreads();  // the previous chunk has been consumed
+    for (int m = threadIdx.x; m < kc; m += T) s_h[m] = (double)slit[k - 1 - (m0 + m)];
+    for (int e = threadIdx.x; e < Tile::OUT + kc - 1; e += T) {
+      const long long q = x0 + m0 + e;
+      s_x[(e % R) * S + e / R] = (q >= 0 && q < n) ? in[q] : 0.0f;
     }
     __syncthreads();
+    // whole groups of R taps, a contiguous share per wave
+    const int groups = kc / R, per = (groups + NW - 1) / NW;
+    const int g0 = wave * per, g1 = g0 + per < groups ? g0 + per : groups;
+    auto column = [&](int g, double (&v)[R]) {
 #pragma unroll
-    for (int q = 0; q < SLIT_PER; ++q) {
-      const int lo = threadIdx.x + q * SLIT_T;  // in[o0 + lo + c - j] = s_in[lo + kc - 1 - (j - j0)]
-      const float* w = s_in + lo + kc - 1;
-      double a = acc[q];
-      for (int jj = 0; jj < kc; ++jj) a += (double)(s_k[jj] * w[-jj]);
-      acc[q] = a;
+      for (int r = 0; r < R; ++r) v[r] = (double)s_x[r * S + lane + g];
+    };
+    // taps of group g over the columns lo (g) and hi (g + 1)
+    auto products = [&](int g, const double (&lo)[R], const double (&hi)[R]) {
+#pragma unroll
+      for (int m = 0; m < R; m += 2) {
+        const double2 h = *reinterpret_cast<const double2*>(s_h + g * R + m);
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = __builtin_fma(h.x, r + m < R ? lo[r + m] : hi[r + m - R], acc[r]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = __builtin_fma(h.y, r + m + 1 < R ? lo[r + m + 1] : hi[r + m + 1 - R], acc[r]);
+      }
+    };
+    double a[R], b[R];
+    if (g0 < g1) column(g0, a);
+    for (int g = g0; g < g1; g += 2) {
+      column(g + 1, b);
+      products(g, a, b);
+      if (g + 1 == g1) break;
+      column(g + 2, a);
+      products(g + 1, b, a);
+    }
+    // the remaining taps, one each for the last waves in turn
+    for (int m = groups * R + (NW - 1 - wave); m < kc; m += NW) {
+      const double h = s_h[m];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int e = r + m;
+        acc[r] = __builtin_fma(h, (double)s_x[(e % R) * S + lane + e / R], acc[r]);
+      }
     }
   }
+  // the waves' sums: output lane * R + r of wave w at [w][r][lane], rows of 65
+  __syncthreads();
+  double* const red = reinterpret_cast<double*>(lds);
 #pragma unroll
-  for (int q = 0; q < SLIT_PER; ++q) {
-    const long long o = o0 + threadIdx.x + q * SLIT_T;
-    if (o < n) out[o] = (float)(acc[q] * (double)scale);
+  for (int r = 0; r < R; ++r) red[(wave * R + r) * 65 + lane] = acc[r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < Tile::OUT; e += T) {
+    if (o0 + e >= n) break;
+    const double* p = red + (e % R) * 65 + e / R;
+    double s = p[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += p[w * R * 65];
+    out[o0 + e] = (float)(s * scale);
   }
 }
