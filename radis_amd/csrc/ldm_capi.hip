@@ -447,7 +447,7 @@ struct LaunchSet {
   size_t fill_lds;
   bool fill_grouped;  // the fill kernel with row groups (some request's LDM is taller than a tile)
   bool fill_half;     // the fill kernel with tile moments (some request runs half-length transforms)
-  bool tile_bounds;  // run k_tile_bounds (else the items hold valid tile line ranges)
+  bool tile_bounds;  // find the tiles' line ranges (else the items hold valid ones)
   int n_cu;
 };
 
@@ -457,7 +457,11 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
   const int4* items = X.items;
   const LdmJob* cj = X.jobs;
   const LdmAxes* ca = X.axes;
-  if (X.n_axis) launch(b, timed, slot, 0, k_axis, dim3(X.n_axis), dim3(256), 0, s, X.jobs, items, dbd);
+  // width extremes, and the fill tiles' line ranges behind them
+  const int n_bounds = X.tile_bounds ? X.n_fill : 0;
+  if (X.n_axis + n_bounds)
+    launch(b, timed, slot, 0, k_axis, dim3(X.n_axis + (n_bounds + 3) / 4), dim3(256), 0, s, X.jobs, items, X.n_axis,
+           X.items + X.n_axis + X.n_wrap, n_bounds, dbd);
   launch(b, timed, slot, 1, k_finalize, dim3(X.n_req), dim3(256), 0, s, X.jobs, X.axes, X.res, dbd);
   items += X.n_axis;
   // The image-correction items run as the first workgroups of the fill
@@ -466,9 +470,6 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
   // pass B, cost more in cross-stream events than the kernel).
   const int4* wrap_fill = items;  // wrap items, then fill items
   items += X.n_wrap;
-  if (X.n_fill && X.tile_bounds)
-    launch(b, timed, slot, 2, k_tile_bounds, dim3((X.n_fill + 3) / 4), dim3(256), 0, s, X.jobs,
-           X.items + (items - X.items), X.n_fill, dbd);
   if (X.n_wrap + X.n_fill) {
     const size_t lds = X.n_wrap ? std::max(X.fill_lds, (size_t)LDM_WRAP_LDS * sizeof(float2)) : X.fill_lds;
     const dim3 grid(X.n_wrap + X.n_fill);

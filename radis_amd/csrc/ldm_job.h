@@ -26,8 +26,10 @@
 constexpr int ldm_fill_pad(int tile_w) { return tile_w >= 64 ? 3 : 2; }
 #define LDM_AX_CHUNK 4096  // lines per axis-reduction workgroup (16 per lane)
 #define LDM_SKY_BLOCK 4096  // lines per width-candidate block
-#define LDM_SKY_GROUP_MIN 8  // fewest candidate blocks per k_axis workgroup
-#define LDM_SKY_WGS 600       // most candidate workgroups of k_axis per request (about)
+// most candidate workgroups of k_axis per request (about): one block each up to
+// there (a block's candidates, a few dozen to a few hundred, are one pass of
+// the workgroup's threads; groups of 8 left a 300,000-line window to 9 workgroups)
+#define LDM_SKY_WGS 1024
 static_assert(LDM_AX_CHUNK == LDM_SKY_BLOCK, "a partial block is one scan chunk");
 #define LDM_TW_LO_BITS 10  // four-step twiddle split W_L^e = hi[e>>10] * lo[e&1023]
 #define LDM_NFOLD_MAX 100000

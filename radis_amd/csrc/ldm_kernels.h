@@ -1,8 +1,8 @@
 // HIP kernels of the DIT/LDM pipeline (gfx950).
 //
-//   k_axis        per-request min/max of the line widths (LDM axis limits)
+//   k_axis        per-request min/max of the line widths (LDM axis limits); line
+//                 range of every fill tile (binary search on nu0)
 //   k_finalize    LDM axes, N_G, N_L, per-row alias-fold counts and norms
-//   k_tile_bounds line range of every fill tile (binary search on nu0)
 //   k_fill        line parameters + bit-exact np.interp indices + 2x2x2
 //                 weights, scattered into an LDS tile [M][W] and flushed once
 //   k_fft_a       four-step pass 1: N1-point DFTs over strided columns of two
@@ -157,6 +157,61 @@ __device__ __forceinline__ unsigned long long double_to_bits(double d) {
   return (unsigned long long)__double_as_longlong(d);
 }
 
+// First index in [lo, hi) with nu0[i] >= v, by a whole wave: 64 probes per
+// round narrow the range 64-fold (ballot + popcount), so ~log64(n) dependent
+// loads instead of log2(n).  Every lane of the wave must call it with the same
+// arguments.
+__device__ __forceinline__ long long lower_bound_nu_wave(const double* __restrict__ nu0, long long lo, long long hi,
+                                                         double v) {
+  const int lane = threadIdx.x & 63;
+  // invariant: the answer lies in [lo, hi]
+  while (hi - lo > 64) {
+    const long long step = (hi - lo + 63) >> 6;
+    const long long idx = lo + (long long)(lane + 1) * step - 1;
+    const bool lt = idx < hi && nu0[idx] < v;
+    // probes are sorted: the c probes below v are lanes 0..c-1
+    const long long c = __popcll(__ballot(lt));
+    const long long nhi = lo + (c + 1) * step - 1;
+    lo += c * step;
+    hi = nhi < hi ? nhi : hi;
+  }
+  const long long idx = lo + lane;
+  const bool lt = idx < hi && nu0[idx] < v;
+  return lo + __popcll(__ballot(lt));
+}
+
+// ---------------------------------------------------------------------------
+// tile_bounds: for every fill tile [k_lo, k_hi) the line range that can
+// put a corner inside it: k0 in [k_lo-1, k_hi-1].  A line's np.interp
+// position is monotone in its shifted centre, so a search on nu0 widened by
+// the largest pressure shift (plus 1e-3 of a grid step for rounding) is a
+// superset; k_fill filters each line by its exact k0.  Item = (job, tile).
+// Run by workgroups of the k_axis launch behind its axis items (neither reads
+// what the other writes): a launch of its own took 5 us and its gap.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void tile_bounds(const LdmJob* __restrict__ jobs, int4* __restrict__ items, int g,
+                                            int n_items, const LdmDb& db) {
+  if (g >= n_items) return;  // g: one item per wave
+  const int4 it = items[g];
+  const LdmJob& J = jobs[it.x];
+  const long long t = it.y / J.fill_groups;  // item y = tile * fill_groups + row group
+  const long long k_lo = t * J.tile_w;
+  long long k_hi = k_lo + J.tile_w;
+  if (k_hi > J.v) k_hi = J.v;
+  long long lo, hi;
+  if (k_lo <= 1) lo = J.i0;
+  else lo = lower_bound_nu_wave(db.nu0, J.i0, J.i1, J.wmin + (double)(k_lo - 1) * J.delta_w - J.shift_margin);
+  if (k_hi >= J.nv) hi = J.i1;
+  else hi = lower_bound_nu_wave(db.nu0, lo, J.i1, J.wmin + (double)k_hi * J.delta_w + J.shift_margin);
+  if (hi < lo) hi = lo;
+  // the range goes into the tile's own work item (offsets from the window
+  // start; windows hold < 2^31 lines), so the fill reads it with the item
+  if ((threadIdx.x & 63) == 0) {
+    items[g].z = (int)(lo - J.i0);
+    items[g].w = (int)(hi - J.i0);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // k_axis: min/max of the Lorentzian (and, for several isotopologues, the
 // Gaussian) FWHM over each request's window; radis/lbl/broadening.py:1823-1852.
@@ -173,9 +228,19 @@ __device__ __forceinline__ unsigned long long double_to_bits(double d) {
 // (rounding is monotone, and different float inputs move exp's argument by
 // far more than an ulp), so the extremes over the candidates are bit-identical
 // to those over every line.
+//
+// A chain of latencies, not of bytes: one candidate block per workgroup and
+// every load of a scanned chunk in flight at once.  1 M lines with isotopologue,
+// shift and n_self columns, window of a third: 20.6 us + 5.1 us for the tile
+// bounds in a launch of their own -> 9.1 us; 32 windows of a 2 M-line list
+// 26.8 -> 19.1 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const int4* __restrict__ items,
-                                              LdmDb db) {
+__global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const int4* __restrict__ items, int n_axis,
+                                              int4* __restrict__ tiles, int n_tiles, LdmDb db) {
+  if ((int)blockIdx.x >= n_axis) {
+    tile_bounds(jobs, tiles, 4 * ((int)blockIdx.x - n_axis) + (int)(threadIdx.x >> 6), n_tiles, db);
+    return;
+  }
   const int4 it = items[blockIdx.x];
   LdmJob& J = jobs[it.x];
   unsigned long long lmin = ~0ull, lmax = 0ull, gmin = ~0ull, gmax = 0ull;
@@ -219,56 +284,100 @@ __global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const i
   } else {
     const long long a = J.i0 + it.z;
     const long long e = a + it.w;
-    // FP32 widths of this lane's lines stay in registers; only the FP32 argmin
-    // and argmax are re-evaluated in FP64.  If another of the lane's lines is
-    // within the FP32 error bound of an extreme (a near tie), every line of the
-    // lane is evaluated in FP64 (rare), so the exact FP64 extremes are found.
+    // FP32 widths of this lane's lines stay in registers; only the lines within
+    // the FP32 error bound of the workgroup's FP32 extremes are evaluated in
+    // FP64 (a line outside it cannot hold the FP64 extreme), about one each.
+    // Comparing within a lane instead had every wave take up to 16 FP64 powers
+    // in turn whenever two of one lane's 16 lines came close.
+    // The Gaussian widths of several isotopologues take the same two steps.
     constexpr int NPER = LDM_AX_CHUNK / 256;
-    float wf[NPER];
-    float fmin = 3.0e38f, fmax = -1.0f;
-    int kmin = -1, kmax = -1;
+    __shared__ float s_ext[4][4], s_dopp[LDM_MAX_ISO];
+    const bool gauss = !J.single_iso;
+    float wf[NPER], gf[NPER];
+    float fmin = 3.0e38f, fmax = -1.0f, hmin = 3.0e38f, hmax = -1.0f;
+    if (gauss) {
+      if (threadIdx.x < LDM_MAX_ISO) s_dopp[threadIdx.x] = (float)J.dopp[threadIdx.x];
+      __syncthreads();
+    }
+    // every load unconditional (the last line again past the end), so that
+    // HALF of a lane's lines are in flight together: a branch per line had each
+    // wait for its own
+    constexpr int HALF = NPER / 2;
+    const float* const nsp = db.n_self ? db.n_self : db.n_air;
+    auto line = [&](int k) { return min(a + threadIdx.x + (long long)k * 256, e - 1); };
+#pragma unroll
+    for (int k0 = 0; k0 < NPER; k0 += HALF) {
+      float ga[HALF], gs[HALF], na[HALF], ns[HALF];
+#pragma unroll
+      for (int k = 0; k < HALF; ++k) {
+        const long long i = line(k0 + k);
+        ga[k] = db.g_air[i];
+        gs[k] = db.g_self[i];
+        na[k] = db.n_air[i];
+        ns[k] = nsp[i];
+      }
+#pragma unroll
+      for (int k = 0; k < HALF; ++k) {
+        const float w = fwhm_lorentz_f32(J, ga[k], gs[k], na[k], ns[k]);
+        wf[k0 + k] = a + threadIdx.x + (long long)(k0 + k) * 256 < e ? w : -1.0f;
+        gf[k0 + k] = -1.0f;
+        if (wf[k0 + k] >= 0.0f) {
+          fmin = fminf(fmin, wf[k0 + k]);
+          fmax = fmaxf(fmax, wf[k0 + k]);
+        }
+      }
+    }
+    if (gauss) {
+      float nu[NPER];
+      int iso[NPER];
+#pragma unroll
+      for (int k = 0; k < NPER; ++k) {
+        nu[k] = (float)db.nu0[line(k)];
+        iso[k] = db.iso ? db.iso[line(k)] : 1;
+      }
+#pragma unroll
+      for (int k = 0; k < NPER; ++k) {
+        if (a + threadIdx.x + (long long)k * 256 < e) gf[k] = nu[k] * s_dopp[iso[k]];
+        if (gf[k] >= 0.0f) {
+          hmin = fminf(hmin, gf[k]);
+          hmax = fmaxf(hmax, gf[k]);
+        }
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      fmin = fminf(fmin, __shfl_xor(fmin, off));
+      fmax = fmaxf(fmax, __shfl_xor(fmax, off));
+      hmin = fminf(hmin, __shfl_xor(hmin, off));
+      hmax = fmaxf(hmax, __shfl_xor(hmax, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      const int w = threadIdx.x >> 6;
+      s_ext[0][w] = fmin; s_ext[1][w] = fmax; s_ext[2][w] = hmin; s_ext[3][w] = hmax;
+    }
+    __syncthreads();
+    auto low = [&](const float* v) { return fminf(fminf(v[0], v[1]), fminf(v[2], v[3])); };
+    auto high = [&](const float* v) { return fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])); };
+    fmin = low(s_ext[0]) * (1.0f + 2e-5f);
+    fmax = high(s_ext[1]) * (1.0f - 2e-5f);
+    hmin = low(s_ext[2]) * (1.0f + 2e-6f);
+    hmax = high(s_ext[3]) * (1.0f - 2e-6f);
+    unsigned wl = 0, wg = 0;  // this lane's lines within the bounds
 #pragma unroll
     for (int k = 0; k < NPER; ++k) {
-      const long long i = a + threadIdx.x + (long long)k * 256;
-      wf[k] = -1.0f;
-      if (i < e) {
-        const float na = db.n_air[i];
-        wf[k] = fwhm_lorentz_f32(J, db.g_air[i], db.g_self[i], na, db.n_self ? db.n_self[i] : na);
-        if (wf[k] < fmin) { fmin = wf[k]; kmin = k; }
-        if (wf[k] > fmax) { fmax = wf[k]; kmax = k; }
-      }
+      if (wf[k] >= 0.0f && (wf[k] <= fmin || wf[k] >= fmax)) wl |= 1u << k;
+      if (gf[k] >= 0.0f && (gf[k] <= hmin || gf[k] >= hmax)) wg |= 1u << k;
     }
-    bool tie = false;
-#pragma unroll
-    for (int k = 0; k < NPER; ++k) {
-      if (wf[k] >= 0.0f && k != kmin && wf[k] <= fmin * (1.0f + 2e-5f)) tie = true;
-      if (wf[k] >= 0.0f && k != kmax && wf[k] >= fmax * (1.0f - 2e-5f)) tie = true;
+    for (; wl; wl &= wl - 1) {
+      const long long i = line(__ffs(wl) - 1);
+      const unsigned long long bl = double_to_bits(fwhm_lorentz(J, db.g_air[i], db.g_self[i], db.n_air[i], nsp[i]));
+      lmin = bl < lmin ? bl : lmin;
+      lmax = bl > lmax ? bl : lmax;
     }
-    auto exact = [&](int k) {
-      const long long i = a + threadIdx.x + (long long)k * 256;
-      const double na = db.n_air[i];
-      return double_to_bits(fwhm_lorentz(J, db.g_air[i], db.g_self[i], na, db.n_self ? (double)db.n_self[i] : na));
-    };
-    if (kmin >= 0) {
-      if (!tie) {
-        lmin = exact(kmin);
-        lmax = exact(kmax);
-      } else {
-        for (int k = 0; k < NPER; ++k)
-          if (wf[k] >= 0.0f) {
-            const unsigned long long bl = exact(k);
-            lmin = bl < lmin ? bl : lmin;
-            lmax = bl > lmax ? bl : lmax;
-          }
-      }
-    }
-    if (!J.single_iso) {
-      for (long long i = a + threadIdx.x; i < e; i += blockDim.x) {
-        const int iso = db.iso ? db.iso[i] : 1;
-        const unsigned long long bg = double_to_bits(fwhm_gauss(db.nu0[i], J.dopp[iso]));
-        gmin = bg < gmin ? bg : gmin;
-        gmax = bg > gmax ? bg : gmax;
-      }
+    for (; wg; wg &= wg - 1) {
+      const long long i = line(__ffs(wg) - 1);
+      const unsigned long long bg = double_to_bits(fwhm_gauss(db.nu0[i], J.dopp[db.iso ? db.iso[i] : 1]));
+      gmin = bg < gmin ? bg : gmin;
+      gmax = bg > gmax ? bg : gmax;
     }
   }
   // wave reduction
@@ -497,70 +606,6 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
     res[blockIdx.x].wg_max = s_wg_max;
     res[blockIdx.x].wl_min = s_wl_min;
     res[blockIdx.x].wl_max = s_wl_max;
-  }
-}
-
-// first index in [lo, hi) with nu0[i] >= v
-__device__ __forceinline__ long long lower_bound_nu(const double* __restrict__ nu0, long long lo, long long hi,
-                                                    double v) {
-  while (lo < hi) {
-    const long long mid = lo + ((hi - lo) >> 1);
-    if (nu0[mid] < v) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-// Same result computed by a whole wave: 64 probes per round narrow the range
-// 64-fold (ballot + popcount), so ~log64(n) dependent loads instead of
-// log2(n).  Every lane of the wave must call it with the same arguments.
-__device__ __forceinline__ long long lower_bound_nu_wave(const double* __restrict__ nu0, long long lo, long long hi,
-                                                         double v) {
-  const int lane = threadIdx.x & 63;
-  // invariant: the answer lies in [lo, hi]
-  while (hi - lo > 64) {
-    const long long step = (hi - lo + 63) >> 6;
-    const long long idx = lo + (long long)(lane + 1) * step - 1;
-    const bool lt = idx < hi && nu0[idx] < v;
-    // probes are sorted: the c probes below v are lanes 0..c-1
-    const long long c = __popcll(__ballot(lt));
-    const long long nhi = lo + (c + 1) * step - 1;
-    lo += c * step;
-    hi = nhi < hi ? nhi : hi;
-  }
-  const long long idx = lo + lane;
-  const bool lt = idx < hi && nu0[idx] < v;
-  return lo + __popcll(__ballot(lt));
-}
-
-// ---------------------------------------------------------------------------
-// k_tile_bounds: for every fill tile [k_lo, k_hi) the line range that can
-// put a corner inside it: k0 in [k_lo-1, k_hi-1].  A line's np.interp
-// position is monotone in its shifted centre, so a search on nu0 widened by
-// the largest pressure shift (plus 1e-3 of a grid step for rounding) is a
-// superset; k_fill filters each line by its exact k0.  Item = (job, tile).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_tile_bounds(LdmJob* __restrict__ jobs, int4* __restrict__ items,
-                                                     int n_items, LdmDb db) {
-  // one wave per item
-  const int g = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  if (g >= n_items) return;
-  const int4 it = items[g];
-  LdmJob& J = jobs[it.x];
-  const long long t = it.y / J.fill_groups;  // item y = tile * fill_groups + row group
-  const long long k_lo = t * J.tile_w;
-  long long k_hi = k_lo + J.tile_w;
-  if (k_hi > J.v) k_hi = J.v;
-  long long lo, hi;
-  if (k_lo <= 1) lo = J.i0;
-  else lo = lower_bound_nu_wave(db.nu0, J.i0, J.i1, J.wmin + (double)(k_lo - 1) * J.delta_w - J.shift_margin);
-  if (k_hi >= J.nv) hi = J.i1;
-  else hi = lower_bound_nu_wave(db.nu0, lo, J.i1, J.wmin + (double)k_hi * J.delta_w + J.shift_margin);
-  if (hi < lo) hi = lo;
-  // the range goes into the tile's own work item (offsets from the window
-  // start; windows hold < 2^31 lines), so the fill reads it with the item
-  if ((threadIdx.x & 63) == 0) {
-    items[g].z = (int)(lo - J.i0);
-    items[g].w = (int)(hi - J.i0);
   }
 }
 
@@ -865,7 +910,7 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
   if (k_hi > J.v) k_hi = J.v;
   const LineConst C(J, A, db);
   const LineCols cols(db);
-  const unsigned lo = (unsigned)(J.i0 + it.z), hi = (unsigned)(J.i0 + it.w);  // written by k_tile_bounds
+  const unsigned lo = (unsigned)(J.i0 + it.z), hi = (unsigned)(J.i0 + it.w);  // written by tile_bounds
   // Thread t takes lines lo + t, lo + t + T, ...: every load instruction of
   // a wave reads 64 consecutive lines.  (Giving each lane its own run of
   // lines spreads a wave's loads over as many cache lines and pages as it has

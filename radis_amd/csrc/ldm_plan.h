@@ -1066,9 +1066,8 @@ LdmItemPlan item_plan(const radis_ldm_db& db, Req& R) {
     P.lo_a = R.i0;
     P.lo_e = fb0 * LDM_SKY_BLOCK;
     P.n_lo = chunks(P.lo_a, P.lo_e);
-    // at least LDM_SKY_GROUP_MIN blocks per workgroup (each partial costs
-    // the reduction a read), and at most about LDM_SKY_WGS workgroups
-    P.G = std::max<int64_t>(LDM_SKY_GROUP_MIN, (fb1 - fb0 + LDM_SKY_WGS - 1) / LDM_SKY_WGS);
+    // at most about LDM_SKY_WGS workgroups (each partial costs the reduction a read)
+    P.G = (fb1 - fb0 + LDM_SKY_WGS - 1) / LDM_SKY_WGS;
     P.g0 = fb0;
     P.fb1 = fb1;
     P.n_g = (int)((fb1 - fb0 + P.G - 1) / P.G);
