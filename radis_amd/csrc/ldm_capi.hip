@@ -284,12 +284,11 @@ int build_layout(radis_ldm_batch* b) {
   // point builds its tables the same way)
   for (auto& kv : sub_off)
     hipLaunchKernelGGL(k_twiddles, dim3((kv.first + 255) / 256), dim3(256), 0, b->ctx->side,
-                       (float2*)((char*)b->twmem + kv.second), kv.first, (float2*)nullptr, 0, (float2*)nullptr, 0ll);
+                       LdmTwiddles{(float2*)((char*)b->twmem + kv.second), nullptr, nullptr, kv.first, 0, 0});
   for (auto& kv : l_off) {
-    const long long nt = ((kv.first + 1023) >> LDM_TW_LO_BITS) + 1024;
-    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((nt + 255) / 256, 4096)), dim3(256), 0, b->ctx->side,
-                       (float2*)nullptr, 0, (float2*)nullptr, 0, (float2*)((char*)b->twmem + kv.second),
-                       (long long)kv.first);
+    const LdmTwiddles t{nullptr, nullptr, (float2*)((char*)b->twmem + kv.second), 0, 0, (long long)kv.first};
+    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((t.total() + 255) / 256, 4096)), dim3(256), 0,
+                       b->ctx->side, t);
   }
   HIPCHK(hipGetLastError());
   for (Req& R : b->reqs) {
@@ -1205,13 +1204,11 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   LdmJob J;
   fill_job(*db, R, base + o_work, out_dev, J);
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_put_job, dim3(1), dim3(64), 0, s, J, (LdmJob*)(base + o_job));
-  const long long n_tw = R.tn1 + R.tn2 + nhi + 1024;
-  hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((n_tw + 255) / 256, 4096)), dim3(256), 0, s, tw1,
-                     R.tn1, tw2, R.tn2, twl, (long long)R.tL);
-  hipLaunchKernelGGL(k_twiddles, dim3(LDM_WRAP_LC / 256), dim3(256), 0, s, (float2*)(base + o_twc), LDM_WRAP_LC,
-                     (float2*)nullptr, 0, (float2*)nullptr, 0ll);
-  hipLaunchKernelGGL(k_make_items, dim3((n_items + 255) / 256), dim3(256), 0, s, (int4*)(base + o_items), P, n_items);
+  const LdmTwiddles wrap{(float2*)(base + o_twc), nullptr, nullptr, LDM_WRAP_LC, 0, 0};
+  const LdmTwiddles tw{tw1, tw2, twl, R.tn1, R.tn2, (long long)R.tL};
+  const long long n_set = n_items + wrap.total() + tw.total();  // one element per thread: below 2^31 in the scratch array
+  hipLaunchKernelGGL(k_setup, dim3((unsigned)(1 + (n_set + 255) / 256)), dim3(256), 0, s, J, (LdmJob*)(base + o_job), P,
+                     (int4*)(base + o_items), n_items, wrap, tw);
   HIPCHK(hipGetLastError());
   const int cls_a = R.plan.fc ? R.tn1 | (R.narrow_a ? FC_NARROW : 0) : 0;
   const int cls_c = (R.plan.fc ? R.tn1 | (R.narrow_c ? FC_NARROW : 0) : 0) | (R.n_share > 1 ? FC_C_SUM : 0);

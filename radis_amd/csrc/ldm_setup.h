@@ -5,17 +5,20 @@
 #include "ldm_fft.h"
 #include "ldm_plan.h"
 
-// Twiddle tables of one size set: W_n1^e (e < n1), W_n2^e (e < n2) and the
-// two-level W_L table: hi[q] = W_L^((q * 1024) mod L), q < ceil(L / 1024),
-// then lo[e] = W_L^e, e < 1024.  W_N^e = exp(-2 pi i e / N), evaluated as
-// sincospi(-2 e / N) in FP64 and rounded to FP32.  Null tables are skipped.
-__global__ __launch_bounds__(256) void k_twiddles(float2* __restrict__ tw1, int n1, float2* __restrict__ tw2, int n2,
-                                                  float2* __restrict__ twl, long long L) {
-  const long long nhi = (L + (1 << LDM_TW_LO_BITS) - 1) >> LDM_TW_LO_BITS;
-  const long long total = (tw1 ? n1 : 0) + (tw2 ? n2 : 0) + (twl ? nhi + (1 << LDM_TW_LO_BITS) : 0);
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    long long k = i;
+// Element i of the twiddle tables of one size set: W_n1^e (e < n1), W_n2^e
+// (e < n2) and the two-level W_L table: hi[q] = W_L^((q * 1024) mod L),
+// q < ceil(L / 1024), then lo[e] = W_L^e, e < 1024.  W_N^e = exp(-2 pi i e / N),
+// evaluated as sincospi(-2 e / N) in FP64 and rounded to FP32.  Null tables are
+// skipped.
+struct LdmTwiddles {
+  float2 *tw1, *tw2, *twl;
+  int n1, n2;
+  long long L;
+  __host__ __device__ long long nhi() const { return (L + (1 << LDM_TW_LO_BITS) - 1) >> LDM_TW_LO_BITS; }
+  __host__ __device__ long long total() const {
+    return (tw1 ? n1 : 0) + (tw2 ? n2 : 0) + (twl ? nhi() + (1 << LDM_TW_LO_BITS) : 0);
+  }
+  __device__ void put(long long k) const {
     float2* dst;
     double e, N;
     if (tw1 && k < n1) {
@@ -28,27 +31,44 @@ __global__ __launch_bounds__(256) void k_twiddles(float2* __restrict__ tw1, int 
         if (tw2) k -= n2;
         dst = twl + k;
         N = (double)L;
-        e = k < nhi ? (double)((k << LDM_TW_LO_BITS) % L) : (double)(k - nhi);
+        e = k < nhi() ? (double)((k << LDM_TW_LO_BITS) % L) : (double)(k - nhi());
       }
     }
     double sn, cs;
     sincospi(-2.0 * e / N, &sn, &cs);
     *dst = make_float2((float)cs, (float)sn);
   }
+};
+
+__global__ __launch_bounds__(256) void k_twiddles(LdmTwiddles t) {
+  const long long total = t.total();
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
+       i += (long long)gridDim.x * blockDim.x)
+    t.put(i);
 }
 
-__global__ __launch_bounds__(256) void k_make_items(int4* __restrict__ items, LdmItemPlan P, int n_items) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_items) items[i] = plan_item(P, i);
-}
-
-// The job table of one request, passed by value (a kernel argument, so a
-// captured launch holds its own copy).
-__global__ __launch_bounds__(64) void k_put_job(LdmJob job, LdmJob* __restrict__ dst) {
+// Everything the no-allocation entry point writes into its scratch array before
+// the pipeline: the job table (passed by value, a kernel argument, so a captured
+// launch holds its own copy) by workgroup 0, then the request's work items, the
+// image correction's W table and the passes' tables, one element per thread.
+// One launch: as four, each a few hundred elements, they took 9 of 61 us of a
+// 20,001-point request.
+__global__ __launch_bounds__(256) void k_setup(LdmJob job, LdmJob* __restrict__ dst, LdmItemPlan P,
+                                               int4* __restrict__ items, int n_items, LdmTwiddles wrap, LdmTwiddles t) {
   static_assert(sizeof(LdmJob) % 4 == 0, "job table copied as 32-bit words");
-  const unsigned* s = (const unsigned*)&job;
-  unsigned* d = (unsigned*)dst;
-  for (int w = threadIdx.x; w < (int)(sizeof(LdmJob) / 4); w += blockDim.x) d[w] = s[w];
+  if (blockIdx.x == 0) {
+    const unsigned* s = (const unsigned*)&job;
+    unsigned* d = (unsigned*)dst;
+    for (int w = threadIdx.x; w < (int)(sizeof(LdmJob) / 4); w += blockDim.x) d[w] = s[w];
+    return;
+  }
+  long long i = (blockIdx.x - 1) * 256ll + threadIdx.x;
+  if (i < n_items) {
+    items[i] = plan_item(P, (int)i);
+    return;
+  }
+  if ((i -= n_items) < wrap.total()) wrap.put(i);
+  else if ((i -= wrap.total()) < t.total()) t.put(i);
 }
 
 // The first `rows` LDM rows of a request de-interleaved into dst[rows][cols]
