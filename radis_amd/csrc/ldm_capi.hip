@@ -246,14 +246,24 @@ int build_layout(radis_ldm_batch* b) {
   size_t total = 0;
   size_t fill_lds = 0;
   bool fill_grouped = false, fill_half = false;
-  choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu);
-  for (Req& R : b->reqs) {
-    int rc = layout_request(R, total);
-    if (rc) return rc;
-    fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R));
-    fill_grouped = fill_grouped || R.fill_groups > 1;
-    fill_half = fill_half || R.half;
-  }
+  auto lay_out = [&](bool lean) {
+    total = fill_lds = 0;
+    fill_grouped = fill_half = false;
+    choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu, lean);
+    for (Req& R : b->reqs) {
+      int rc = layout_request(R, total);
+      if (rc) return rc;
+      fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R));
+      fill_grouped = fill_grouped || R.fill_groups > 1;
+      fill_half = fill_half || R.half;
+    }
+    return 0;
+  };
+  // beyond the budget: without the whole-length transforms' further shares
+  const size_t tables = (size_t)1 << 22;
+  int rc0 = lay_out(false);
+  if (!rc0 && b->ctx->budget > 0 && b->ctx->in_use + (int64_t)(total + tables) > b->ctx->budget) rc0 = lay_out(true);
+  if (rc0) return rc0;
   // --- twiddle tables, deduplicated by size
   std::map<int, size_t> sub_off;
   std::map<int64_t, size_t> l_off;
@@ -504,11 +514,12 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
     break;
 #define FC_AN(N)                                                                                                      \
   case N | FC_NARROW:                                                                                                 \
-    launch_part(b, timed, slot, 4, f, l, k_fft_a_c<N, FC_COLS_A_NARROW, N>, grid_p, dim3(N), 0, s, cj, ca, it, G.count); \
+    launch_part(b, timed, slot, 4, f, l, k_fft_a_c<N, FC_COLS_A_NARROW, fc_narrow_ta(N)>, grid_p,      \
+                dim3(fc_narrow_ta(N)), 0, s, cj, ca, it, G.count);                                                    \
     break;
     switch (G.cls) {
       FC_A(256) FC_A(320) FC_A(384) FC_A(512) FC_A(640) FC_A(768) FC_A(1024)
-      FC_AN(256)
+      FC_AN(256) FC_AN(384) FC_AN(512)
       default: launch_part(b, timed, slot, 4, f, l, k_fft_a, grid, dim3(LDM_FFT_T), 0, s, cj, ca, it, G.count);
     }
 #undef FC_A

@@ -453,11 +453,13 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
   const LdmJob& J = jobs[it.x];
   if (J.status) return;
   const int N1 = J.tn1;
-  const int item = it.y * J.split_b + it.z, share = item % J.n_share;
-  const int k1_0 = (item / J.n_share) * B;
-  const long long L = J.tL;
+  const int share = it.w & 15, k1_0 = (it.w >> 4) * B;
+  const int L = (int)J.tL;  // <= 2^21
   const int P = axes[it.x].p, M = axes[it.x].m;
-  const int p0 = P * share / J.n_share, p1 = P * (share + 1) / J.n_share;  // this workgroup's pairs
+  // this workgroup's pairs (share_inv, as a division is 40 instructions)
+  const unsigned inv = J.share_inv;
+  const int p0 = (int)((unsigned)(P * share) * inv >> 16);
+  const int p1 = share + 1 == J.n_share ? P : (int)((unsigned)(P * (share + 1)) * inv >> 16);
   fc_load_tw_stages<N2, T, PV>(s_tw, J.tw2);
   // The rows' lineshape coefficients (a_l, b_m, 1/F(0), fold count) staged
   // in LDS.  Read from global memory they are scalar loads, and the LDS
@@ -485,7 +487,7 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
   const float2* Yb = J.ybuf + (long long)k1_0 * N2;
   float2 pre[SH::IT0][SH::R0];
   auto prefetch = [&](int p) {
-    const float2* Yp = Yb + (long long)p * L;
+    const float2* Yp = Yb + (long long)p * (long long)L;
 #pragma unroll
     for (int s = 0; s < SH::IT0; ++s) {
       const int t = threadIdx.x + s * T;
@@ -506,8 +508,8 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
     const int t = threadIdx.x + s * T;
 #pragma unroll
     for (int q = 0; q < SH::RL; ++q) {
-      const long long k = (long long)(k1_0 + (t & (B - 1))) + (long long)N1 * ((t >> LB) + q * NSL);
-      const long long kk = (k <= L - k) ? k : (L - k);
+      const int k = k1_0 + (t & (B - 1)) + N1 * (t >> LB) + q * (N1 * NSL);
+      const int kk = min(k, L - k);
       xs[s][q] = (float)kk * J.inv_Lws;
     }
   }
@@ -525,7 +527,7 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
 #pragma unroll
   for (int s = 0; s < SH::ITL; ++s) {
     const int t = threadIdx.x + s * T;
-    const long long ks = (long long)(k1_0 + (t & (B - 1))) + (long long)N1 * (t >> LB);  // bin of q = 0
+    const int ks = k1_0 + (t & (B - 1)) + N1 * (t >> LB);  // bin of q = 0
     u0[s][0] = (float)ks * J.inv_Lws;                    // q = 0, 1, ..., RL/2-1
     u0[s][1] = (float)(L / SH::RL - ks) * J.inv_Lws;     // q = RL-1, RL-2, ..., RL/2
   }
@@ -558,7 +560,10 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
     __syncthreads();  // WK is the job's: uniform over the workgroup
   }
   float gcache[SH::ITL][SH::RL];
-  int g_l = -1;
+  // the L-axis node of the next row; the Gaussian factors are refilled when it
+  // wraps (counted, as a division and a remainder per row are 100 instructions)
+  int m_next = NLr > 0 ? (2 * p0) % NLr : 0;
+  bool refill = true;
   auto gauss_fill = [&](int r) {
     const float a = row_c(r).x;
 #pragma unroll
@@ -567,6 +572,10 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
       for (int q = 0; q < SH::RL; ++q) gcache[s][q] = __expf(-(a * xs[s][q] * xs[s][q]));
   };
   auto row_ft = [&](int r, float (&F)[SH::ITL][SH::RL]) {
+    if (refill) gauss_fill(r);
+    const int m = m_next;
+    refill = ++m_next == NLr;
+    if (refill) m_next = 0;
     const float4 c = row_c(r);
     const float bco = c.y;
     const float E = __expf(-bco * dlt);
@@ -597,7 +606,6 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
           }
     }
     if (w_lo >= 0 || w_hi >= 0) {
-      const int m = r % NLr;
       if (w_lo >= 0) F[0][0] += wh(0, w_lo, m);
       if (w_hi >= 0) {
         const float hv = wh(1, w_hi, m);
@@ -619,10 +627,8 @@ __global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_f
     // uses them (they are then not live across the earlier stages)
     float fa[SH::ITL][SH::RL], fb[SH::ITL][SH::RL];
     auto lineshapes = [&] {
-      if (ra / NLr != g_l) { g_l = ra / NLr; gauss_fill(ra); }
       row_ft(ra, fa);
       if (rb < M) {
-        if (rb / NLr != g_l) { g_l = rb / NLr; gauss_fill(rb); }
         row_ft(rb, fb);
       } else {
 #pragma unroll

@@ -87,11 +87,14 @@ constexpr int fc_pow2_floor(int n) { return n < 2 ? 1 : 2 * fc_pow2_floor(n >> 1
 // workgroup of pass B for N2
 constexpr int fc_cols_a(int n1) { return fc_pow2_floor(FC_CAP_A / n1); }
 constexpr int fc_cols_c(int n1) { return fc_pow2_floor(FC_CAP / n1); }
-// narrow pass A and C tiles, for launches whose wide ones would leave CUs
-// idle: 16 and 8 columns, 16 elements per thread.  At n1 = 256 a 72-block pass A
-// took 9.2 -> 6.9 us and an 8-block pass C 8.1 -> 6.8 us; with an odd factor
-// (n1 = 320: a first stage of 3.2 passes) pass C took 8.2 -> 15.5 us.
-constexpr bool fc_narrow(int n1) { return n1 == 256; }
+// narrow pass A and C tiles (16 and 8 columns), for launches whose wide ones
+// would leave CUs idle.  Pass A, wide -> narrow: n1 = 256, 72 blocks 9.2 -> 6.9 us;
+// n1 = 384, 48 blocks 9.6 -> 7.1 us; n1 = 512, 112 blocks 13.3 -> 7.5 us; but
+// n1 = 320 (a middle stage of 0.5 passes) 224 blocks 12.5 -> 13.6 us.  Pass C
+// at n1 = 256 8.1 -> 6.8 us; at 384 and 512 6 -> 9 to 11 us, at 320 8.2 -> 10.4 us.
+constexpr bool fc_narrow_a(int n1) { return n1 == 256 || n1 == 384 || n1 == 512; }
+constexpr bool fc_narrow_c(int n1) { return n1 == 256; }
+constexpr int fc_narrow_ta(int n1) { return n1 == 384 ? 768 : n1; }  // threads of a narrow pass A tile
 #define FC_COLS_A_NARROW 16
 #define FC_COLS_C_NARROW 8
 #define FC_NARROW (1 << 21)  // pass A and C launch-class flag
@@ -225,8 +228,9 @@ struct LdmJob {
   int tn1, tn2;
   // pass B's partial spectra: share s of a row block's pairs goes to
   // bbuf + s * share_stride (n_share of them, added by pass C); a pass B item
-  // (y, z) is number y * split_b + z, row block number / n_share
+  // (y, z, w) is number y * split_b + z, row block w >> 4, share w & 15
   int n_share, split_b;
+  unsigned share_inv;            // 2^16 / n_share: share s takes the pairs from P s share_inv >> 16
   long long share_stride;
   // half-length transforms: per cell IMG_NODES values of the correction
   double* img_u;                 // [n_cell][IMG_NODES]

@@ -759,7 +759,8 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.ldm = (float*)(work + R.off_ldm);
   J.ybuf = (float2*)(work + R.off_y);
   J.bbuf = (float2*)(work + R.off_share);
-  J.share_stride = R.half ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
+  J.share_inv = 65536u / (unsigned)R.n_share;
+  J.share_stride = R.half || R.n_share > 2 ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
   J.mom = R.half ? (float*)(work + R.off_mom) : nullptr;
   J.img_u = R.half ? (double*)(work + R.off_img) : nullptr;
   J.cell_tiles = R.cell_tiles;
@@ -886,10 +887,16 @@ int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
 // share costs an inverse transform and 8 tL bytes written and read.
 constexpr int FC_B_SPLIT_WGS_PER_CU = 4;
 constexpr int FC_B_SPLIT_MIN_PAIRS = 2;
+// bytes of Y up to which a whole-length transform's workspace may grow by more
+// than the one further partial spectrum that it always had room for
+constexpr int64_t FC_B_SPLIT_WHOLE_Y = 64 << 20;
 constexpr int FC_B_SPLIT_MAX = 4;
 constexpr double HALF_MIN_POINTS = 1 << 19;
-constexpr int FC_A_NARROW_PER_CU = 1, FC_C_NARROW_PER_CU = 1;
-void choose_split_b(Req* reqs, int n, int n_cu) {
+// wide column blocks below which the narrow ones run: a CU each (n1 = 256), or
+// half of that (384, 512: 768-thread tiles of three passes; between 128 and 256
+// wide blocks of 384 they took 14.5 -> 17.9 us)
+constexpr int FC_A_NARROW_DIV = 2, FC_C_NARROW_PER_CU = 1;
+void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   // Half-length transforms pay where the launch's passes are more than a chain
   // of latencies: below HALF_MIN_POINTS (pairs times planned length) the
   // shorter passes take as long as the whole ones and the correction is extra.
@@ -912,15 +919,16 @@ void choose_split_b(Req* reqs, int n, int n_cu) {
     Req& R = reqs[i];
     R.split_b = R.n_share = 1;
     if (!R.plan.fc) continue;
-    if (fc_narrow(R.tn1)) {
-      R.narrow_a = cols_a[R.tn1] < (long long)FC_A_NARROW_PER_CU * n_cu;
-      R.narrow_c = cols_c[R.tn1] < (long long)FC_C_NARROW_PER_CU * n_cu;
-    }
+    R.narrow_a = fc_narrow_a(R.tn1) && cols_a[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_A_NARROW_DIV);
+    R.narrow_c = fc_narrow_c(R.tn1) && cols_c[R.tn1] < (long long)FC_C_NARROW_PER_CU * n_cu;
     const int pairs = (R.m_cap + 1) / 2, rb = R.tn1 >> R.bX[1];
-    // whole length: two shares at most (the workspace holds two)
+    // whole length: two shares, or more where its workspace is small (a share's
+    // chain of pairs is what a lone small request waits for: 20,001 points,
+    // twelve pairs in two shares 14.4 us)
     const long long room = std::max<long long>(0, (long long)FC_B_SPLIT_WGS_PER_CU * n_cu - images[R.tn2]);
     int ns = (int)std::min<long long>(room / blocks[R.tn2], pairs / FC_B_SPLIT_MIN_PAIRS);
-    ns = std::min(ns, R.half ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);
+    const bool room_whole = (int64_t)pairs * R.plan.L * 8 <= FC_B_SPLIT_WHOLE_Y && !lean;
+    ns = std::min(ns, R.half || room_whole ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);
     if (R.half && ns > 2) ns = std::min(ns, pairs - 1 - pairs / 8);  // they share Y's unused half with the moments
     if (ns > 1) {
       R.n_share = ns;
@@ -938,7 +946,8 @@ int layout_request(Req& R, size_t& total) {
   const int64_t V = R.nv + 1;
   R.stride = (int64_t)align_up((size_t)V, 64);
   R.bA = R.bX[0];
-  R.bB = R.half ? 0 : R.bX[1];  // (the run-time-sized pass B's; the item numbers of a half-length one go past n1 >> bX)
+  // (the run-time-sized pass B's; the item numbers of a half-length one and of more than two shares go past n1 >> bX)
+  R.bB = R.half || R.n_share > 2 ? 0 : R.bX[1];
   R.bC = R.bX[2];
   const int pcap = (R.m_cap + 1) / 2;
   // LDM: pcap pairs of rows, rows 2p and 2p+1 interleaved (element n of row
@@ -964,8 +973,10 @@ int layout_request(Req& R, size_t& total) {
     if (o > total) return fail(RADIS_LDM_EINVAL, "internal: half-length buffers exceed the workspace");
     R.off_b2 = R.off_y;
   } else {
-    // pass B's second share of the pairs
-    R.off_b2 = total; if (R.split_b > 1) total = align_up(total + (size_t)R.plan.L * 8, 256);
+    // pass B's second share of the pairs, or all of more than two shares
+    R.off_b2 = total;
+    if (R.n_share > 2) R.off_share = total;
+    if (R.split_b > 1) total = align_up(total + (size_t)(R.n_share > 2 ? R.n_share : 1) * R.plan.L * 8, 256);
   }
   R.off_rows = total; total = align_up(total + (size_t)R.m_cap * 16, 256);
   // axis partials: at most one per chunk, plus the two partial blocks at the window edges
@@ -988,7 +999,7 @@ int check_layout(const Req& R, size_t total) {
                   (R.split_b == 1 || R.off_b2 + (size_t)R.plan.L * 8 <= total) && R.off_rows + (size_t)R.m_cap * 16 <= total &&
                   R.off_axp + parts * 32 <= total && (size_t)R.n_axp <= parts &&
                   R.off_wrap + (size_t)R.wrap_rows * R.plan.wrap_k * 4 <= total &&
-                  R.off_share + (size_t)(R.n_share - 1) * (R.half ? (size_t)R.tL * 8 : R.off_b2 - R.off_b) + (size_t)R.tL * 8 <= total &&
+                  R.off_share + (size_t)(R.n_share - 1) * (R.half || R.n_share > 2 ? (size_t)R.tL * 8 : R.off_b2 - R.off_b) + (size_t)R.tL * 8 <= total &&
                   (!R.half || (R.tL * 2 == R.plan.L && (size_t)R.tL >= V && (long long)R.n_cell * R.cell_tiles >= R.n_tiles &&
                                R.off_y + (size_t)((R.m_cap + 1) / 2) * R.tL * 8 <= R.off_img &&
                                R.off_img + (size_t)R.n_cell * IMG_NODES * 8 <= R.off_mom &&
@@ -1010,7 +1021,7 @@ struct LdmItemPlan {
   long long hi_a, hi_e;         // lines [hi_a, hi_e) scanned in chunks
   int n_lo, n_g, n_hi;          // items of the three axis parts
   int n_wrap, n_fill, pcap, n_colA, n_rowB, n_colC;
-  int split_b;                  // pass B's item numbers are y * split_b + z
+  int split_b, n_share;         // pass B's item numbers are y * split_b + z; w: row block << 4 | share
   int n_img, img_parts;         // image items (half-length transforms), parts per cell
 };
 
@@ -1040,7 +1051,7 @@ __host__ __device__ inline int4 plan_item(const LdmItemPlan& P, int i) {
   if (k < P.n_wrap) return make_int4(0, k, 0, 0);                 // L-axis node pair
   if ((k -= P.n_wrap) < P.n_fill) return make_int4(0, k, 0, 0);  // fill tile
   if ((k -= P.n_fill) < P.pcap * P.n_colA) return make_int4(0, k / P.n_colA, k % P.n_colA, 0);  // (pair, column block)
-  if ((k -= P.pcap * P.n_colA) < P.n_rowB) return make_int4(0, k / P.split_b, k % P.split_b, 0);  // pass B, number k = y * split_b + z
+  if ((k -= P.pcap * P.n_colA) < P.n_rowB) return make_int4(0, k / P.split_b, k % P.split_b, (k / P.n_share) << 4 | k % P.n_share);  // pass B, number k = y * split_b + z
   if ((k -= P.n_rowB) < P.n_colC) return make_int4(0, 0, k, 0);   // pass C column block
   k -= P.n_colC;
   return make_int4(0, k / P.img_parts, k % P.img_parts, 0);       // image item (cell, part of the nodes), after plan_items
@@ -1085,6 +1096,7 @@ LdmItemPlan item_plan(const radis_ldm_db& db, Req& R) {
   P.pcap = (R.m_cap + 1) / 2;
   P.n_colA = R.tn2 >> R.bX[0];
   P.split_b = R.split_b;
+  P.n_share = R.n_share;
   P.n_rowB = (R.tn1 >> R.bX[1]) * R.n_share;
   P.n_colC = R.tn2 >> R.bX[2];
   P.img_parts = image_parts(R.n_cell);

@@ -10,7 +10,7 @@
 #include "ldm_plan.h"
 
 int main() {
-  int fails = 0, halves = 0, wholes = 0, shared = 0;
+  int fails = 0, halves = 0, wholes = 0, shared = 0, whole_shared = 0;
 #define CHECK(c, ...) \
   if (!(c)) { std::fprintf(stderr, "check failed: %s: ", #c); std::fprintf(stderr, __VA_ARGS__); std::fprintf(stderr, "\n"); ++fails; }
   radis_ldm_db db;
@@ -35,7 +35,18 @@ int main() {
           CHECK(R.tL == (int64_t)R.tn1 * R.tn2, "split");
           if (!R.half) {
             ++wholes;
-            CHECK(R.tL == R.plan.L && R.n_cell == 0 && R.n_share <= 2, "whole length");
+            CHECK(R.tL == R.plan.L && R.n_cell == 0 && R.n_share <= 4, "whole length");
+            if (R.n_share > 2) {  // their buffers behind Y, every (row block, share) once
+              ++whole_shared;
+              const size_t y1 = R.off_y + (size_t)((m_cap + 1) / 2) * R.plan.L * 8;
+              CHECK(R.off_share >= y1 && R.off_share + (size_t)R.n_share * R.tL * 8 <= R.off_rows, "whole-length shares");
+              std::set<int> once;
+              const LdmItemPlan P = item_plan(db, R);
+              const int b0 = plan_items(P) - P.n_rowB - P.n_colC;
+              for (int i = b0; i < b0 + P.n_rowB; ++i) once.insert(plan_item(P, i).w);
+              for (int w : once) CHECK((w >> 4) < (R.tn1 >> R.bX[1]) && (w & 15) < R.n_share, "row block and share");
+              CHECK((int)once.size() == P.n_rowB, "every row block and share once");
+            }
             continue;
           }
           ++halves;
@@ -62,7 +73,7 @@ int main() {
           for (int i = b0; i < b0 + P.n_rowB; ++i) {
             const int4 t = plan_item(P, i);
             const int k = t.y * R.split_b + t.z;
-            CHECK(k / R.n_share < rb, "row block");
+            CHECK(k / R.n_share < rb && t.w == (k / R.n_share << 4 | k % R.n_share), "row block");
             seen.insert({k / R.n_share, k % R.n_share});
           }
           CHECK((int)seen.size() == P.n_rowB, "every row block and share once");
@@ -75,7 +86,18 @@ int main() {
           CHECK((int)seen.size() == P.n_img && P.n_img == R.n_cell * ((R.n_cell * IMG_NODES + IMG_TARGETS - 1) / IMG_TARGETS),
                 "every cell and part once");
         }
-  CHECK(halves > 1000 && wholes > 1000 && shared > 100, "%d half-length, %d whole, %d with more than two shares", halves, wholes, shared);
+  // the shares' pairs: [P s inv >> 16, P (s + 1) inv >> 16), the last up to P
+  for (unsigned n = 1; n <= 8; ++n)
+    for (unsigned P = 0; P <= 128 * 128 / 2; ++P) {
+      const unsigned inv = 65536u / n;
+      unsigned at = 0;
+      for (unsigned s = 0; s < n; ++s) {
+        const unsigned e = s + 1 == n ? P : (unsigned)(P * (s + 1)) * inv >> 16;
+        if (e < at || e - at > P / n + 2) { CHECK(false, "share %u of %u, %u pairs", s, n, P); break; }
+        at = e;
+      }
+    }
+  CHECK(halves > 1000 && wholes > 1000 && shared > 100 && whole_shared > 100, "%d half-length, %d whole, %d with more than two shares", halves, wholes, shared);
   std::printf("%d half-length plans (%d with more than two shares), %d whole, %d failed checks\n", halves, shared, wholes, fails);
   return fails ? 1 : 0;
 }
