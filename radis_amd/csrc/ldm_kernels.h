@@ -131,18 +131,21 @@ __device__ __forceinline__ double fwhm_gauss(double nu0, double dopp) {
 
 // Lorentzian FWHM, radis/lbl/broadening.py:341-383 (x2 at 1854), with
 // diluent {'air': 1-x}; (Tref/T)**n as pow, as NumPy evaluates it (the
-// width extremes the LDM axes start from).  A called function: k_axis and
-// k_finalize evaluate it at several sites, and one copy of its two FP64 pow
-// routines keeps their code short (short kernels that fetch their code cold
-// once per spectrum).
-__device__ __noinline__ double fwhm_lorentz(const LdmJob& J, double g_air, double g_self, double n_air,
-                                               double n_self) {
+// width extremes the LDM axes start from).  The power is a called function:
+// k_axis and k_finalize evaluate it at several sites, and one copy keeps their
+// code short.
+__device__ __noinline__ double pow_call(double x, double y) { return pow(x, y); }
+// from the powers ra = (Tref/T)**n_air, rs = (Tref/T)**n_self
+__device__ __forceinline__ double fwhm_lorentz(const LdmJob& J, double g_air, double g_self, double ra, double rs) {
 #pragma clang fp contract(off)
-  const double ra = pow(J.ratio_T, n_air);
-  const double rs = (n_self == n_air) ? ra : pow(J.ratio_T, n_self);
   const double air = ((ra * g_air) * J.p_atm) * J.x_air;
   const double slf = rs * ((g_self * J.p_atm) * J.x_self);
   return (air + slf) * 2.0;
+}
+__device__ __forceinline__ double fwhm_lorentz_n(const LdmJob& J, double g_air, double g_self, double n_air,
+                                                 double n_self) {
+  const double ra = pow_call(J.ratio_T, n_air);
+  return fwhm_lorentz(J, g_air, g_self, ra, n_self == n_air ? ra : pow_call(J.ratio_T, n_self));
 }
 
 // FP32 Lorentzian FWHM (relative error ~1e-6), for filtering and fast paths.
@@ -156,6 +159,54 @@ __device__ __forceinline__ double bits_to_double(unsigned long long b) { return 
 __device__ __forceinline__ unsigned long long double_to_bits(double d) {
   return (unsigned long long)__double_as_longlong(d);
 }
+
+// The value of lane i ^ X (lane_xor) in 64 bits.
+template <int X>
+__device__ __forceinline__ unsigned long long lane_xor64(unsigned long long v) {
+  const unsigned lo = __float_as_uint(lane_xor<X>(__uint_as_float((unsigned)v)));
+  const unsigned hi = __float_as_uint(lane_xor<X>(__uint_as_float((unsigned)(v >> 32))));
+  return (unsigned long long)hi << 32 | lo;
+}
+// The least (MAX: largest) v of this lane's row of 16 lanes, in registers (a
+// shuffle goes through LDS).
+template <bool MAX>
+__device__ __forceinline__ unsigned long long row_extreme(unsigned long long v) {
+  auto take = [&](unsigned long long o) { v = (MAX ? o > v : o < v) ? o : v; };
+  take(lane_xor64<1>(v));
+  take(lane_xor64<2>(v));
+  take(lane_xor64<7>(v));
+  take(lane_xor64<8>(v));
+  return v;
+}
+
+// Width extremes as FP64 bit patterns; reduce() leaves every lane of every wave
+// with those of a workgroup of 256 (gauss false: without the Gaussian ones).
+struct WidthExtremes {
+  unsigned long long lmin = ~0ull, lmax = 0ull, gmin = ~0ull, gmax = 0ull;
+  __device__ __forceinline__ void lorentz(unsigned long long b) {
+    lmin = b < lmin ? b : lmin;
+    lmax = b > lmax ? b : lmax;
+  }
+  __device__ __forceinline__ void rows(bool gauss) {
+    lmin = row_extreme<false>(lmin);
+    lmax = row_extreme<true>(lmax);
+    if (gauss) {
+      gmin = row_extreme<false>(gmin);
+      gmax = row_extreme<true>(gmax);
+    }
+  }
+  __device__ __forceinline__ void reduce(unsigned long long (*red)[16], bool gauss) {
+    rows(gauss);
+    if ((threadIdx.x & 15) == 0) {
+      const int r = threadIdx.x >> 4;
+      red[0][r] = lmin; red[1][r] = lmax; red[2][r] = gmin; red[3][r] = gmax;
+    }
+    __syncthreads();
+    const int r = threadIdx.x & 15;
+    lmin = red[0][r]; lmax = red[1][r]; gmin = red[2][r]; gmax = red[3][r];
+    rows(gauss);
+  }
+};
 
 // First index in [lo, hi) with nu0[i] >= v, by a whole wave: 64 probes per
 // round narrow the range 64-fold (ballot + popcount), so ~log64(n) dependent
@@ -243,7 +294,7 @@ __global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const i
   }
   const int4 it = items[blockIdx.x];
   LdmJob& J = jobs[it.x];
-  unsigned long long lmin = ~0ull, lmax = 0ull, gmin = ~0ull, gmax = 0ull;
+  WidthExtremes X;
   if (it.w < 0) {
     const int gb0 = it.z, G = -it.w;
     const int dmax = J.log_r > 0.0 ? 2 : 0, dmin = dmax + 1;
@@ -256,30 +307,35 @@ __global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const i
     // and last line (nu0 sorted)
     const int ns = db.n_iso_slots;
     const int nc = J.single_iso ? 0 : G * ns;
-    // one pass over the two candidate lists and the isotopologue ranges, so
-    // that their loads are in flight together
-    const int nmax = max(max(na, nb), nc);
-    for (int c = threadIdx.x; c < nmax; c += blockDim.x) {
-      float4 qa = make_float4(0.f, 0.f, 0.f, 0.f), qb = qa;
-      int2 r = make_int2(-1, -1);
-      if (c < na) qa = db.sky[a0 + c];
-      if (c < nb) qb = db.sky[b0 + c];
-      if (c < nc) r = db.iso_rng[(long long)(gb0 + c / ns) * ns + (c - (c / ns) * ns)];
-      if (c < na) {
-        const unsigned long long bl = double_to_bits(fwhm_lorentz(J, qa.x, qa.y, qa.z, qa.w));
-        lmax = bl > lmax ? bl : lmax;
-      }
-      if (c < nb) {
-        const unsigned long long bl = double_to_bits(fwhm_lorentz(J, qb.x, qb.y, qb.z, qb.w));
-        lmin = bl < lmin ? bl : lmin;
-      }
+    for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+      const int s = c - (c / ns) * ns;
+      const int2 r = db.iso_rng[(long long)(gb0 + c / ns) * ns + s];
       if (r.x >= 0) {
-        const int s = c - (c / ns) * ns;
         const unsigned long long g0 = double_to_bits(fwhm_gauss(db.nu0[r.x], J.dopp[s]));
         const unsigned long long g1 = double_to_bits(fwhm_gauss(db.nu0[r.y], J.dopp[s]));
-        gmin = g0 < gmin ? g0 : gmin;
-        gmax = g1 > gmax ? g1 : gmax;
+        X.gmin = g0 < X.gmin ? g0 : X.gmin;
+        X.gmax = g1 > X.gmax ? g1 : X.gmax;
       }
+    }
+    // Both lists as one (a thread's candidates of the two, one after the other,
+    // were twice the chain of FP64 powers); a list with n_self takes a lane for
+    // each of a candidate's two powers.
+    const int two = db.n_self ? 1 : 0, n = (na + nb) << two;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+      const int c = i >> two;
+      const bool up = c < na;
+      const float4 q = db.sky[up ? a0 + c : b0 + c - na];
+      const bool self = two && (i & 1);
+      const double r = pow_call(J.ratio_T, self ? q.w : q.z);
+      double ra = r, rs = r;
+      if (two) {
+        const double o = bits_to_double(lane_xor64<1>(double_to_bits(r)));  // n is even: both lanes are here
+        if (self) ra = o;
+        else rs = o;
+      }
+      const unsigned long long bl = double_to_bits(fwhm_lorentz(J, q.x, q.y, ra, rs));
+      if (up) X.lmax = bl > X.lmax ? bl : X.lmax;
+      else X.lmin = bl < X.lmin ? bl : X.lmin;
     }
   } else {
     const long long a = J.i0 + it.z;
@@ -369,44 +425,25 @@ __global__ __launch_bounds__(256) void k_axis(LdmJob* __restrict__ jobs, const i
     }
     for (; wl; wl &= wl - 1) {
       const long long i = line(__ffs(wl) - 1);
-      const unsigned long long bl = double_to_bits(fwhm_lorentz(J, db.g_air[i], db.g_self[i], db.n_air[i], nsp[i]));
-      lmin = bl < lmin ? bl : lmin;
-      lmax = bl > lmax ? bl : lmax;
+      X.lorentz(double_to_bits(fwhm_lorentz_n(J, db.g_air[i], db.g_self[i], db.n_air[i], nsp[i])));
     }
     for (; wg; wg &= wg - 1) {
       const long long i = line(__ffs(wg) - 1);
       const unsigned long long bg = double_to_bits(fwhm_gauss(db.nu0[i], J.dopp[db.iso ? db.iso[i] : 1]));
-      gmin = bg < gmin ? bg : gmin;
-      gmax = bg > gmax ? bg : gmax;
+      X.gmin = bg < X.gmin ? bg : X.gmin;
+      X.gmax = bg > X.gmax ? bg : X.gmax;
     }
   }
-  // wave reduction
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o;
-    o = __shfl_xor(lmin, off); lmin = o < lmin ? o : lmin;
-    o = __shfl_xor(lmax, off); lmax = o > lmax ? o : lmax;
-    o = __shfl_xor(gmin, off); gmin = o < gmin ? o : gmin;
-    o = __shfl_xor(gmax, off); gmax = o > gmax ? o : gmax;
-  }
-  __shared__ unsigned long long red[4][4];
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) { red[0][w] = lmin; red[1][w] = lmax; red[2][w] = gmin; red[3][w] = gmax; }
-  __syncthreads();
+  __shared__ unsigned long long red[4][16];
+  X.reduce(red, !J.single_iso);
   if (threadIdx.x == 0) {
-    const int nw = blockDim.x >> 6;
-    for (int k = 1; k < nw; ++k) {
-      lmin = red[0][k] < lmin ? red[0][k] : lmin;
-      lmax = red[1][k] > lmax ? red[1][k] : lmax;
-      gmin = red[2][k] < gmin ? red[2][k] : gmin;
-      gmax = red[3][k] > gmax ? red[3][k] : gmax;
-    }
     // per-chunk partials, reduced by k_finalize (same-address global atomics
     // from every workgroup would serialise in L2)
     unsigned long long* P = J.ax_part + 4 * (long long)it.y;
-    P[0] = lmin;
-    P[1] = lmax;
-    P[2] = gmin;
-    P[3] = gmax;
+    P[0] = X.lmin;
+    P[1] = X.lmax;
+    P[2] = X.gmin;
+    P[3] = X.gmax;
   }
 }
 
@@ -443,9 +480,8 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
   LdmJob& J = jobs[blockIdx.x];
   LdmAxes& A = axes[blockIdx.x];
   __shared__ double wgax[LDM_MAX_AX], wlax[LDM_MAX_AX], lgax[LDM_MAX_AX], llax[LDM_MAX_AX];
-  __shared__ double s_wg_min, s_wl_min, s_wg_max, s_wl_max;
-  __shared__ int s_ng, s_nl, s_status;
-  __shared__ unsigned long long s_w[4][4];
+  __shared__ int s_status;
+  __shared__ unsigned long long red[4][16];
   // This kernel is a chain of dependent memory round trips, so everything it
   // reads is loaded up front: the job's values, the partial extremes and,
   // for a single isotopologue, the window's end lines (its Gaussian width
@@ -463,7 +499,7 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
   float* const row_a = J.row_a;
   float* const row_b = J.row_b;
   float* const row_inv_f0 = J.row_inv_f0;
-  const bool ends = threadIdx.x == 0 && single && i1 > i0;
+  const bool ends = single && i1 > i0;  // every lane: the same two values
   if (J.half)  // the image correction is accumulated by the pass B launch
     for (int e = threadIdx.x; e < J.n_cell * IMG_NODES; e += blockDim.x) J.img_u[e] = 0.0;
   const double nu_a = ends ? db.nu0[i0] : 0.0, nu_b = ends ? db.nu0[i1 - 1] : 0.0;
@@ -479,95 +515,87 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
     // as the host decides it for host-given ratios
     if (!(qi > 0x1p-60 && qi < 0x1p+100)) J.i_fast = 0;
   }
+  int ng = 0, nl = 0, st0 = 0;
+  double wg_min = 0, wl_min = 0, wg_max = 0, wl_max = 0;
   {
     // reduce the per-item width extremes written by k_axis, or, when the
     // window is the whole single-isotopologue list, evaluate the list's two
     // Pareto sets here (the extremes k_axis would find, bit for bit: same
     // candidates' superset property and same FP64 expression)
-    unsigned long long lmin = ~0ull, lmax = 0ull, gmin = ~0ull, gmax = 0ull;
+    WidthExtremes X;
     if (J.sky_whole) {
       const int dmax = J.log_r > 0.0 ? 2 : 0;
       const int a1 = db.gsky_off[dmax + 1], b1 = db.gsky_off[dmax + 2];
       for (int c = db.gsky_off[dmax] + threadIdx.x; c < b1; c += blockDim.x) {
         const float4 q = db.sky[c];
-        const unsigned long long bl = double_to_bits(fwhm_lorentz(J, q.x, q.y, q.z, q.w));
-        if (c < a1) lmax = bl > lmax ? bl : lmax;
-        else lmin = bl < lmin ? bl : lmin;
+        const unsigned long long bl = double_to_bits(fwhm_lorentz_n(J, q.x, q.y, q.z, q.w));
+        if (c < a1) X.lmax = bl > X.lmax ? bl : X.lmax;
+        else X.lmin = bl < X.lmin ? bl : X.lmin;
       }
     } else {
       for (long long c = threadIdx.x; c < nch; c += blockDim.x) {
         const unsigned long long* P = part + 4 * c;
-        lmin = P[0] < lmin ? P[0] : lmin;
-        lmax = P[1] > lmax ? P[1] : lmax;
-        gmin = P[2] < gmin ? P[2] : gmin;
-        gmax = P[3] > gmax ? P[3] : gmax;
+        X.lmin = P[0] < X.lmin ? P[0] : X.lmin;
+        X.lmax = P[1] > X.lmax ? P[1] : X.lmax;
+        X.gmin = P[2] < X.gmin ? P[2] : X.gmin;
+        X.gmax = P[3] > X.gmax ? P[3] : X.gmax;
       }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-      unsigned long long o;
-      o = __shfl_xor(lmin, off); lmin = o < lmin ? o : lmin;
-      o = __shfl_xor(lmax, off); lmax = o > lmax ? o : lmax;
-      o = __shfl_xor(gmin, off); gmin = o < gmin ? o : gmin;
-      o = __shfl_xor(gmax, off); gmax = o > gmax ? o : gmax;
+    if (threadIdx.x == 0) s_status = 0;
+    X.reduce(red, !single);
+    // every wave goes on by itself from the same extremes: no broadcast
+    if (i1 > i0) {
+      wg_min = single ? fwhm_gauss(nu_a, dopp1) : bits_to_double(X.gmin);
+      wg_max = single ? fwhm_gauss(nu_b, dopp1) : bits_to_double(X.gmax);
+      wl_min = bits_to_double(X.lmin);
+      wl_max = bits_to_double(X.lmax);
+      if (!(wg_min > 0.0) || !(wl_min > 0.0)) {
+        st0 |= LDM_ST_WIDTH;
+      } else {
+        // N = ceil((log(w_max + 1e-4) - log(w_min)) / dx) + 1, radis/lbl/broadening.py:1835-1836:
+        // the four logarithms by four lanes
+        const int k = threadIdx.x & 3;
+        const double lg = log_call(k == 0 ? wg_max + 1e-4 : k == 1 ? wg_min : k == 2 ? wl_max + 1e-4 : wl_min);
+        const unsigned long long b = double_to_bits(lg);
+        auto lane = [&](int i) {
+          return bits_to_double((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(b >> 32), i) << 32 |
+                                (unsigned)__builtin_amdgcn_readlane((int)b, i));
+        };
+        ng = (int)ceil((lane(0) - lane(1)) / dxG) + 1;
+        nl = (int)ceil((lane(2) - lane(3)) / dxL) + 1;
+        if (ng > LDM_MAX_AX || nl > LDM_MAX_AX || ng < 2 || nl < 2) st0 |= LDM_ST_AXIS;
+        else if (ng * nl > m_cap) st0 |= LDM_ST_CAP;
+      }
     }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { s_w[0][w] = lmin; s_w[1][w] = lmax; s_w[2][w] = gmin; s_w[3][w] = gmax; }
-    __syncthreads();
+    if (st0) { ng = 0; nl = 0; }
     if (threadIdx.x == 0) {
-      for (int k = 1; k < (int)(blockDim.x >> 6); ++k) {
-        lmin = s_w[0][k] < lmin ? s_w[0][k] : lmin;
-        lmax = s_w[1][k] > lmax ? s_w[1][k] : lmax;
-        gmin = s_w[2][k] < gmin ? s_w[2][k] : gmin;
-        gmax = s_w[3][k] > gmax ? s_w[3][k] : gmax;
-      }
-      int status = 0, ng = 0, nl = 0;
-      double wg_min = 0, wl_min = 0, wg_max = 0, wl_max = 0;
-      if (i1 > i0) {
-        if (single) {
-          wg_min = fwhm_gauss(nu_a, dopp1);
-          wg_max = fwhm_gauss(nu_b, dopp1);
-        } else {
-          wg_min = bits_to_double(gmin);
-          wg_max = bits_to_double(gmax);
-        }
-        wl_min = bits_to_double(lmin);
-        wl_max = bits_to_double(lmax);
-        if (!(wg_min > 0.0) || !(wl_min > 0.0)) {
-          status |= LDM_ST_WIDTH;
-        } else {
-          // N = ceil((log(w_max + 1e-4) - log(w_min)) / dx) + 1, radis/lbl/broadening.py:1835-1836
-          ng = (int)ceil((log_call(wg_max + 1e-4) - log_call(wg_min)) / dxG) + 1;
-          nl = (int)ceil((log_call(wl_max + 1e-4) - log_call(wl_min)) / dxL) + 1;
-          if (ng > LDM_MAX_AX || nl > LDM_MAX_AX || ng < 2 || nl < 2) status |= LDM_ST_AXIS;
-          else if (ng * nl > m_cap) status |= LDM_ST_CAP;
-        }
-      }
-      if (status) { ng = 0; nl = 0; }
-      s_ng = ng; s_nl = nl; s_status = status;
-      s_wg_min = wg_min; s_wl_min = wl_min;
-      s_wg_max = wg_max; s_wl_max = wl_max;
       A.ng = ng;
       A.nl = nl;
       A.m = ng * nl;
       A.p = (ng * nl + 1) / 2;
     }
-    __syncthreads();
   }
-  // axis nodes w_min * exp(dx * i) and their logs, radis/lbl/broadening.py:1837
-  for (int i = threadIdx.x; i < s_ng; i += blockDim.x) {
-    wgax[i] = s_wg_min * exp_call(dxG * (double)i);
-    lgax[i] = log_call(wgax[i]);
-    A.laG[i] = lgax[i];
-  }
-  for (int i = threadIdx.x; i < s_nl; i += blockDim.x) {
-    wlax[i] = s_wl_min * exp_call(dxL * (double)i);
-    llax[i] = log_call(wlax[i]);
-    A.laL[i] = llax[i];
+  // axis nodes w_min * exp(dx * i) and their logs, radis/lbl/broadening.py:1837:
+  // the G axis by waves 0 and 1, the L axis by waves 2 and 3 (each axis has at
+  // most LDM_MAX_AX = 128 nodes)
+  {
+    const bool lor = threadIdx.x >= LDM_MAX_AX;
+    const int i = threadIdx.x & (LDM_MAX_AX - 1);
+    if (i < (lor ? nl : ng)) {
+      const double w = (lor ? wl_min : wg_min) * exp_call((lor ? dxL : dxG) * (double)i), lw = log_call(w);
+      (lor ? wlax : wgax)[i] = w;
+      (lor ? llax : lgax)[i] = lw;
+      (lor ? A.laL : A.laG)[i] = lw;
+    }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i + 1 < s_ng; i += blockDim.x) A.slG[i] = 1.0 / (lgax[i + 1] - lgax[i]);
-  for (int i = threadIdx.x; i + 1 < s_nl; i += blockDim.x) A.slL[i] = 1.0 / (llax[i + 1] - llax[i]);
-  if (threadIdx.x == 0 && s_ng > 0) {
+  {
+    const bool lor = threadIdx.x >= LDM_MAX_AX;
+    const int i = threadIdx.x & (LDM_MAX_AX - 1);
+    const double* const la = lor ? llax : lgax;
+    if (i + 1 < (lor ? nl : ng)) (lor ? A.slL : A.slG)[i] = 1.0 / (la[i + 1] - la[i]);
+  }
+  if (threadIdx.x == 0 && ng > 0) {
     // FP32 fast positions work in log2 units (the hardware logarithm)
     const double LOG2E = 1.4426950408889634, LN2 = 0.6931471805599453;
     J.laG0_f = (float)(lgax[0] * LOG2E);
@@ -575,8 +603,7 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
     J.inv_dxG_f = (float)(LN2 / dxG);
     J.inv_dxL_f = (float)(LN2 / dxL);
   }
-  const int ng = s_ng, nl = s_nl;
-  int status = 0;
+  int status = threadIdx.x == 0 ? st0 : 0;
   const double PI = 3.141592653589793;
   const double h = 0.5 / wstep;                      // n/(2 wstep) step
   const double xrev0 = (double)(L / 2) * (1.0 / ((double)L * wstep));  // rfftfreq(L, wstep)[-1]
@@ -602,10 +629,10 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
     res[blockIdx.x].ng = ng;
     res[blockIdx.x].nl = nl;
     res[blockIdx.x].status = st;
-    res[blockIdx.x].wg_min = s_wg_min;
-    res[blockIdx.x].wg_max = s_wg_max;
-    res[blockIdx.x].wl_min = s_wl_min;
-    res[blockIdx.x].wl_max = s_wl_max;
+    res[blockIdx.x].wg_min = wg_min;
+    res[blockIdx.x].wg_max = wg_max;
+    res[blockIdx.x].wl_min = wl_min;
+    res[blockIdx.x].wl_max = wl_max;
   }
 }
 
