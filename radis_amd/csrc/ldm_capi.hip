@@ -561,11 +561,11 @@ int launch_set(const LaunchSet& X, const LdmDb& dbd, radis_ldm_batch* b, hipStre
     break;
 #define FC_C(N) FC_C1(N, 0, false, fc_cols_c(N), FC_T) FC_C1(N, FC_C_SUM, true, fc_cols_c(N), FC_T)
 #define FC_CN(N)                                              \
-  FC_C1(N, FC_NARROW, false, FC_COLS_C_NARROW, (N) / 2)       \
-  FC_C1(N, FC_NARROW | FC_C_SUM, true, FC_COLS_C_NARROW, (N) / 2)
+  FC_C1(N, FC_NARROW, false, fc_cols_c_narrow(N), fc_narrow_tc(N))       \
+  FC_C1(N, FC_NARROW | FC_C_SUM, true, fc_cols_c_narrow(N), fc_narrow_tc(N))
     switch (G.cls) {
       FC_C(256) FC_C(320) FC_C(384) FC_C(512) FC_C(640) FC_C(768) FC_C(1024)
-      FC_CN(256)
+      FC_CN(256) FC_CN(320) FC_CN(384) FC_CN(512)
       default: launch_part(b, timed, slot, 6, f, l, k_fft_c, grid, dim3(LDM_FFT_T), 0, s, cj, it, G.count);
     }
 #undef FC_C

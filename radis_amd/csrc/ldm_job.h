@@ -87,16 +87,20 @@ constexpr int fc_pow2_floor(int n) { return n < 2 ? 1 : 2 * fc_pow2_floor(n >> 1
 // workgroup of pass B for N2
 constexpr int fc_cols_a(int n1) { return fc_pow2_floor(FC_CAP_A / n1); }
 constexpr int fc_cols_c(int n1) { return fc_pow2_floor(FC_CAP / n1); }
-// narrow pass A and C tiles (16 and 8 columns), for launches whose wide ones
-// would leave CUs idle.  Pass A, wide -> narrow: n1 = 256, 72 blocks 9.2 -> 6.9 us;
+// narrow pass A and C tiles, for launches whose wide ones would leave CUs idle.
+// Pass A (16 columns), wide -> narrow: n1 = 256, 72 blocks 9.2 -> 6.9 us;
 // n1 = 384, 48 blocks 9.6 -> 7.1 us; n1 = 512, 112 blocks 13.3 -> 7.5 us; but
-// n1 = 320 (a middle stage of 0.5 passes) 224 blocks 12.5 -> 13.6 us.  Pass C
-// at n1 = 256 8.1 -> 6.8 us; at 384 and 512 6 -> 9 to 11 us, at 320 8.2 -> 10.4 us.
+// n1 = 320 (a middle stage of half a pass) 224 blocks 12.5 -> 13.6 us.  Pass C
+// (8 columns at n1 = 256, 4 above, a thread pass per last stage where that is
+// odd): n1 = 256 8.1 -> 6.8 us (4 columns: 14.9 us); 320, 32 blocks 8.5 -> 7.7 us and
+// with derived quantities, whose FP64 the few CUs are bound by, 16.0 -> 10.3 us;
+// 384, 8 blocks 7.7 -> 7.2 us; 512, 16 blocks 8.3 -> 7.2 us.
 constexpr bool fc_narrow_a(int n1) { return n1 == 256 || n1 == 384 || n1 == 512; }
-constexpr bool fc_narrow_c(int n1) { return n1 == 256; }
-constexpr int fc_narrow_ta(int n1) { return n1 == 384 ? 768 : n1; }  // threads of a narrow pass A tile
+constexpr bool fc_narrow_c(int n1) { return n1 <= 512; }
+constexpr int fc_narrow_ta(int n1) { return n1 == 384 ? 768 : n1; }  // threads of a narrow tile
+constexpr int fc_narrow_tc(int n1) { return n1 == 320 ? 320 : n1 == 384 ? 192 : n1 / 2; }
+constexpr int fc_cols_c_narrow(int n1) { return n1 == 256 ? 8 : 4; }
 #define FC_COLS_A_NARROW 16
-#define FC_COLS_C_NARROW 8
 #define FC_NARROW (1 << 21)  // pass A and C launch-class flag
 constexpr int fc_rows_b(int n2) { return FC_CAP_B / n2; }
 

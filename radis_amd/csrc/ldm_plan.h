@@ -864,7 +864,7 @@ int plan_exec(Req& R) {
   if (R.plan.fc) {
     R.bX[0] = floor_log2(R.narrow_a ? FC_COLS_A_NARROW : fc_cols_a(R.tn1));
     R.bX[1] = floor_log2(fc_rows_b(R.tn2));
-    R.bX[2] = floor_log2(R.narrow_c ? FC_COLS_C_NARROW : fc_cols_c(R.tn1));
+    R.bX[2] = floor_log2(R.narrow_c ? fc_cols_c_narrow(R.tn1) : fc_cols_c(R.tn1));
   } else {
     R.bX[0] = std::min({6, floor_log2(LDM_CAP / R.tn1), ctz(R.tn2)});
     R.bX[1] = std::min(floor_log2((R.tn2 <= LDM_CAP_B ? LDM_CAP_B : LDM_CAP) / R.tn2), ctz(R.tn1));
@@ -894,8 +894,9 @@ constexpr int FC_B_SPLIT_MAX = 4;
 constexpr double HALF_MIN_POINTS = 1 << 19;
 // wide column blocks below which the narrow ones run: a CU each (n1 = 256), or
 // half of that (384, 512: 768-thread tiles of three passes; between 128 and 256
-// wide blocks of 384 they took 14.5 -> 17.9 us)
-constexpr int FC_A_NARROW_DIV = 2, FC_C_NARROW_PER_CU = 1;
+// wide blocks of 384 they took 14.5 -> 17.9 us); pass C: a CU each, or a fourth (the batch's 320 class
+// of more blocks took 11.2 -> 12.8 us)
+constexpr int FC_A_NARROW_DIV = 2, FC_C_NARROW_DIV = 4;
 void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   // Half-length transforms pay where the launch's passes are more than a chain
   // of latencies: below HALF_MIN_POINTS (pairs times planned length) the
@@ -920,7 +921,7 @@ void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
     R.split_b = R.n_share = 1;
     if (!R.plan.fc) continue;
     R.narrow_a = fc_narrow_a(R.tn1) && cols_a[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_A_NARROW_DIV);
-    R.narrow_c = fc_narrow_c(R.tn1) && cols_c[R.tn1] < (long long)FC_C_NARROW_PER_CU * n_cu;
+    R.narrow_c = fc_narrow_c(R.tn1) && cols_c[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_C_NARROW_DIV);
     const int pairs = (R.m_cap + 1) / 2, rb = R.tn1 >> R.bX[1];
     // whole length: two shares, or more where its workspace is small (a share's
     // chain of pairs is what a lone small request waits for: 20,001 points,
