@@ -9,7 +9,7 @@
 //
 // Plan for N = 2^a * f, f in {1, 3, 5}: the odd factor f first (no twiddles),
 // then radix-16 stages, then one radix-2/4/8 stage for the remaining power
-// (pass B at N = 256 runs a variant with radix-4 end stages, fc_pv_ends4).
+// (fc_plan: the sizes with another one).
 // Columns: B = 2^bs independent columns of length N, element i of column b at
 // LDS slot pad_idx(i*B + b) (the same layout as the generic transform).
 #pragma once
@@ -19,21 +19,30 @@
 constexpr int fc_odd(int n) { return n % 3 == 0 ? 3 : (n % 5 == 0 ? 5 : 1); }
 constexpr int fc_log2(int n) { return n <= 1 ? 0 : 1 + fc_log2(n >> 1); }
 constexpr bool fc_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
-// Plan variant pv = 1 at N = 256 (pass B): radices 4, 16, 4 instead of
-// 16, 16.  Pass B keeps its first and last stages' elements in registers
-// (the next pair's prefetch; the accumulated spectrum and the lineshape
-// FTs), so a radix-16 end stage over 8 rows of 256 held 16 elements per
-// thread on half the threads (187 VGPRs); radix-4 ends hold 2 x 4 on all.
-constexpr bool fc_pv_ends4(int n, int pv) { return pv == 1 && n == 256; }
+// Radices (hexadecimal digits, the first stage's lowest)
+// of the sizes whose plan is not the general one; 0: general.  64 and 512 take
+// radix-8 stages only: as many stages as 16 x 4 and 16 x 16 x 2, with every
+// thread busy in each (a radix-16 stage of a 2048-element tile is 128
+// butterflies on 256 threads).  Plan variant pv = 1 (pass B): it keeps its first
+// and last stages' elements in registers (the next pair's prefetch; the
+// accumulated spectrum and the lineshape FTs), so a radix-16 end stage over 8
+// rows of 256 held 16 elements per thread on half the threads (187 VGPRs);
+// radix-4 ends at 256 and radix-8 ends at 1024 hold 8 on all.
+constexpr int fc_plan(int n, int pv) {
+  return n == 64 ? 0x88 : n == 512 ? 0x888 : pv == 1 && n == 256 ? 0x4f4 : pv == 1 && n == 1024 ? 0x8f8 : 0;  // f: 16
+}
 // number of stages and radix of stage s
 constexpr int fc_nstages(int n, int pv = 0) {
-  if (fc_pv_ends4(n, pv)) return 3;
+  if (fc_plan(n, pv)) return fc_plan(n, pv) >> 8 ? 3 : 2;
   const int f = fc_odd(n);
   const int a = fc_log2(n / f);
   return (f > 1 ? 1 : 0) + a / 4 + (a % 4 ? 1 : 0);
 }
 constexpr int fc_radix(int n, int s, int pv = 0) {
-  if (fc_pv_ends4(n, pv)) return s == 1 ? 16 : 4;
+  if (fc_plan(n, pv)) {
+    const int r = fc_plan(n, pv) >> (4 * s) & 15;
+    return r == 15 ? 16 : r;
+  }
   const int f = fc_odd(n);
   const int a = fc_log2(n / f);
   if (f > 1) {
@@ -423,14 +432,14 @@ __global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob
 // (2 x B x n_wh floats, n_wh >= N_L of every request with a correction).
 // ---------------------------------------------------------------------------
 template <int N2>
-__global__ __launch_bounds__(FC_T_B, (N2 >= 1024 || N2 == 256) ? 4 : 2) void k_fft_b_c(const LdmJob* __restrict__ jobs,
+__global__ __launch_bounds__(FC_T_B, N2 >= 256 ? 4 : 2) void k_fft_b_c(const LdmJob* __restrict__ jobs,
                                                       const LdmAxes* __restrict__ axes,
                                                       const int4* __restrict__ items, int n_rows_lds, int n_wh,
                                                       const int4* __restrict__ img, int n_img) {
   constexpr int CAP = FC_CAP_B, T = FC_T_B;
   constexpr int B = fc_rows_b(N2), LB = fc_log2(B);
   static_assert(fc_pow2(N2), "pass B rows are powers of two");
-  constexpr int PV = N2 == 256 ? 1 : 0;  // plan variant (fc_pv_ends4)
+  constexpr int PV = 1;  // plan variant (fc_plan)
   using SH = FcShape<N2, B, T, PV>;
   constexpr int NR0 = N2 / SH::R0;
   constexpr int NSL = fc_ns(N2, fc_nstages(N2, PV) - 1, PV);
