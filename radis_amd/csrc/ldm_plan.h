@@ -36,6 +36,7 @@ const int STAT_BLOCK = 4096;             // lines per host-side statistics block
 const int FILL_LDS_TARGET = 44 * 1024;   // preferred LDS bytes of one fill tile (FP64 cells; 3 tiles per CU)
 const int FILL_LDS_MAX = 60 * 1024;      // hard limit (plus ~2.2 KB of static axis tables, < 64 KB)
 const int MIN_TILE_W = 16, MAX_TILE_W = 4096;
+const int FILL_NARROW_W = 64;          // least width a tile is halved to for launches of few
 const int FILL_GROUP_TILE_W = 32;      // tile width of fills in row groups
 const int N1_MAX = 1024, N2_MAX = 8192;
 // grids beyond N1_MAX * N2_MAX: run-time-sized passes A and C with n1 up to
@@ -126,7 +127,7 @@ struct Req {
   int m_need = 0;      // bound for the current conditions
   int m_cap = 0;       // allocated rows
   int wrap_rows = 0;   // L-axis nodes of the image-correction table (N_L <= M/2: N_G >= 2)
-  int tile_w = 0, n_tiles = 0;
+  int tile_w = 0, n_tiles = 0, tile_shrink = 0;  // tile_shrink: halvings of a tile for launches of few
   int fill_rows = 0, fill_groups = 1;  // row groups of a fill tile (an LDM taller than one tile's LDS)
   int64_t stride = 0;
   int scale_log2 = 0;
@@ -817,6 +818,7 @@ bool half_ok(const Req& R, int tile_w) {
 // tn1, tn2), from its plan, its row capacity and its conditions.
 int plan_exec(Req& R) {
   R.tile_w = R.r.tile_w ? R.r.tile_w : choose_tile(R.m_cap);
+  if (!R.r.tile_w && R.tile_w > FILL_NARROW_W) R.tile_w = std::max(FILL_NARROW_W, R.tile_w >> R.tile_shrink);
   R.fill_rows = R.m_cap;
   R.fill_groups = 1;
   if (fill_tile_bytes(R.m_cap, R.tile_w) > (size_t)FILL_LDS_MAX) {
@@ -885,6 +887,7 @@ int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
 // (pass C adds their partial spectra): as many as fit FC_B_SPLIT_WGS_PER_CU
 // workgroups per CU at once, with FC_B_SPLIT_MIN_PAIRS pairs each; every
 // share costs an inverse transform and 8 tL bytes written and read.
+constexpr int FILL_TILES_PER_CU = 2;
 constexpr int FC_B_SPLIT_WGS_PER_CU = 4;
 constexpr int FC_B_SPLIT_MIN_PAIRS = 2;
 // bytes of Y up to which a whole-length transform's workspace may grow by more
@@ -898,6 +901,18 @@ constexpr double HALF_MIN_POINTS = 1 << 19;
 // of more blocks took 11.2 -> 12.8 us)
 constexpr int FC_A_NARROW_DIV = 2, FC_C_NARROW_DIV = 4;
 void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
+  // The widest tiles that fit LDS leave CUs idle on short grids: halve them until
+  // there are two a CU (50,001 points, 16 rows: 196 tiles of 256 points 17.9 us, 782
+  // of 64 12.0 us, 1563 of 32 12.2 us; 120,417 points: 471 of 256 14.0, 941 of 128
+  // 12.8, 1882 of 64 15.3 us).
+  long long tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    const int w = reqs[i].r.tile_w ? reqs[i].r.tile_w : choose_tile(reqs[i].m_cap);
+    tiles += (reqs[i].nv + w) / w;
+  }
+  int shrink = 0;
+  while (tiles << shrink < (long long)FILL_TILES_PER_CU * n_cu && shrink < 8) ++shrink;
+  for (int i = 0; i < n; ++i) reqs[i].tile_shrink = shrink;
   // Half-length transforms pay where the launch's passes are more than a chain
   // of latencies: below HALF_MIN_POINTS (pairs times planned length) the
   // shorter passes take as long as the whole ones and the correction is extra.
