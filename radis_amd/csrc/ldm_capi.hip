@@ -292,13 +292,21 @@ int build_layout(radis_ldm_batch* b) {
   b->ctx->in_use += (int64_t)twsz;
   // tables computed on the device (k_twiddles; the no-allocation entry
   // point builds its tables the same way)
+  std::vector<LdmTwiddles> tabs;
   for (auto& kv : sub_off)
-    hipLaunchKernelGGL(k_twiddles, dim3((kv.first + 255) / 256), dim3(256), 0, b->ctx->side,
-                       LdmTwiddles{(float2*)((char*)b->twmem + kv.second), nullptr, nullptr, kv.first, 0, 0});
-  for (auto& kv : l_off) {
-    const LdmTwiddles t{nullptr, nullptr, (float2*)((char*)b->twmem + kv.second), 0, 0, (long long)kv.first};
-    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((t.total() + 255) / 256, 4096)), dim3(256), 0,
-                       b->ctx->side, t);
+    tabs.push_back({(float2*)((char*)b->twmem + kv.second), nullptr, nullptr, kv.first, 0, 0});
+  for (auto& kv : l_off)
+    tabs.push_back({nullptr, nullptr, (float2*)((char*)b->twmem + kv.second), 0, 0, (long long)kv.first});
+  for (size_t at = 0; at < tabs.size(); at += LDM_TW_TABLES) {
+    const size_t n = std::min<size_t>(LDM_TW_TABLES, tabs.size() - at);
+    LdmTwiddleSet set{};
+    long long most = 0;
+    for (size_t i = 0; i < n; ++i) {
+      set.t[i] = tabs[at + i];
+      most = std::max(most, set.t[i].total());
+    }
+    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)std::min<long long>((most + 255) / 256, 4096), (unsigned)n), dim3(256), 0,
+                       b->ctx->side, set);
   }
   HIPCHK(hipGetLastError());
   for (Req& R : b->reqs) {
@@ -925,8 +933,6 @@ int radis_ldm_batch_create(radis_ldm_ctx* ctx, const radis_ldm_db* db, int n, co
       ok = b->jobs_h[k] && b->res_h[k] &&
            hipEventCreateWithFlags(&b->ev_done[k], hipEventDisableTiming) == hipSuccess;
       if (ok) std::memset(b->res_h[k], 0, sizeof(LdmResult) * n);
-      for (auto& e : b->st_ev[k])
-        if (ok && hipEventCreate(&e) != hipSuccess) ok = false;
     }
     if (!ok) rc = fail(RADIS_LDM_ENOMEM, "batch bookkeeping allocation failed");
   }
@@ -1109,6 +1115,14 @@ int radis_ldm_batch_workspace_bytes(const radis_ldm_batch* b, int64_t* bytes) {
 
 int radis_ldm_batch_enable_timing(radis_ldm_batch* b, int enable) {
   if (!b) return fail(RADIS_LDM_EINVAL, "null batch");
+  // the kernels' events exist from the first timed run on (32 of them created and
+  // destroyed took a tenth of a served batch)
+  if (enable) {
+    HIPCHK(hipSetDevice(b->ctx->device));
+    for (auto& slot : b->st_ev)
+      for (auto& e : slot)
+        if (!e) HIPCHK(hipEventCreate(&e));
+  }
   b->timing = enable != 0;
   return 0;
 }

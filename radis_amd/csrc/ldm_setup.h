@@ -40,7 +40,15 @@ struct LdmTwiddles {
   }
 };
 
-__global__ __launch_bounds__(256) void k_twiddles(LdmTwiddles t) {
+// The tables of a batch layout, a row of workgroups each (one launch: a launch
+// per table, up to 13 of a few hundred elements, was 40 us of a served batch's
+// set-up, which waits for them).
+#define LDM_TW_TABLES 32
+struct LdmTwiddleSet {
+  LdmTwiddles t[LDM_TW_TABLES];
+};
+__global__ __launch_bounds__(256) void k_twiddles(LdmTwiddleSet set) {
+  const LdmTwiddles& t = set.t[blockIdx.y];
   const long long total = t.total();
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
        i += (long long)gridDim.x * blockDim.x)
