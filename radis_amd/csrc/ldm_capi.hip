@@ -41,7 +41,9 @@ namespace {
 // runs on holds its own copy until the process ends.  In host code the name
 // is a stand-in, not a device address: kernels get the address that
 // hipGetSymbolAddress returns for the current device (scratch_address).
-static __device__ __align__(256) unsigned char scratch[RADIS_LDM_NOALLOC_BYTES];
+// (SCRATCH_TABLES bytes beyond the documented size: the axis tables' tile ranges.)
+#define SCRATCH_TABLES 4096
+static __device__ __align__(256) unsigned char scratch[RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES];
 
 namespace {
 
@@ -1168,7 +1170,7 @@ int radis_ldm_batch_copy_ldm(radis_ldm_batch* b, int i, float* dst, void* stream
   const long long cols = R.nv + 1;
   const long long n = (long long)rows * cols;
   hipLaunchKernelGGL(k_copy_ldm, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     (const float*)((char*)b->work + R.off_ldm), (long long)R.stride, rows, cols, dst);
+                     (const LdmJob*)b->jobs_d + i, (const LdmAxes*)b->axes_d + i, rows, cols, dst);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1213,7 +1215,7 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   const size_t o_twl = take((size_t)(nhi + 1024) * 8);
   const size_t o_twc = take((size_t)LDM_WRAP_LC * 8);
   const size_t o_work = take(work);
-  if (off > (size_t)RADIS_LDM_NOALLOC_BYTES)
+  if (off > (size_t)RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES)
     return fail(RADIS_LDM_ERANGE, "request needs %zu bytes of scratch, above the %lld of radis_ldm_run_noalloc "
                                   "(use a batch)", off, (long long)RADIS_LDM_NOALLOC_BYTES);
   const size_t o_items = items_in_work ? o_work + R.off_free : o_items_;

@@ -13,8 +13,11 @@
 // Columns: B = 2^bs independent columns of length N, element i of column b at
 // LDS slot pad_idx(i*B + b) (the same layout as the generic transform).
 #pragma once
+#include <type_traits>
+
 #include "ldm_fft.h"
 #include "ldm_image.h"
+#include "ldm_kernels.h"
 
 constexpr int fc_odd(int n) { return n % 3 == 0 ? 3 : (n % 5 == 0 ? 5 : 1); }
 constexpr int fc_log2(int n) { return n <= 1 ? 0 : 1 + fc_log2(n >> 1); }
@@ -350,25 +353,38 @@ __global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob
     // upper half of every column (n1 >= N1/2, n >= L/2) is zero and its
     // loads are skipped
     const bool upper_zero = (long long)V <= J.tL / 2;
-    // the two LDM rows, zero beyond V (and row b zero when the pair is odd)
+    // the two LDM rows, zero beyond V and where the fill wrote none (and row b
+    // zero when the pair is odd)
+    const PairColumns written(J, axes[it.x], p);
+    auto rows = [&](auto sparse) {
 #pragma unroll
-    for (int s = 0; s < SH::IT0; ++s) {
-      const int it0 = threadIdx.x + s * T;
+      for (int s = 0; s < SH::IT0; ++s) {
+        const int it0 = threadIdx.x + s * T;
 #pragma unroll
-      for (int q = 0; q < SH::R0; ++q) {
-        // s*(T/B) + q*NR0 is the smallest row n1 = e >> LB of this (s, q)
-        if (upper_zero && s * (T >> LB) + q * NR0 >= N1 / 2) {
-          v[s][q] = make_float2(0.0f, 0.0f);
-          continue;
+        for (int q = 0; q < SH::R0; ++q) {
+          // s*(T/B) + q*NR0 is the smallest row n1 = e >> LB of this (s, q)
+          if (upper_zero && s * (T >> LB) + q * NR0 >= N1 / 2) {
+            v[s][q] = make_float2(0.0f, 0.0f);
+            continue;
+          }
+          const int e = it0 + q * NR0 * B;
+          const int n = n2_0 + (e & (B - 1)) + N2 * (e >> LB);
+          const bool in = (SH::ITEMS0 % T == 0 || it0 < SH::ITEMS0) && n < V;
+          if constexpr (decltype(sparse)::value) {
+            // (lanes skipped: at one common address per pair they took longer)
+            float2 z = make_float2(0.0f, 0.0f);
+            if (in & written(n)) z = gld(rz, 8u * (unsigned)n);
+            v[s][q] = make_float2(z.x, has_b ? z.y : 0.0f);
+          } else {
+            const unsigned o = in ? 8u * (unsigned)n : 0u;  // n < V < 2^28
+            const float2 z = gld(rz, o);
+            v[s][q] = make_float2(in ? z.x : 0.0f, (in && has_b) ? z.y : 0.0f);
+          }
         }
-        const int e = it0 + q * NR0 * B;
-        const int n = n2_0 + (e & (B - 1)) + N2 * (e >> LB);
-        const bool in = (SH::ITEMS0 % T == 0 || it0 < SH::ITEMS0) && n < V;
-        const unsigned o = in ? 8u * (unsigned)n : 0u;  // n < V < 2^28
-        const float2 z = gld(rz, o);
-        v[s][q] = make_float2(in ? z.x : 0.0f, (in && has_b) ? z.y : 0.0f);
       }
-    }
+    };
+    if (written.all) rows(std::false_type{});
+    else rows(std::true_type{});
     return true;
   };
   // W_N1 table: the same for every request of this N1

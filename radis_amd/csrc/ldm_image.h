@@ -113,7 +113,8 @@ struct TileMoments {
       dst[threadIdx.x & 7] = s;
     }
   }
-  __device__ __forceinline__ void nodes(const LdmJob& J, int ng, int nl, int tile) {
+  // (the rows of G-axis nodes [l0, l1]: the others hold zeros)
+  __device__ __forceinline__ void nodes(const LdmJob& J, int l0, int l1, int nl, int tile) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     const int m = threadIdx.x, parts = tile_parts(W);
     if (m >= nl) return;  // N_L <= LDM_MAX_AX < LDM_FILL_T
@@ -121,7 +122,7 @@ struct TileMoments {
     for (int part = 0; part < parts; ++part) {
       const float4* x = red + part * (M + 1) + m;
 #pragma unroll 4
-      for (int l = 0; l < ng; ++l) {
+      for (int l = l0; l <= l1; ++l) {
         const float2 q = rows[l * nl + m];
         const float4 d = x[l * nl];
         const float hs = 0.5f * q.y;

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#define LDM_AX_PAIRS 256   // pairs of LDM rows with a table of their columns
 #define LDM_MAX_AX 128     // maximum N_G or N_L
 #define LDM_MAX_ISO 16     // isotopologue slots
 #define LDM_MAX_RAD 12     // radix stages per sub-FFT
@@ -276,7 +277,7 @@ struct LdmJob {
   // reduction targets and status, initialised by the host every run
   unsigned long long wl_min_bits, wl_max_bits, wg_min_bits, wg_max_bits;
   int status;
-  int pad0_;
+  int sparse_g;                  // 1: rows of G-axis nodes beyond a tile's reach are neither written nor read (LdmAxes::tlo)
 };
 
 // Device-computed LDM axes of one request (written by k_finalize).
@@ -284,6 +285,13 @@ struct LdmAxes {
   int ng, nl, m, p;                          // N_G, N_L, rows M = N_G*N_L, pairs P = ceil(M/2)
   double laG[LDM_MAX_AX], slG[LDM_MAX_AX];   // log of G-axis nodes, 1/(la[j+1]-la[j])
   double laL[LDM_MAX_AX], slL[LDM_MAX_AX];
+  // first and last fill tile whose lines can reach the rows of G-axis node l
+  // (both non-decreasing in l); beside them only the first tile and the last
+  // two of the grid, which hold the lines clamped onto its ends, have every row
+  int tlo[LDM_MAX_AX], thi[LDM_MAX_AX];
+  // the columns [x, x + y) of pair p's rows from these tiles, p < LDM_AX_PAIRS (pass A
+  // loads them with the axis sizes)
+  int2 pair[LDM_AX_PAIRS];
 };
 
 // Per-request results copied back to the host after every run.

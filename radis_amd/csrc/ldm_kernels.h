@@ -595,6 +595,43 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
     const double* const la = lor ? llax : lgax;
     if (i + 1 < (lor ? nl : ng)) (lor ? A.slL : A.slG)[i] = 1.0 / (la[i + 1] - la[i]);
   }
+  // A line of G-axis index j has node_j <= w < node_j+1, and w = nu0 times its
+  // isotopologue's constant: the rows of node l (j = l - 1, l) are reached from
+  // a range of nu0 only, widened by 1e-4 (an index is exact far inside that), the
+  // pressure shift and the stencil's columns.  j is clamped to [0, ng - 2].
+  if (J.sparse_g && ng > 2) {
+    double dmin = dopp1, dmax = dopp1;
+    if (!single) {
+      dmin = 1e300;
+      dmax = 0.0;
+      for (int s = 0; s < LDM_MAX_ISO; ++s) {
+        const double d = J.dopp[s];
+        if (d > 0.0) {
+          dmin = fmin(dmin, d);
+          dmax = fmax(dmax, d);
+        }
+      }
+    }
+    const double inv = J.inv_delta_w, wmin = J.wmin, shift = J.shift_margin;
+    const int last = J.n_tiles - 1, W = J.tile_w;
+    const double iw = 1.0 / (double)W, plo = (1.0 - 1e-4) * 0.5 * LDM_C_CGS / dmax, phi = (1.0 + 1e-4) * 0.5 * LDM_C_CGS / dmin;
+    auto first_tile = [&](int l) -> int {
+      if (l < 2) return 0;
+      return (int)fmin(fmax(floor(((wgax[l - 1] * plo - shift - wmin) * inv - 2.0) * iw), 0.0), (double)last);
+    };
+    auto last_tile = [&](int l) -> int {
+      if (l > ng - 3) return last;
+      return (int)fmin(fmax(floor(((wgax[l + 1] * phi + shift - wmin) * inv + 3.0) * iw), 0.0), (double)last);
+    };
+    if ((int)threadIdx.x < ng) {
+      A.tlo[threadIdx.x] = first_tile(threadIdx.x);
+      A.thi[threadIdx.x] = last_tile(threadIdx.x);
+    }
+    if ((int)threadIdx.x < (ng * nl + 1) / 2) {  // a thread for each of LDM_AX_PAIRS
+      const int p = threadIdx.x, t0 = first_tile(2 * p / nl), t1 = last_tile(min(2 * p + 1, ng * nl - 1) / nl);
+      A.pair[p] = make_int2(t0 * W, (t1 + 1 - t0) * W);
+    }
+  }
   if (threadIdx.x == 0 && ng > 0) {
     // FP32 fast positions work in log2 units (the hardware logarithm)
     const double LOG2E = 1.4426950408889634, LN2 = 0.6931471805599453;
@@ -922,6 +959,53 @@ __device__ __forceinline__ void line_terms(const LineConst& C, const LineRaw& r,
 // keeps rows [g * fill_rows, g * fill_rows + MR) only: each of its 8 atomics
 // checks its corner's row.  A request with fill_groups = 1 has one group of
 // every row.  HALF: some request of the launch runs half-length transforms.
+// The G-axis nodes [l0, l1] whose rows a tile's lines can reach (LdmAxes::tlo,
+// thi; every node in the grid's first tile and its last two).  With one isotopologue
+// the Gaussian width goes with nu0, so a tile meets two or three of the nodes
+// whatever N_G is: writing and reading the other rows' zeros was five sixths of
+// the LDM's traffic at N_G = 12, a third at N_G = 3.
+struct GNodes {
+  int l0, l1;
+  __device__ __forceinline__ GNodes(const LdmJob& J, const LdmAxes& A, int ng, int tile) : l0(0), l1(ng - 1) {
+    if (!J.sparse_g || ng <= 2 || tile == 0 || tile >= J.n_tiles - 2) return;  // uniform
+    const int lane = threadIdx.x & 63;
+    l0 = l1 = -1;
+    for (int base = 0; base < ng; base += 64) {
+      const int l = base + lane;
+      const bool in = l < ng;
+      const unsigned long long lo = __ballot(in && A.tlo[in ? l : 0] <= tile), hi = __ballot(in && A.thi[in ? l : 0] >= tile);
+      if (lo) l1 = base + 63 - __builtin_clzll(lo);
+      if (l0 < 0 && hi) l0 = base + __builtin_ctzll(hi);
+    }
+  }
+};
+// The columns of a pair of rows that the fill wrote: [0, w0), [a, a + len) and
+// [w1, V).  Without a branch, so that a thread's loads stay in flight together.
+static_assert(LDM_AX_PAIRS == 256, "k_finalize: a thread per pair");
+struct PairColumns {
+  int w0, a, w1;
+  unsigned len;
+  bool all;  // uniform
+  __device__ __forceinline__ PairColumns(const LdmJob& J, const LdmAxes& A, int p)
+      : w0(0), a(0), w1(0x7fffffff), len(~0u), all(!J.sparse_g || A.ng <= 2) {
+    if (all) return;
+    const int nl = A.nl, W = J.tile_w;
+    w0 = W;
+    w1 = (J.n_tiles - 2) * W;
+    if (p < LDM_AX_PAIRS) {
+      const int2 c = A.pair[p];
+      a = c.x;
+      len = (unsigned)c.y;
+    } else {
+      a = A.tlo[2 * p / nl] * W;
+      len = (unsigned)((A.thi[min(2 * p + 1, A.m - 1) / nl] + 1) * W - a);
+    }
+  }
+  __device__ __forceinline__ bool operator()(int n) const {
+    return ((unsigned)(n - a) < len) | (n < w0) | (n >= w1);
+  }
+};
+
 template <bool NONEQ, bool PLAIN, bool GROUPED, bool HALF>
 __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, const int4 it, const LdmDb& db,
                                           double* acc) {
@@ -969,6 +1053,8 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
     for (int e = threadIdx.x; e < n2; e += blockDim.x) a2[e] = make_double2(0.0, 0.0);
     if ((n & 1) && threadIdx.x == 0) acc[n - 1] = 0.0;
   }
+  // the G-axis nodes this tile's lines can reach: the flush writes their rows
+  const GNodes act(J, A, ng, tile);
   lds_barrier();
   const int wlen = (int)(k_hi - k_lo);
   const int sg = nl * Wp;
@@ -1041,11 +1127,14 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
   // per step: (2p, c), (2p+1, c), (2p, c+1), (2p+1, c+1); the second row of
   // an odd last pair is written as zeros.  W is a power of two; even rows
   // start 16-byte aligned.
-  const int P2 = (MR + 1) >> 1;
+  // Only the pairs with a row of a node the tile can reach: pass A does not read
+  // the others there (GNodes).
+  const int P0 = max(act.l0 * nl >> 1, r0 >> 1) - (r0 >> 1);
+  const int P2 = min((act.l1 + 1) * nl - r0 + 1, MR + 1) >> 1;
   const int W2 = W >> 1, sh2 = __builtin_ctz(W2);
   const long long pstride = 2 * J.ldm_stride;                   // floats per pair
   float* const out = J.ldm + 2 * k_lo + (long long)(r0 >> 1) * pstride;  // column k_lo of the group's first pair
-  for (int w = threadIdx.x; w < (P2 << sh2); w += LDM_FILL_T) {
+  for (int w = (P0 << sh2) + threadIdx.x; w < (P2 << sh2); w += LDM_FILL_T) {
     const int p = w >> sh2, c = 2 * (w & (W2 - 1));
     const double* src = acc + (2 * p) * Wp + c;
     const double2 a = *reinterpret_cast<const double2*>(src);
@@ -1061,7 +1150,7 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
   }
   if (half) {
     lds_barrier();
-    mom.nodes(J, ng, nl, tile);
+    mom.nodes(J, act.l0, act.l1, nl, tile);
   }
 }
 
@@ -1104,11 +1193,12 @@ __global__ __launch_bounds__(LDM_FFT_T, 4) void k_fft_a(const LdmJob* __restrict
   const float2* rz = reinterpret_cast<const float2*>(J.ldm) + (long long)p * J.ldm_stride;  // rows 2p, 2p+1
   const bool has_b = (2 * p + 1) < axes[it.x].m;
   const long long V = J.v;
+  const PairColumns written(J, axes[it.x], p);
   for (int e = threadIdx.x; e < (N1 << bs); e += LDM_FFT_T) {
     const int n1 = e >> bs, b = e & (B - 1);
     const long long n = n2_0 + b + (long long)N2 * n1;
     float xa = 0.0f, xb = 0.0f;
-    if (n < V) {
+    if (n < V && written((int)n)) {
       const float2 z = rz[n];
       xa = z.x;
       if (has_b) xb = z.y;

@@ -134,6 +134,7 @@ struct Req {
   int bA = 0, bB = 0, bC = 0;  // log2 of the pass A / C column blocks and pass B row blocks
   // what the passes run (plan_exec): the planned split, or for half the planned
   // length (half) one of its halves; bX: log2 of the columns / rows per workgroup
+  bool sparse_g = false;  // skip the rows of G-axis nodes beyond a tile's reach
   bool half = false, may_half = false, narrow_a = false, narrow_c = false;
   int64_t tL = 0;
   int tn1 = 0, tn2 = 0, bX[3] = {0, 0, 0};
@@ -796,6 +797,7 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.wl_max_bits = 0ull;
   J.wg_min_bits = ~0ull;
   J.wg_max_bits = 0ull;
+  J.sparse_g = R.sparse_g ? 1 : 0;
   J.status = 0;
 }
 
@@ -813,6 +815,13 @@ bool half_ok(const Req& R, int tile_w) {
   const double sigma = R.wg_hi * std::sqrt(std::max(1.0, IMG_TMAX / R.r.Tgas)) / (2.3548 * R.delta_w);
   return gap >= (double)IMG_TILES_PER_GAP * tile_w && gap >= IMG_SIGMAS_PER_GAP * sigma;
 }
+
+// Pairs times transform length from which the rows of the G-axis nodes that a
+// tile cannot reach are skipped: below it the passes are chains of latencies that
+// the ranges' look-up only lengthens (2.3 M points: fill and pass A -1.9 us,
+// k_finalize +1.2; 3.1 M, N_G = 3: pass A 12.4 -> 14.5 us), above it the bytes count (7.3 M, N_G = 3: fill and pass A -3.9 us,
+// k_finalize +0.6; 47 M, N_G = 12: -57 us of 534).
+constexpr long long SPARSE_G_POINTS = 1 << 22;
 
 // Tile width, row groups and the transform a request runs (Req::half, tL,
 // tn1, tn2), from its plan, its row capacity and its conditions.
@@ -863,6 +872,7 @@ int plan_exec(Req& R) {
     }
   }
   R.n_tiles = (int)((V + R.tile_w - 1) / R.tile_w);
+  R.sparse_g = (long long)((R.m_cap + 1) / 2) * R.tL >= SPARSE_G_POINTS;
   if (R.plan.fc) {
     R.bX[0] = floor_log2(R.narrow_a ? FC_COLS_A_NARROW : fc_cols_a(R.tn1));
     R.bX[1] = floor_log2(fc_rows_b(R.tn2));
