@@ -85,24 +85,27 @@ def stage_bytes(n_lines, info, db):
     tile_bounds : 0 (a few dozen probes of nu0 per tile: latency, not bytes)
     wrap        : 0 (4 K bytes per L-axis node of the image-correction table)
     fill        : 28 B/line (nu0 f64; S_ref, El, g_air, g_self, n_air f32) [+4 n_self] [+4 delta] [+1 iso]
-                  + 4*M*(N_v+1) LDM write
-    fft_a       : 4*M*(N_v+1) LDM read + 8*P*L packed-row spectra write
+                  + 4*R*(N_v+1) LDM write
+    fft_a       : 4*R*(N_v+1) LDM read + 8*P*L packed-row spectra write
     fft_b       : 8*P*L read + 8*L write
     fft_c       : 8*L read + 4*N_v abscoeff write
-    with L the length the passes run at (transform_len).
+    with L the length the passes run at (transform_len) and R the rows that
+    move per column: M, or from P L = 2^22 on (rows of G-axis nodes beyond a
+    tile's reach are skipped) at least the two nodes its lines fall between.
     """
     M = int(info.n_g * info.n_l)
     P = (M + 1) // 2
     L = transform_len(info)
     V = int(info.n_v) + 1
+    R = min(M, 2 * int(info.n_l)) if P * L >= 1 << 22 else M
     ns = 4 if db.has_nself else 0
     per_fill = 28 + ns + (4 if db.has_delta else 0) + (1 if db.has_iso else 0)
     return {
         "axis": int(info.axis_scanned) * (12 + ns + (9 if db.has_iso else 0)) + 16 * int(info.axis_candidates),
         "finalize": 0,
         "tile_bounds": 0,
-        "fill": n_lines * per_fill + 4 * M * V,
-        "fft_a": 4 * M * V + 8 * P * L,
+        "fill": n_lines * per_fill + 4 * R * V,
+        "fft_a": 4 * R * V + 8 * P * L,
         "fft_b": 8 * P * L + 8 * L,
         "fft_c": 8 * L + 4 * int(info.n_v),
         "wrap": 0,
