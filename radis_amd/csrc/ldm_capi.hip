@@ -251,7 +251,8 @@ int build_layout(radis_ldm_batch* b) {
   auto lay_out = [&](bool lean) {
     total = fill_lds = 0;
     fill_grouped = fill_half = false;
-    choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu, lean);
+    const int rc = choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu, lean);
+    if (rc) return rc;
     for (Req& R : b->reqs) {
       int rc = layout_request(R, total);
       if (rc) return rc;
@@ -879,7 +880,8 @@ int radis_ldm_request_bytes(const radis_ldm_db* db, const radis_ldm_request* req
   int rc = plan_one(*db, *req, R);
   if (rc) return rc;
   R.m_cap = R.m_need;
-  choose_split_b(&R, 1, db->ctx->n_cu);
+  rc = choose_split_b(&R, 1, db->ctx->n_cu);
+  if (rc) return rc;
   size_t total = 0;
   rc = layout_request(R, total);
   if (rc) return rc;
@@ -1189,7 +1191,8 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   int rc = plan_one(*db, *req, R);
   if (rc) return rc;
   R.m_cap = R.m_need;
-  choose_split_b(&R, 1, ctx->n_cu);
+  rc = choose_split_b(&R, 1, ctx->n_cu);
+  if (rc) return rc;
   size_t work = 0;
   rc = layout_request(R, work);
   if (rc) return rc;

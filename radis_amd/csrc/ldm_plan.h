@@ -910,7 +910,7 @@ constexpr double HALF_MIN_POINTS = 1 << 19;
 // wide blocks of 384 they took 14.5 -> 17.9 us); pass C: a CU each, or a fourth (the batch's 320 class
 // of more blocks took 11.2 -> 12.8 us)
 constexpr int FC_A_NARROW_DIV = 2, FC_C_NARROW_DIV = 4;
-void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
+int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   // The widest tiles that fit LDS leave CUs idle on short grids: halve them until
   // there are two a CU (50,001 points, 16 rows: 196 tiles of 256 points 17.9 us, 782
   // of 64 12.0 us, 1563 of 32 12.2 us; 120,417 points: 471 of 256 14.0, 941 of 128
@@ -934,7 +934,9 @@ void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   for (int i = 0; i < n; ++i) {
     Req& R = reqs[i];
     R.narrow_a = R.narrow_c = false;
-    if (plan_exec(R)) continue;  // reported by layout_request
+    // a request that cannot be laid out has no split to count
+    const int rc = plan_exec(R);
+    if (rc) return rc;
     if (!R.plan.fc) continue;
     cols_a[R.tn1] += (long long)((R.m_cap + 1) / 2) * (R.tn2 >> R.bX[0]);
     cols_c[R.tn1] += R.tn2 >> R.bX[2];
@@ -961,6 +963,7 @@ void choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
       R.split_b = 2;
     }
   }
+  return 0;
 }
 
 // Workspace of one request (tile width, pass splits and the offsets of its
