@@ -267,7 +267,9 @@ int radis_ldm_batch_line_terms(radis_ldm_batch *b, int i, int64_t *k0, int32_t *
                                float *tg, float *tl, float *I, void *stream);
 /* Copy request i's LDM as filled by the last run into dst (device,
  * row-major [n_g*n_l][n_v+1], rows r = l*N_L + m); the counterpart of the
- * LDM array of radis/lbl/broadening.py:2340-2346 (transposed). */
+ * LDM array of radis/lbl/broadening.py:2340-2346 (transposed).  A set_request
+ * that grows the workspace releases that LDM: RADIS_LDM_EINVAL until the next
+ * run. */
 int radis_ldm_batch_copy_ldm(radis_ldm_batch *b, int i, float *dst, void *stream);
 
 /* --- no-allocation entry point --------------------------------------------- */

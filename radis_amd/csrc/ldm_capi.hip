@@ -1169,6 +1169,8 @@ int radis_ldm_batch_copy_ldm(radis_ldm_batch* b, int i, float* dst, void* stream
   if (rc) return rc;
   const int rows = b->res_h[b->last_slot][i].ng * b->res_h[b->last_slot][i].nl;
   if (rows == 0) return 0;
+  // the device's job table still names the released buffers of the layout before
+  if (b->jobs_last.empty()) return fail(RADIS_LDM_EINVAL, "no run since the batch was laid out again: run it first");
   const long long cols = R.nv + 1;
   const long long n = (long long)rows * cols;
   hipLaunchKernelGGL(k_copy_ldm, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,

@@ -45,3 +45,23 @@ def test_tile_too_wide_for_two_rows_is_an_error(dev):
     assert oracle.rel_peak_error(b.results(b.run())[0], ref) <= TOL
     b.close()
     db.close()
+
+
+def test_ldm_copy_after_the_workspace_grew(dev):
+    """The LDM of the last run goes with its workspace: an error until the
+    next run, which fills it again."""
+    db = engine.LineDatabase(dev, _lines(2000, 2000.0, 2040.0, 5))
+    mk = lambda dx: engine.make_request(db, 2000.0, 2040.0, 0.002, 900.0, 1.3, 0.3, dxG=dx, dxL=dx)  # noqa: E731
+    b = engine.SpectrumBatch(db, [mk(0.45)])
+    b.run()
+    assert b.ldm(0).max() > 0
+    rows = int(b.info(0).m_cap)
+    b.set_request(0, mk(0.05))
+    assert b.info(0).m_cap > rows
+    with pytest.raises(_native.LdmError, match="run it first"):
+        b.ldm(0)
+    b.run()
+    ldm = b.ldm(0)
+    assert ldm.shape[0] > rows and np.all(np.isfinite(ldm)) and ldm.max() > 0
+    b.close()
+    db.close()
