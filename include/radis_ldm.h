@@ -203,7 +203,10 @@ int radis_ldm_request_bytes(const radis_ldm_db *db, const radis_ldm_request *req
  * buffer set-up and command recording (gpu.py:205-297).  A request's
  * conditions may later be changed with radis_ldm_batch_set_request as long
  * as the grid (wmin, wmax, wstep, fft_len) is unchanged; the workspace grows
- * by 1.5x when the new LDM size needs it (vulkan_compute_lib.py:1308-1323). */
+ * by 1.5x when the new LDM size needs it (vulkan_compute_lib.py:1308-1323).
+ * Conditions that the half-length passes do not take (RADIS_LDM_PERIOD_L above)
+ * have the next run, capture or replay lay the batch out again first (it then
+ * allocates, and waits for the stream). */
 int radis_ldm_batch_create(radis_ldm_ctx *ctx, const radis_ldm_db *db, int n,
                            const radis_ldm_request *reqs, radis_ldm_batch **out);
 int radis_ldm_batch_set_request(radis_ldm_batch *b, int i, const radis_ldm_request *req);
@@ -213,7 +216,9 @@ int radis_ldm_batch_set_request(radis_ldm_batch *b, int i, const radis_ldm_reque
  * Replaces gpuApp.iterate's run() (gpu.py:352-357). */
 int radis_ldm_batch_run(radis_ldm_batch *b, float *const *out_dev, void *stream);
 /* Capture the pipeline into a hipGraph bound to out_dev and replay it.
- * Conditions changed with _set_request are picked up by later replays. */
+ * Conditions changed with _set_request are picked up by later replays; one
+ * that grew the workspace ends the graph (replay: RADIS_LDM_EINVAL, capture
+ * again). */
 int radis_ldm_batch_graph_capture(radis_ldm_batch *b, float *const *out_dev, void *stream);
 int radis_ldm_batch_graph_replay(radis_ldm_batch *b, void *stream);
 /* Sizes and device results of request i.  n_g/n_l/status are read back

@@ -204,6 +204,8 @@ struct radis_ldm_batch {
   // launches of the FFT passes (see LaunchGroup)
   using Group = LaunchGroup;
   std::vector<Group> grp_a, grp_b, grp_c;
+  bool laid = false;         // the buffers and work items of a layout are there
+  bool check_half = false;   // conditions set since the layout: a half-length request may not be one any more
   bool tiles_valid = false;  // fill tile bounds computed for the current layout
   size_t fill_lds = 0;
   bool fill_grouped = false;  // some request fills its tiles in row groups
@@ -242,6 +244,7 @@ void free_layout(radis_ldm_batch* b) {
 
 int build_layout(radis_ldm_batch* b) {
   free_layout(b);
+  b->laid = false;
   b->jobs_last.clear();
   b->tiles_valid = false;
   // --- workspace
@@ -396,6 +399,8 @@ int build_layout(radis_ldm_batch* b) {
   b->fill_lds = std::max<size_t>(fill_lds, 4);
   b->fill_grouped = fill_grouped;
   b->fill_half = fill_half;
+  b->laid = true;
+  b->check_half = false;
   return 0;
 }
 
@@ -651,6 +656,47 @@ int wait_slot(radis_ldm_batch* b, int slot) {
 int wait_pending(radis_ldm_batch* b) {
   int rc = wait_slot(b, 0);
   if (!rc) rc = wait_slot(b, 1);
+  return rc;
+}
+
+// The launch sequence captured on s (not capturing itself) for b->graph_outs.
+int capture_graph(radis_ldm_batch* b, hipStream_t s) {
+  if (b->gexec) { (void)hipGraphExecDestroy(b->gexec); b->gexec = nullptr; }
+  if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
+  b->graph_valid = false;
+  if (!s) {
+    if (!b->own_stream) HIPCHK(hipStreamCreateWithFlags(&b->own_stream, hipStreamNonBlocking));
+    s = b->own_stream;
+  }
+  HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  const int rc = launch_kernels(b, s, false, 0, true);
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(s, &g);
+  if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
+  if (e != hipSuccess) return fail(RADIS_LDM_EHIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
+  b->graph = g;
+  HIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
+  b->graph_valid = true;
+  return 0;
+}
+
+// Before a launch on s: lay the batch out again where conditions set since the
+// last layout left the half-length rule (such a request then runs the whole
+// length), or where that layout failed.  Here and not in set_request, so that
+// the last run's LDM and a captured graph last until then; the graph is captured
+// again for the new layout.
+int ensure_layout(radis_ldm_batch* b, hipStream_t s) {
+  if (b->laid && !b->check_half) return 0;
+  bool again = !b->laid;
+  for (const Req& R : b->reqs) again = again || (R.half && !half_ok(R, R.tile_w));
+  b->check_half = false;
+  if (!again) return 0;
+  int rc = wait_pending(b);
+  if (rc) return rc;
+  HIPCHK(hipStreamSynchronize(s));  // LDM copies on it still read the old workspace
+  const bool graph = b->graph_valid;
+  rc = build_layout(b);
+  if (!rc && graph) rc = capture_graph(b, nullptr);
   return rc;
 }
 
@@ -974,12 +1020,10 @@ int radis_ldm_batch_set_request(radis_ldm_batch* b, int i, const radis_ldm_reque
   rc = bound_request(*b->db, T);
   if (rc) return rc;
   const bool grow = T.m_need > R.m_cap;
-  // conditions the half-length transform does not take (a Gaussian beyond
-  // IMG_TMAX kelvin's, min-RMS weights)
-  const bool whole = R.half && !half_ok(T, R.tile_w);
   R = T;
-  if (grow || whole) {
-    if (grow) R.m_cap = std::max(T.m_need, (int)std::ceil(1.5 * R.m_cap));  // vulkan_compute_lib.py:1308-1313
+  b->check_half = true;
+  if (grow) {
+    R.m_cap = std::max(T.m_need, (int)std::ceil(1.5 * R.m_cap));  // vulkan_compute_lib.py:1308-1313
     rc = build_layout(b);
     if (rc) return rc;
   }
@@ -991,13 +1035,15 @@ int radis_ldm_batch_run(radis_ldm_batch* b, float* const* out_dev, void* stream)
   for (int j = 0; j < b->n; ++j)
     if (!out_dev[j]) return fail(RADIS_LDM_EINVAL, "null output pointer for request %d", j);
   HIPCHK(hipSetDevice(b->ctx->device));
+  hipStream_t s = (hipStream_t)stream;
+  int rc = ensure_layout(b, s);
+  if (rc) return rc;
   const int slot = b->next_slot;
-  int rc = wait_slot(b, slot);
+  rc = wait_slot(b, slot);
   if (rc) return rc;
   for (int j = 0; j < b->n; ++j) b->outs[j] = out_dev[j];
   rc = refresh_jobs(b, slot, b->outs);
   if (rc) return rc;
-  hipStream_t s = (hipStream_t)stream;
   rc = enqueue(b, s, b->timing, slot);
   if (rc) return rc;
   b->slot_timed[slot] = b->timing;
@@ -1021,36 +1067,26 @@ int radis_ldm_batch_graph_capture(radis_ldm_batch* b, float* const* out_dev, voi
   HIPCHK(hipSetDevice(b->ctx->device));
   int rc = wait_pending(b);
   if (rc) return rc;
-  if (b->gexec) { (void)hipGraphExecDestroy(b->gexec); b->gexec = nullptr; }
-  if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
-  b->graph_outs.assign(out_dev, out_dev + b->n);
+  b->graph_valid = false;
   hipStream_t s = (hipStream_t)stream;
-  if (!s) {
-    if (!b->own_stream) HIPCHK(hipStreamCreateWithFlags(&b->own_stream, hipStreamNonBlocking));
-    s = b->own_stream;
-  }
-  HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  rc = launch_kernels(b, s, false, 0, true);
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(s, &g);
-  if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-  if (e != hipSuccess) return fail(RADIS_LDM_EHIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-  b->graph = g;
-  HIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
-  b->graph_valid = true;
-  return 0;
+  rc = ensure_layout(b, s);
+  if (rc) return rc;
+  b->graph_outs.assign(out_dev, out_dev + b->n);
+  return capture_graph(b, s);
 }
 
 int radis_ldm_batch_graph_replay(radis_ldm_batch* b, void* stream) {
   if (!b) return fail(RADIS_LDM_EINVAL, "null batch");
   if (!b->graph_valid || !b->gexec) return fail(RADIS_LDM_EINVAL, "no valid captured graph (capture again after a re-plan)");
   HIPCHK(hipSetDevice(b->ctx->device));
+  hipStream_t s = (hipStream_t)stream;
+  int rc = ensure_layout(b, s);
+  if (rc) return rc;
   const int slot = b->next_slot;
-  int rc = wait_slot(b, slot);
+  rc = wait_slot(b, slot);
   if (rc) return rc;
   rc = refresh_jobs(b, slot, b->graph_outs);
   if (rc) return rc;
-  hipStream_t s = (hipStream_t)stream;
   rc = upload_jobs(b, s, slot);
   if (rc) return rc;
   HIPCHK(hipGraphLaunch(b->gexec, s));

@@ -65,3 +65,70 @@ def test_ldm_copy_after_the_workspace_grew(dev):
     assert ldm.shape[0] > rows and np.all(np.isfinite(ldm)) and ldm.max() > 0
     b.close()
     db.close()
+
+
+def test_conditions_that_end_the_half_length_keep_graph_and_ldm(dev):
+    """set_request to min-RMS weights and to a temperature that the
+    half-length passes do not take: the LDM of the last run stays readable,
+    and the C entry's replays of the captured graph go on (no capture by the
+    caller), with eager runs between them."""
+    lines = _lines(3000, 2000.0, 2040.0, 7)
+    db = engine.LineDatabase(dev, lines)
+    mk = lambda T, p, opt="simple": engine.make_request(db, 2000.0, 2040.0, 0.001, T, p, 0.3, dxG=0.3, dxL=0.3,  # noqa: E731
+                                                        optimization=opt)
+    ref = {}
+    for T, p, opt in [(900.0, 1.0, "simple"), (900.0, 1.0, "min-RMS"), (4.0e6, 2.0, "simple"), (300.0, 1.5, "simple")]:
+        ref[T, p, opt] = oracle.eq_abscoeff(lines.as_dict(), 2000.0, 2040.0, 0.001, T, p, 0.3, 0.3, 0.3,
+                                            optimization=opt)
+    for first in ("min-RMS", "hot"):
+        change = (900.0, 1.0, "min-RMS") if first == "min-RMS" else (4.0e6, 2.0, "simple")
+        # (neighbouring rows hold tens of times a line with opposite signs: the parity bound)
+        tol = 1e-4 if first == "min-RMS" else TOL
+        rows = [mk(4.0e6, 2.0)] * 4  # row capacity for every condition
+        b = engine.SpectrumBatch(db, [mk(900.0, 1.0)] * 4)
+        for i, r in enumerate(rows):
+            b.set_request(i, r)  # (grows the workspace before the capture)
+            b.set_request(i, mk(900.0, 1.0))
+        outs = b.capture()
+        replay = lambda: b._lib.radis_ldm_batch_graph_replay(b._h, engine._stream_handle(None))  # noqa: E731
+        assert replay() == 0
+        assert oracle.rel_peak_error(b.results(outs)[1], ref[900.0, 1.0, "simple"]) <= TOL
+        ldm = b.ldm(1)
+        b.set_request(1, mk(*change))
+        np.testing.assert_array_equal(b.ldm(1), ldm)
+        for k in range(3):
+            assert replay() == 0
+            got = b.results(outs)
+            assert oracle.rel_peak_error(got[1], ref[change]) <= tol, (first, k)
+            assert oracle.rel_peak_error(got[0], ref[900.0, 1.0, "simple"]) <= TOL, (first, k)
+            eager = b.results(b.run())
+            assert oracle.rel_peak_error(eager[1], ref[change]) <= tol, (first, k)
+        b.set_request(1, mk(300.0, 1.5))
+        for k in range(2):
+            assert replay() == 0
+            assert oracle.rel_peak_error(b.results(outs)[1], ref[300.0, 1.5, "simple"]) <= TOL, (first, k)
+        b.close()
+    db.close()
+
+
+def test_batch_after_a_layout_that_did_not_fit(dev):
+    """A growth refused by the budget leaves no buffers: runs report the error
+    (nothing is launched) until the budget allows the layout."""
+    lines = _lines(2000, 2000.0, 2040.0, 9)
+    db = engine.LineDatabase(dev, lines)
+    mk = lambda dx: engine.make_request(db, 2000.0, 2040.0, 0.002, 900.0, 1.3, 0.3, dxG=dx, dxL=dx)  # noqa: E731
+    b = engine.SpectrumBatch(db, [mk(0.45)])
+    b.run()
+    dev.set_budget(dev.bytes_in_use())
+    try:
+        with pytest.raises(_native.BudgetExceeded):
+            b.set_request(0, mk(0.05))
+        for _ in range(2):
+            with pytest.raises(_native.BudgetExceeded):
+                b.run()
+    finally:
+        dev.set_budget(0)
+    ref = oracle.eq_abscoeff(lines.as_dict(), 2000.0, 2040.0, 0.002, 900.0, 1.3, 0.3, 0.05, 0.05)
+    assert oracle.rel_peak_error(b.results(b.run())[0], ref) <= TOL
+    b.close()
+    db.close()
