@@ -251,25 +251,15 @@ int build_layout(radis_ldm_batch* b) {
   size_t total = 0;
   size_t fill_lds = 0;
   bool fill_grouped = false, fill_half = false;
-  auto lay_out = [&](bool lean) {
-    total = fill_lds = 0;
-    fill_grouped = fill_half = false;
-    const int rc = choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu, lean);
+  int rc = choose_split_b(b->reqs.data(), (int)b->reqs.size(), b->ctx->n_cu, true);
+  if (rc) return rc;
+  for (Req& R : b->reqs) {
+    rc = layout_request(R, total);
     if (rc) return rc;
-    for (Req& R : b->reqs) {
-      int rc = layout_request(R, total);
-      if (rc) return rc;
-      fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R));
-      fill_grouped = fill_grouped || R.fill_groups > 1;
-      fill_half = fill_half || R.half;
-    }
-    return 0;
-  };
-  // beyond the budget: without the whole-length transforms' further shares
-  const size_t tables = (size_t)1 << 22;
-  int rc0 = lay_out(false);
-  if (!rc0 && b->ctx->budget > 0 && b->ctx->in_use + (int64_t)(total + tables) > b->ctx->budget) rc0 = lay_out(true);
-  if (rc0) return rc0;
+    fill_lds = std::max(fill_lds, fill_tile_bytes(R.fill_rows, R.tile_w) + fill_moment_bytes(R));
+    fill_grouped = fill_grouped || R.fill_groups > 1;
+    fill_half = fill_half || R.half;
+  }
   // --- twiddle tables, deduplicated by size
   std::map<int, size_t> sub_off;
   std::map<int64_t, size_t> l_off;
@@ -925,17 +915,9 @@ int radis_ldm_request_bytes(const radis_ldm_db* db, const radis_ldm_request* req
   Req R;
   int rc = plan_one(*db, *req, R);
   if (rc) return rc;
-  R.m_cap = R.m_need;
-  rc = choose_split_b(&R, 1, db->ctx->n_cu);
+  int64_t b = 0;
+  rc = request_bytes(R, db->ctx->n_cu, b);
   if (rc) return rc;
-  size_t total = 0;
-  rc = layout_request(R, total);
-  if (rc) return rc;
-  // the batch's work items and job table (16 B per item, a few per tile and block)
-  int64_t b = (int64_t)total + (int64_t)R.n_tiles * R.fill_groups * 16;
-  // twiddle tables, plus alignment slack: an upper bound of what a batch of
-  // this one request allocates
-  b += (int64_t)(R.plan.n1 + R.plan.n2 + 1024 + (R.plan.L >> LDM_TW_LO_BITS) + 1) * 8 + 64 * 1024;
   *bytes = b;
   if (info) {
     std::memset(info, 0, sizeof *info);

@@ -441,7 +441,7 @@ __global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob
 // spectrum goes through LDS into the inverse transform, whose last stage
 // writes B with the W_L twiddle.  Item (job, y, z): number
 // y * split_b + z, row block number / n_share, share number % n_share of its
-// pairs, whose partial spectrum goes to bbuf + share * share_stride (pass C
+// pairs, whose partial spectrum goes to bbuf + share_at[share] (pass C
 // adds them).  The dynamic LDS (sized per
 // launch) holds the rows' lineshape coefficients (n_rows_lds float4), then
 // the image-correction values of the block's rows at its two corrected bins
@@ -481,10 +481,8 @@ __global__ __launch_bounds__(FC_T_B, N2 >= 256 ? 4 : 2) void k_fft_b_c(const Ldm
   const int share = it.w & 15, k1_0 = (it.w >> 4) * B;
   const int L = (int)J.tL;  // <= 2^21
   const int P = axes[it.x].p, M = axes[it.x].m;
-  // this workgroup's pairs (share_inv, as a division is 40 instructions)
-  const unsigned inv = J.share_inv;
-  const int p0 = (int)((unsigned)(P * share) * inv >> 16);
-  const int p1 = share + 1 == J.n_share ? P : (int)((unsigned)(P * (share + 1)) * inv >> 16);
+  const int2 mine = share_pairs(J, P, share);  // this workgroup's pairs
+  const int p0 = mine.x, p1 = mine.y;
   fc_load_tw_stages<N2, T, PV>(s_tw, J.tw2);
   // The rows' lineshape coefficients (a_l, b_m, 1/F(0), fold count) staged
   // in LDS.  Read from global memory they are scalar loads, and the LDS
@@ -688,7 +686,7 @@ __global__ __launch_bounds__(FC_T_B, N2 >= 256 ? 4 : 2) void k_fft_b_c(const Ldm
     }
   }
   __syncthreads();
-  float2* Bo = J.bbuf + share * J.share_stride + (long long)k1_0 * N2;
+  float2* Bo = J.bbuf + J.share_at[share] + (long long)k1_0 * N2;
   // output n2 of this thread's last-stage element (s, q): j0 + s*(T/B) + q*NS, row k1 fixed
   TwProg<SH::ITL, SH::RL> tw;
   tw.init(J, k1_0 + (threadIdx.x & (B - 1)), threadIdx.x >> LB, T >> LB, NSL);
@@ -750,9 +748,9 @@ __global__ __launch_bounds__(T, 4) void k_fft_c_c(const LdmJob* __restrict__ job
       }
     }
   };
-  fetch(J.bbuf, false);
+  fetch(SUM ? J.bbuf + J.share_at[0] : J.bbuf, false);
   if constexpr (SUM) {
-    for (int s = 1; s < J.n_share; ++s) fetch(J.bbuf + s * J.share_stride, true);
+    for (int s = 1; s < J.n_share; ++s) fetch(J.bbuf + J.share_at[s], true);
   }
   auto ld = [&](int s, int q, int) -> float2 { return v[s][q]; };
   ImageEval img{};

@@ -58,6 +58,7 @@ static_assert(LDM_AX_CHUNK == LDM_SKY_BLOCK, "a partial block is one scan chunk"
 #define FC_T 512
 #define FC_CAP_B 2048  // complex elements of a pass B tile
 #define FC_T_B 256
+#define FC_B_SPLIT_MAX 4  // most workgroups per pass B row block
 #define FC_C_SUM (1 << 20)  // pass C launch-class flag: B is the sum of two pass B shares
 #define FC_B_ROWS_LDS 512  // rows whose lineshape coefficients pass B stages in LDS (more: read from global memory)
 // Half-length transforms (ldm_image.h): the compiled passes run at half the
@@ -232,11 +233,12 @@ struct LdmJob {
   long long tL;
   int tn1, tn2;
   // pass B's partial spectra: share s of a row block's pairs goes to
-  // bbuf + s * share_stride (n_share of them, added by pass C); a pass B item
+  // bbuf + share_at[s] (n_share of them, added by pass C); a pass B item
   // (y, z, w) is number y * split_b + z, row block w >> 4, share w & 15
   int n_share, split_b;
   unsigned share_inv;            // 2^16 / n_share: share s takes the pairs from P s share_inv >> 16
-  long long share_stride;
+  long long share_at[FC_B_SPLIT_MAX];  // (share_in_y: written by k_finalize)
+  int share_in_y;                // 1: bbuf is Y
   // half-length transforms: per cell IMG_NODES values of the correction
   double* img_u;                 // [n_cell][IMG_NODES]
   int cell_tiles, n_cell;        // fill tiles per cell, cells
@@ -252,7 +254,7 @@ struct LdmJob {
   float* row_inv_f0;             // [m_cap] 1/F_lm(0)
   float* ldm;                    // [ceil(m_cap/2)][ldm_stride] float2: rows 2p, 2p+1 interleaved
   float2* ybuf;                  // [(m_cap+1)/2][L]
-  float2* bbuf;                  // [n_share][share_stride] pass B's partial spectra
+  float2* bbuf;                  // [n_share] pass B's partial spectra, at share_at
   float2* bbuf2;                 // null: pass B not split
   float* out;                    // [nv]
   // derived outputs (null = not wanted): absorbance, transmittance, emissivity, radiance

@@ -179,6 +179,14 @@ __device__ __forceinline__ unsigned long long row_extreme(unsigned long long v) 
   return v;
 }
 
+// Pairs [x, y) of pass B's share of P pairs (share_inv, as a division is 40
+// instructions).
+__device__ __forceinline__ int2 share_pairs(const LdmJob& J, int P, int share) {
+  const unsigned inv = J.share_inv;
+  const int p0 = (int)((unsigned)(P * share) * inv >> 16);
+  return make_int2(p0, share + 1 == J.n_share ? P : (int)((unsigned)(P * (share + 1)) * inv >> 16));
+}
+
 // Width extremes as FP64 bit patterns; reduce() leaves every lane of every wave
 // with those of a workgroup of 256 (gauss false: without the Gaussian ones).
 struct WidthExtremes {
@@ -503,6 +511,7 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
   if (J.half)  // the image correction is accumulated by the pass B launch
     for (int e = threadIdx.x; e < J.n_cell * IMG_NODES; e += blockDim.x) J.img_u[e] = 0.0;
   const double nu_a = ends ? db.nu0[i0] : 0.0, nu_b = ends ? db.nu0[i1 - 1] : 0.0;
+  const int n_share = J.share_in_y ? J.n_share : 0;
   // Q(Tref)/Q(T) of the slots with a partition-function spline (the fill
   // reads these after this kernel): calc_linestrength_eq's Qref/Q,
   // radis/lbl/base.py:2605-2697
@@ -574,6 +583,16 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
       A.m = ng * nl;
       A.p = (ng * nl + 1) / 2;
     }
+  }
+  // A partial spectrum in Y replaces its share's first pair: of its rows only the
+  // share's workgroup reads them, all before it writes.  A share without pairs
+  // (P far below the planned ones) takes one that nobody reads: P + share < pairs
+  // planned, as those are at least two per share.  (By wave 3: wave 0 is the one
+  // the others wait for.)
+  if (const int s = (int)threadIdx.x - 192; s >= 0 && s < n_share) {
+    const int P = (ng * nl + 1) / 2;
+    const int2 p = share_pairs(J, P, s);
+    J.share_at[s] = (p.y > p.x ? p.x : P + s) * J.tL;
   }
   // axis nodes w_min * exp(dx * i) and their logs, radis/lbl/broadening.py:1837:
   // the G axis by waves 0 and 1, the L axis by waves 2 and 3 (each axis has at

@@ -128,6 +128,7 @@ struct Req {
   int m_cap = 0;       // allocated rows
   int wrap_rows = 0;   // L-axis nodes of the image-correction table (N_L <= M/2: N_G >= 2)
   int tile_w = 0, n_tiles = 0, tile_shrink = 0;  // tile_shrink: halvings of a tile for launches of few
+  int wide_tiles = 0;  // tiles at the width before any halving (request_bytes)
   int fill_rows = 0, fill_groups = 1;  // row groups of a fill tile (an LDM taller than one tile's LDS)
   int64_t stride = 0;
   int scale_log2 = 0;
@@ -142,6 +143,7 @@ struct Req {
   double wg_hi = 0;    // bound of the Gaussian FWHM (cm-1)
   int split_b = 1;     // 2: pass B's pairs are split over several workgroups per row block
   int n_share = 1;     // workgroups per pass B row block, each taking a share of the pairs
+  bool share_in_y = false;  // the shares' partial spectra lie in Y (LdmJob::share_at)
   int n_axp = 0;       // axis partials (items of k_axis)
   bool sky_whole = false;  // width extremes from the whole list's Pareto sets in k_finalize (no k_axis items)
   size_t off_ldm = 0, off_y = 0, off_b = 0, off_b2 = 0, off_rows = 0, off_axp = 0, off_wrap = 0;
@@ -762,7 +764,9 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.ybuf = (float2*)(work + R.off_y);
   J.bbuf = (float2*)(work + R.off_share);
   J.share_inv = 65536u / (unsigned)R.n_share;
-  J.share_stride = R.half || R.n_share > 2 ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
+  J.share_in_y = R.share_in_y ? 1 : 0;
+  const long long share_stride = R.half || R.n_share > 2 || R.share_in_y ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
+  for (int i = 0; i < R.n_share; ++i) J.share_at[i] = i * share_stride;
   J.mom = R.half ? (float*)(work + R.off_mom) : nullptr;
   J.img_u = R.half ? (double*)(work + R.off_img) : nullptr;
   J.cell_tiles = R.cell_tiles;
@@ -843,6 +847,8 @@ int plan_exec(Req& R) {
     R.fill_groups = (R.m_cap + rows - 1) / rows;
   }
   const int64_t V = R.nv + 1;
+  const int wide = R.r.tile_w ? R.r.tile_w : R.fill_groups > 1 ? R.tile_w : choose_tile(R.m_cap);
+  R.wide_tiles = (int)((V + wide - 1) / wide);
   // The passes' bytes and operations go with the transform length, and half of
   // the planned one still holds the grid: compiled passes run at L / 2 (half
   // of n1 down to 256, else half of n2) wherever the correction of its images
@@ -900,10 +906,10 @@ int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
 constexpr int FILL_TILES_PER_CU = 2;
 constexpr int FC_B_SPLIT_WGS_PER_CU = 4;
 constexpr int FC_B_SPLIT_MIN_PAIRS = 2;
-// bytes of Y up to which a whole-length transform's workspace may grow by more
-// than the one further partial spectrum that it always had room for
+// bytes of Y up to which a whole-length transform has more than two shares (not
+// lean: up to which its workspace may grow by more than the one further partial
+// spectrum)
 constexpr int64_t FC_B_SPLIT_WHOLE_Y = 64 << 20;
-constexpr int FC_B_SPLIT_MAX = 4;
 constexpr double HALF_MIN_POINTS = 1 << 19;
 // wide column blocks below which the narrow ones run: a CU each (n1 = 256), or
 // half of that (384, 512: 768-thread tiles of three passes; between 128 and 256
@@ -946,21 +952,26 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   for (int i = 0; i < n; ++i) {
     Req& R = reqs[i];
     R.split_b = R.n_share = 1;
+    R.share_in_y = false;
     if (!R.plan.fc) continue;
     R.narrow_a = fc_narrow_a(R.tn1) && cols_a[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_A_NARROW_DIV);
     R.narrow_c = fc_narrow_c(R.tn1) && cols_c[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_C_NARROW_DIV);
     const int pairs = (R.m_cap + 1) / 2, rb = R.tn1 >> R.bX[1];
-    // whole length: two shares, or more where its workspace is small (a share's
-    // chain of pairs is what a lone small request waits for: 20,001 points,
-    // twelve pairs in two shares 14.4 us)
+    // whole length: two shares, or more where Y is small (a share's chain of pairs
+    // is what a lone small request waits for: 20,001 points, twelve pairs in two
+    // shares 14.6 us, in four 10.0).  In the no-allocation entry point's scratch
+    // array their partial spectra have buffers of their own; batches are lean,
+    // with the spectra in Y: requests are admitted by request_bytes, and three
+    // further spectra were up to a fifth of a small request's workspace.
     const long long room = std::max<long long>(0, (long long)FC_B_SPLIT_WGS_PER_CU * n_cu - images[R.tn2]);
     int ns = (int)std::min<long long>(room / blocks[R.tn2], pairs / FC_B_SPLIT_MIN_PAIRS);
-    const bool room_whole = (int64_t)pairs * R.plan.L * 8 <= FC_B_SPLIT_WHOLE_Y && !lean;
+    const bool room_whole = (int64_t)pairs * R.plan.L * 8 <= FC_B_SPLIT_WHOLE_Y;
     ns = std::min(ns, R.half || room_whole ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);
     if (R.half && ns > 2) ns = std::min(ns, pairs - 1 - pairs / 8);  // they share Y's unused half with the moments
     if (ns > 1) {
       R.n_share = ns;
       R.split_b = 2;
+      R.share_in_y = lean && !R.half;
     }
   }
   return 0;
@@ -984,9 +995,8 @@ int layout_request(Req& R, size_t& total) {
   R.off_ldm = total; total = align_up(total + (size_t)pcap * 2 * R.stride * 4, 256);
   // one partial spectrum of length L (two of L / 2)
   R.off_b = total;   total = align_up(total + (size_t)R.plan.L * 8, 256);
-  // Y, for the whole length whatever runs (a request's workspace does not
-  // depend on its conditions); half-length transforms use its first half, and
-  // their correction and further partial spectra lie in the second
+  // Y, for the whole length whatever runs; half-length transforms use its first
+  // half, and their correction and further partial spectra lie in the second
   R.off_y = total;   total = align_up(total + (size_t)pcap * R.plan.L * 8, 256);
   R.off_share = R.off_b;
   if (R.half) {
@@ -1001,6 +1011,8 @@ int layout_request(Req& R, size_t& total) {
     R.off_free = align_up(o, 256);
     if (o > total) return fail(RADIS_LDM_EINVAL, "internal: half-length buffers exceed the workspace");
     R.off_b2 = R.off_y;
+  } else if (R.share_in_y) {
+    R.off_b2 = R.off_share = R.off_y;
   } else {
     // pass B's second share of the pairs, or all of more than two shares
     R.off_b2 = total;
@@ -1028,7 +1040,8 @@ int check_layout(const Req& R, size_t total) {
                   (R.split_b == 1 || R.off_b2 + (size_t)R.plan.L * 8 <= total) && R.off_rows + (size_t)R.m_cap * 16 <= total &&
                   R.off_axp + parts * 32 <= total && (size_t)R.n_axp <= parts &&
                   R.off_wrap + (size_t)R.wrap_rows * R.plan.wrap_k * 4 <= total &&
-                  R.off_share + (size_t)(R.n_share - 1) * (R.half || R.n_share > 2 ? (size_t)R.tL * 8 : R.off_b2 - R.off_b) + (size_t)R.tL * 8 <= total &&
+                  (R.share_in_y ? !R.half && R.off_share == R.off_y && (R.m_cap + 1) / 2 >= 2 * R.n_share
+                                : R.off_share + (size_t)(R.n_share - 1) * (R.half || R.n_share > 2 ? (size_t)R.tL * 8 : R.off_b2 - R.off_b) + (size_t)R.tL * 8 <= total) &&
                   (!R.half || (R.tL * 2 == R.plan.L && (size_t)R.tL >= V && (long long)R.n_cell * R.cell_tiles >= R.n_tiles &&
                                R.off_y + (size_t)((R.m_cap + 1) / 2) * R.tL * 8 <= R.off_img &&
                                R.off_img + (size_t)R.n_cell * IMG_NODES * 8 <= R.off_mom &&
@@ -1087,6 +1100,23 @@ __host__ __device__ inline int4 plan_item(const LdmItemPlan& P, int i) {
 }
 
 namespace {
+
+// Bytes that a batch of this one request allocates, at most; in a batch of
+// several it takes no more: more points there only favour the half length, more
+// row blocks fewer shares.
+int request_bytes(Req& R, int n_cu, int64_t& bytes) {
+  R.m_cap = R.m_need;
+  int rc = choose_split_b(&R, 1, n_cu, true);
+  if (rc) return rc;
+  size_t total = 0;
+  rc = layout_request(R, total);
+  if (rc) return rc;
+  // work items and job table (16 B per item, a few per tile and block)
+  bytes = (int64_t)total + (int64_t)R.wide_tiles * R.fill_groups * 16;
+  // twiddle tables, plus alignment slack
+  bytes += (int64_t)(R.plan.n1 + R.plan.n2 + 1024 + (R.plan.L >> LDM_TW_LO_BITS) + 1) * 8 + 64 * 1024;
+  return 0;
+}
 
 // Work-item plan of one request (after layout_request): axis items (edge
 // chunks scanned line by line, whole blocks through their width candidates

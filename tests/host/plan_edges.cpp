@@ -1,6 +1,11 @@
 // Edges of the host planning, one section per argument:
 //   wide_tile   an explicit fill tile too wide for two LDM rows is refused by
 //               the planning itself, alone and beside requests that plan
+//   shares_in_y pass B's partial spectra in Y: no share's overlaps what another
+//               reads or writes
+//   bytes       the admission figure: at most one transform's buffers and a
+//               second partial spectrum, and no less than what batches of such
+//               requests lay out
 #include <cstdio>
 #include <cstring>
 
@@ -50,10 +55,103 @@ void wide_tile() {
         }
 }
 
+// Partial spectra in Y: every share of every number of pairs up to the planned
+// one writes a pair of its own that no other share reads (share_pairs, and
+// k_finalize for share_at).
+void shares_in_y() {
+  int split = 0;
+  for (int64_t nv : {4000, 9000, 20001, 50001, 150001})
+    for (int m_cap = 1; m_cap <= 144; ++m_cap) {
+      Req R = request(nv, m_cap, 0, RADIS_LDM_MIN_RMS);
+      CHECK(choose_split_b(&R, 1, 256, true) == 0, "%s", g_err);
+      size_t total = 0;
+      CHECK(layout_request(R, total) == 0 && check_layout(R, total) == 0, "%s", g_err);
+      CHECK(!R.half && R.share_in_y == (R.n_share > 1), "whole length");
+      if (R.n_share == 1) continue;
+      ++split;
+      const int pcap = (m_cap + 1) / 2, n = R.n_share;
+      const unsigned inv = 65536u / n;
+      for (int P = 0; P <= pcap; ++P) {
+        auto lo = [&](int s) { return s == n ? P : (int)((unsigned)(P * s) * inv >> 16); };
+        std::vector<int> reader(pcap, -1), writer(pcap, -1);
+        for (int s = 0; s < n; ++s)
+          for (int p = lo(s); p < lo(s + 1); ++p) reader[p] = s;
+        for (int p = 0; p < P; ++p) CHECK(reader[p] >= 0, "pair %d of %d unread", p, P);
+        for (int s = 0; s < n; ++s) {
+          const int at = lo(s + 1) > lo(s) ? lo(s) : P + s;
+          CHECK(at < pcap && writer[at] < 0 && (reader[at] < 0 || reader[at] == s), "share %d of %d, %d of %d pairs: at %d", s, n, P, pcap, at);
+          if (at < pcap) writer[at] = s;
+        }
+      }
+    }
+  CHECK(split > 300, "%d split", split);
+}
+
+// LDM, Y, a partial spectrum (two where pass B is split over two shares: four
+// pairs or more, and twice the row blocks fit four workgroups per CU), rows,
+// axis partials, correction table, fill items at the full tile width, tables.
+int64_t figure(const Req& R, int n_cu) {
+  size_t t = 0;
+  auto put = [&](size_t n) { t = align_up(t + n, 256); };
+  const size_t pcap = (R.m_cap + 1) / 2, L = R.plan.L;
+  put(pcap * 2 * align_up(R.nv + 1, 64) * 4);
+  put(pcap * L * 8);
+  put(L * 8);
+  if (R.plan.fc && pcap >= 4 && 2 * (R.plan.n1 / fc_rows_b(R.plan.n2)) <= 4 * n_cu) put(L * 8);
+  put((size_t)R.m_cap * 16);
+  put((size_t)((R.i1 - R.i0 + LDM_AX_CHUNK - 1) / LDM_AX_CHUNK + 2) * 32);
+  put((size_t)(R.plan.wrap_k ? std::max(1, std::min(R.m_cap / 2, LDM_MAX_AX)) : 0) * R.plan.wrap_k * 4);
+  int w = R.r.tile_w ? R.r.tile_w : choose_tile(R.m_cap), groups = 1;
+  if (fill_tile_bytes(R.m_cap, w) > (size_t)FILL_LDS_MAX) {
+    if (!R.r.tile_w) w = FILL_GROUP_TILE_W;
+    const int rows = (int)((size_t)FILL_LDS_TARGET / fill_tile_bytes(1, w)) & ~1;
+    groups = (R.m_cap + rows - 1) / rows;
+  }
+  return (int64_t)t + (R.nv + w) / w * groups * 16 + (int64_t)(R.plan.n1 + R.plan.n2 + 1024 + (L >> LDM_TW_LO_BITS) + 1) * 8 + 64 * 1024;
+}
+
+void bytes() {
+  int halves = 0, wholes = 0;
+  for (int64_t nv = 2000; nv < 1000000; nv = nv * 21 / 20 + 7)
+    for (int m_cap : {1, 4, 9, 16, 18, 30, 61, 144, 700})
+      for (int flags : {0, RADIS_LDM_MIN_RMS})
+        for (int tile : {0, 32}) {
+          Req R = request(nv, m_cap, tile, flags);
+          int64_t b = 0;
+          CHECK(request_bytes(R, 256, b) == 0, "%s", g_err);
+          CHECK(b <= figure(R, 256), "nv %lld, %d rows: %lld B, %lld for two shares", (long long)nv, m_cap, (long long)b,
+                (long long)figure(R, 256));
+          (R.half ? halves : wholes)++;
+          // alone, with others of its kind, and with others of other sizes
+          for (int n : {1, 2, 5, 9})
+            for (int mixed : {0, 1}) {
+              std::vector<Req> reqs;
+              int64_t sum = 0;
+              for (int i = 0; i < n; ++i) {
+                Req Q = mixed && i ? request(nv * (1 + i) / 3 + 1500, 4 + 7 * i, 0, i % 2 ? RADIS_LDM_MIN_RMS : 0) : request(nv, m_cap, tile, flags);
+                int64_t q = 0;
+                CHECK(request_bytes(Q, 256, q) == 0, "%s", g_err);
+                sum += q;
+                reqs.push_back(mixed && i ? request(nv * (1 + i) / 3 + 1500, 4 + 7 * i, 0, i % 2 ? RADIS_LDM_MIN_RMS : 0) : request(nv, m_cap, tile, flags));
+              }
+              CHECK(choose_split_b(reqs.data(), n, 256, true) == 0, "%s", g_err);
+              size_t total = 0;
+              int64_t tw = LDM_WRAP_LC * 8;
+              for (Req& Q : reqs) {
+                CHECK(layout_request(Q, total) == 0, "%s", g_err);
+                tw += ((int64_t)Q.tn1 + Q.tn2 + 1024 + (Q.tL + 1023) / 1024) * 8 + 3 * 256;
+              }
+              CHECK((int64_t)total + tw <= sum, "nv %lld, %d rows, %d requests: %lld B of %lld", (long long)nv, m_cap, n,
+                    (long long)total + tw, (long long)sum);
+            }
+        }
+  CHECK(halves > 100 && wholes > 100, "%d half, %d whole", halves, wholes);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"bytes", bytes}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

@@ -132,3 +132,52 @@ def test_batch_after_a_layout_that_did_not_fit(dev):
     assert oracle.rel_peak_error(b.results(b.run())[0], ref) <= TOL
     b.close()
     db.close()
+
+
+@pytest.mark.parametrize("nv", [4_000, 9_000, 20_001, 50_001, 150_001])
+def test_noalloc_with_several_pass_b_shares(dev, nv):
+    """The scratch array's lone requests split a whole-length transform's pairs
+    over up to four pass B workgroups per row block."""
+    import torch
+
+    ws, wmin, T, p, x = 0.002, 2000.0, 900.0, 1.3, 0.3
+    wmax = wmin + (nv - 1.5) * ws
+    lines = _lines(3000, wmin, wmax, nv)
+    db = engine.LineDatabase(dev, lines)
+    for dx in (0.1, 0.2):
+        for opt, tol in (("simple", TOL), ("min-RMS", 1e-4)):
+            out = torch.full((nv,), float("nan"), dtype=torch.float32, device="cuda")
+            res = torch.zeros(48, dtype=torch.uint8, device="cuda")
+            req = engine.make_request(db, wmin, wmax, ws, T, p, x, dxG=dx, dxL=dx, optimization=opt)
+            inf = engine.run_noalloc(db, req, out, res)
+            assert engine.read_result(res).status == 0
+            ref = oracle.eq_abscoeff(lines.as_dict(), wmin, wmax, ws, T, p, x, dx, dx, optimization=opt)
+            err = oracle.rel_peak_error(np.ldexp(out.double().cpu().numpy(), inf.scale_log2), ref)
+            print(f"N_v={nv} L={inf.fft_len} {inf.n1}x{inf.n2} rows={inf.m_cap} {opt}: {err:.2e}", flush=True)
+            assert err <= tol
+    db.close()
+
+
+@pytest.mark.parametrize("nv", [4_000, 9_000, 20_001, 50_001, 150_001])
+def test_partial_spectra_in_y(dev, nv):
+    """A batch's lone whole-length request keeps pass B's partial spectra in Y:
+    as many pairs as planned, and so few (after set_request) that shares have
+    none."""
+    ws, wmin, T, p, x = 0.002, 2000.0, 900.0, 1.3, 0.3
+    wmax = wmin + (nv - 1.5) * ws
+    lines = _lines(3000, wmin, wmax, nv)
+    db = engine.LineDatabase(dev, lines)
+    mk = lambda dx: engine.make_request(db, wmin, wmax, ws, T, p, x, dxG=dx, dxL=dx, period_fft_len=True)  # noqa: E731
+    b = engine.SpectrumBatch(db, [mk(0.1)])
+    assert b.workspace_bytes() <= db.request_bytes(mk(0.1))[0]
+    for dx in (0.1, 3.0, 1.0, 0.5, 0.3, 0.2, 0.1):
+        b.set_request(0, mk(dx))
+        for k in range(2):
+            got = b.results(b.run())[0]
+            inf = b.info(0)
+            ref = oracle.eq_abscoeff(lines.as_dict(), wmin, wmax, ws, T, p, x, dx, dx, L=int(inf.fft_len))
+            err = oracle.rel_peak_error(got, ref)
+            print(f"N_v={nv} dx={dx} M={inf.n_g}x{inf.n_l} of {inf.m_cap}: {err:.2e}", flush=True)
+            assert err <= TOL
+    b.close()
+    db.close()

@@ -31,3 +31,11 @@ def section(tmp_path_factory):
 
 def test_tile_too_wide_for_two_rows_is_refused(section):
     section("wide_tile")
+
+
+def test_admission_bytes(section):
+    section("bytes")
+
+
+def test_partial_spectra_in_y(section):
+    section("shares_in_y")
