@@ -41,8 +41,6 @@ namespace {
 // runs on holds its own copy until the process ends.  In host code the name
 // is a stand-in, not a device address: kernels get the address that
 // hipGetSymbolAddress returns for the current device (scratch_address).
-// (SCRATCH_TABLES bytes beyond the documented size: the axis tables' tile ranges.)
-#define SCRATCH_TABLES 4096
 static __device__ __align__(256) unsigned char scratch[RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES];
 
 namespace {
@@ -1220,45 +1218,29 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   const int n_items = plan_items(P) + P.n_img;
   rc = check_layout(R, work);
   if (rc) return rc;
-  // scratch layout
-  size_t off = 0;
-  auto take = [&](size_t n) {
-    const size_t o = off;
-    off = align_up(off + n, 256);
-    return o;
-  };
-  const size_t o_job = take(sizeof(LdmJob)), o_axes = take(sizeof(LdmAxes)), o_res = take(sizeof(LdmResult));
-  // (a half-length transform's items lie in the part of its workspace that it
-  // leaves unused)
-  const size_t items_bytes = (size_t)n_items * sizeof(int4);
-  const bool items_in_work = R.half && R.off_free + items_bytes <= R.off_y + (size_t)P.pcap * R.plan.L * 8;
-  const size_t o_items_ = items_in_work ? 0 : take(items_bytes);
-  const long long nhi = (R.tL + 1023) >> LDM_TW_LO_BITS;
-  const size_t o_tw1 = take((size_t)R.plan.n1 * 8), o_tw2 = take((size_t)R.plan.n2 * 8);
-  const size_t o_twl = take((size_t)(nhi + 1024) * 8);
-  const size_t o_twc = take((size_t)LDM_WRAP_LC * 8);
-  const size_t o_work = take(work);
-  if (off > (size_t)RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES)
+  NoallocLayout S;
+  noalloc_layout(R, P, n_items, work, S);
+  if (S.bytes > (size_t)RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES)
     return fail(RADIS_LDM_ERANGE, "request needs %zu bytes of scratch, above the %lld of radis_ldm_run_noalloc "
-                                  "(use a batch)", off, (long long)RADIS_LDM_NOALLOC_BYTES);
-  const size_t o_items = items_in_work ? o_work + R.off_free : o_items_;
+                                  "(use a batch)", S.bytes, (long long)RADIS_LDM_NOALLOC_BYTES);
+  const long long nhi = (R.tL + 1023) >> LDM_TW_LO_BITS;
   char* const base = ctx->scratch;
-  float2* tw1 = (float2*)(base + o_tw1);
-  float2* tw2 = (float2*)(base + o_tw2);
-  float2* twl = (float2*)(base + o_twl);
+  float2* tw1 = (float2*)(base + S.tw1);
+  float2* tw2 = (float2*)(base + S.tw2);
+  float2* twl = (float2*)(base + S.twl);
   R.tw1 = tw1;
   R.tw2 = tw2;
   R.twl_hi = twl;
   R.twl_lo = twl + nhi;
-  R.tw_wrap = (float2*)(base + o_twc);
+  R.tw_wrap = (float2*)(base + S.twc);
   LdmJob J;
-  fill_job(*db, R, base + o_work, out_dev, J);
+  fill_job(*db, R, base + S.work, out_dev, J);
   hipStream_t s = (hipStream_t)stream;
-  const LdmTwiddles wrap{(float2*)(base + o_twc), nullptr, nullptr, LDM_WRAP_LC, 0, 0};
+  const LdmTwiddles wrap{(float2*)(base + S.twc), nullptr, nullptr, LDM_WRAP_LC, 0, 0};
   const LdmTwiddles tw{tw1, tw2, twl, R.tn1, R.tn2, (long long)R.tL};
   const long long n_set = n_items + wrap.total() + tw.total();  // one element per thread: below 2^31 in the scratch array
-  hipLaunchKernelGGL(k_setup, dim3((unsigned)(1 + (n_set + 255) / 256)), dim3(256), 0, s, J, (LdmJob*)(base + o_job), P,
-                     (int4*)(base + o_items), n_items, wrap, tw);
+  hipLaunchKernelGGL(k_setup, dim3((unsigned)(1 + (n_set + 255) / 256)), dim3(256), 0, s, J, (LdmJob*)(base + S.job), P,
+                     (int4*)(base + S.items), n_items, wrap, tw);
   HIPCHK(hipGetLastError());
   const int cls_a = R.plan.fc ? R.tn1 | (R.narrow_a ? FC_NARROW : 0) : 0;
   const int cls_c = (R.plan.fc ? R.tn1 | (R.narrow_c ? FC_NARROW : 0) : 0) | (R.n_share > 1 ? FC_C_SUM : 0);
@@ -1267,10 +1249,10 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
       gb{cls_b, 0, P.n_rowB, std::min(R.m_cap, FC_B_ROWS_LDS), R.half ? 0 : R.wrap_rows, 0, P.n_img},
       gc{cls_c, 0, P.n_colC, 0, 0, 0, 0};
   LaunchSet X{};
-  X.jobs = (LdmJob*)(base + o_job);
-  X.axes = (LdmAxes*)(base + o_axes);
-  X.res = result_dev ? (LdmResult*)result_dev : (LdmResult*)(base + o_res);
-  X.items = (int4*)(base + o_items);
+  X.jobs = (LdmJob*)(base + S.job);
+  X.axes = (LdmAxes*)(base + S.axes);
+  X.res = result_dev ? (LdmResult*)result_dev : (LdmResult*)(base + S.res);
+  X.items = (int4*)(base + S.items);
   X.n_req = 1;
   X.n_axis = P.n_lo + P.n_g + P.n_hi;
   X.n_wrap = P.n_wrap;

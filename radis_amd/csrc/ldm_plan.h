@@ -1189,4 +1189,39 @@ int plan_one(const radis_ldm_db& db, const radis_ldm_request& rq, Req& R) {
   return bound_request(db, R);
 }
 
+// The no-allocation entry point's scratch array: where each table and the
+// workspace of `work` bytes lie, and how many bytes they take.  The array is
+// SCRATCH_TABLES bytes larger than documented, for what the splits of lone
+// requests add to the tables: narrow fill tiles, pass A blocks and several pass B
+// shares (at most a few items per CU each, 16 B), a width item per candidate block
+// (LDM_SKY_WGS of them) and the tile ranges of the axes: up to 19 KB counted over
+// 10^6 plans.
+#define SCRATCH_TABLES (64 << 10)
+struct NoallocLayout {
+  size_t job, axes, res, items, tw1, tw2, twl, twc, work, bytes;
+};
+void noalloc_layout(const Req& R, const LdmItemPlan& P, int n_items, size_t work, NoallocLayout& S) {
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    const size_t o = off;
+    off = align_up(off + n, 256);
+    return o;
+  };
+  S.job = take(sizeof(LdmJob));
+  S.axes = take(sizeof(LdmAxes));
+  S.res = take(sizeof(LdmResult));
+  // (a half-length transform's items lie in the part of its workspace that it
+  // leaves unused)
+  const size_t items_bytes = (size_t)n_items * sizeof(int4);
+  const bool items_in_work = R.half && R.off_free + items_bytes <= R.off_y + (size_t)P.pcap * R.plan.L * 8;
+  S.items = items_in_work ? 0 : take(items_bytes);
+  S.tw1 = take((size_t)R.plan.n1 * 8);
+  S.tw2 = take((size_t)R.plan.n2 * 8);
+  S.twl = take((size_t)(((R.tL + 1023) >> LDM_TW_LO_BITS) + 1024) * 8);
+  S.twc = take((size_t)LDM_WRAP_LC * 8);
+  S.work = take(work);
+  if (items_in_work) S.items = S.work + R.off_free;
+  S.bytes = off;
+}
+
 }  // namespace

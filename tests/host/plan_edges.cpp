@@ -3,6 +3,8 @@
 //               the planning itself, alone and beside requests that plan
 //   shares_in_y pass B's partial spectra in Y: no share's overlaps what another
 //               reads or writes
+//   scratch     the no-allocation entry point's array holds what it held with
+//               the plain splits' tables
 //   bytes       the admission figure: at most one transform's buffers and a
 //               second partial spectrum, and no less than what batches of such
 //               requests lay out
@@ -148,10 +150,80 @@ void bytes() {
   CHECK(halves > 100 && wholes > 100, "%d half, %d whole", halves, wholes);
 }
 
+// Bytes of scratch with the tables of the plain splits: full-width fill tiles and
+// column blocks, one pass B share (two where it is split), width candidates in
+// groups of eight blocks or more, axes without tile ranges.
+size_t plain_scratch(const radis_ldm_db& db, const Req& R, const LdmItemPlan& P) {
+  size_t t = 0;
+  auto put = [&](size_t n) { t = align_up(t + n, 256); };
+  const size_t pcap = (R.m_cap + 1) / 2, L = R.plan.L;
+  put(1024);
+  put(sizeof(LdmAxes) - sizeof(LdmAxes::pair) - 2 * sizeof(LdmAxes::tlo));
+  put(sizeof(LdmResult));
+  const int64_t blocks = P.n_g ? P.fb1 - P.g0 : 0, G = std::max<int64_t>(8, (blocks + 599) / 600);
+  size_t items = P.n_lo + (blocks + G - 1) / G + P.n_hi + (R.wrap_rows + 1) / 2 + (size_t)R.wide_tiles * R.fill_groups;
+  const bool two = R.plan.fc && pcap >= 4 && 2 * (R.plan.n1 / fc_rows_b(R.plan.n2)) <= 1024;
+  if (R.plan.fc)
+    items += pcap * (R.plan.n2 / fc_cols_a(R.plan.n1)) + (two ? 2 : 1) * (R.plan.n1 / fc_rows_b(R.plan.n2)) + R.plan.n2 / fc_cols_c(R.plan.n1);
+  else
+    items += pcap * P.n_colA + P.n_rowB + P.n_colC;
+  put(items * 16);
+  put(R.plan.n1 * 8);
+  put(R.plan.n2 * 8);
+  put((size_t)(((L + 1023) >> LDM_TW_LO_BITS) + 1024) * 8);
+  put(LDM_WRAP_LC * 8);
+  size_t work = 0;
+  auto buf = [&](size_t n) { work = align_up(work + n, 256); };
+  buf(pcap * 2 * align_up(R.nv + 1, 64) * 4);
+  buf(pcap * L * 8);
+  buf(L * 8);
+  if (two) buf(L * 8);
+  buf((size_t)R.m_cap * 16);
+  buf((size_t)((R.i1 - R.i0 + LDM_AX_CHUNK - 1) / LDM_AX_CHUNK + 2) * 32);
+  buf((size_t)R.wrap_rows * R.plan.wrap_k * 4);
+  put(work);
+  return t;
+}
+
+void scratch() {
+  int at_limit = 0;
+  auto check = [&](int64_t n, int64_t nv, int m_cap, int tile, int flags) {
+    radis_ldm_db db;
+    db.n = n;
+    db.has_sky = n >= LDM_SKY_BLOCK;
+    Req R = request(nv, m_cap, tile, flags);
+    R.i0 = 1;
+    R.i1 = n;
+    if (flags & (RADIS_LDM_GENERIC_FFT | RADIS_LDM_PERIOD_L))
+      CHECK(plan_fft(nv, 0, R.plan, 0, !(flags & RADIS_LDM_GENERIC_FFT), (flags & RADIS_LDM_PERIOD_L) != 0) == 0, "%s", g_err);
+    CHECK(choose_split_b(&R, 1, 256) == 0, "%s", g_err);
+    size_t work = 0;
+    CHECK(layout_request(R, work) == 0 && check_layout(R, work) == 0, "%s", g_err);
+    const LdmItemPlan P = item_plan(db, R);
+    NoallocLayout S;
+    noalloc_layout(R, P, plan_items(P) + P.n_img, work, S);
+    const size_t before = plain_scratch(db, R, P), limit = (size_t)RADIS_LDM_NOALLOC_BYTES;
+    // what fits with the plain splits fits the array
+    if (before <= limit) CHECK(S.bytes <= limit + SCRATCH_TABLES, "%lld lines, nv %lld, %d rows: %zu, plain %zu", (long long)n, (long long)nv, m_cap, S.bytes, before);
+    if (before > limit / 2) CHECK(S.bytes <= before + SCRATCH_TABLES, "%lld lines, nv %lld, %d rows: %zu, plain %zu", (long long)n, (long long)nv, m_cap, S.bytes, before);
+    at_limit += before > limit / 2 && before < 2 * limit;
+    // and the tables and the workspace do not overlap
+    CHECK(S.work + work <= S.bytes && S.twc + (size_t)LDM_WRAP_LC * 8 <= S.work && S.twl < S.twc &&
+              (S.items < S.tw1 || (S.items >= S.work + R.off_free && S.items + 16 * (size_t)(plan_items(P) + P.n_img) <= S.work + work)), "scratch layout");
+  };
+  check(2000000, 521910, 40, 32, RADIS_LDM_PERIOD_L);  // within 2 KB of the limit
+  for (int64_t n : {1000, 300000, 4100000, 100000000})
+    for (int64_t nv = 3000; nv < 5000000; nv = nv * 11 / 10 + 1)
+      for (int m_cap = 1; m_cap < 9000; m_cap = m_cap * 5 / 4 + 1)
+        for (int flags : {0, RADIS_LDM_MIN_RMS, RADIS_LDM_GENERIC_FFT, RADIS_LDM_PERIOD_L})
+          if ((size_t)((m_cap + 1) / 2) * nv * 24 < (2u << 30)) check(n, nv, m_cap, 0, flags);
+  CHECK(at_limit > 100, "%d near the limit", at_limit);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"bytes", bytes}, {"shares_in_y", shares_in_y}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

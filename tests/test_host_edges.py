@@ -39,3 +39,7 @@ def test_admission_bytes(section):
 
 def test_partial_spectra_in_y(section):
     section("shares_in_y")
+
+
+def test_scratch_array_holds_every_split(section):
+    section("scratch")
