@@ -27,10 +27,15 @@
 constexpr int ldm_fill_pad(int tile_w) { return tile_w >= 64 ? 3 : 2; }
 #define LDM_AX_CHUNK 4096  // lines per axis-reduction workgroup (16 per lane)
 #define LDM_SKY_BLOCK 4096  // lines per width-candidate block
-// most candidate workgroups of k_axis per request (about): one block each up to
-// there (a block's candidates, a few dozen to a few hundred, are one pass of
-// the workgroup's threads; groups of 8 left a 300,000-line window to 9 workgroups)
+// candidate workgroups of a k_axis launch (about) up to which each takes one
+// block (a block's candidates, a few dozen to a few hundred, are one pass of the
+// workgroup's threads; groups of 8 left a 300,000-line window to 9 workgroups),
+// and the most per request.  Launches of more take up to LDM_SKY_GROUP blocks
+// per workgroup: windows of a 5 M-line list, one block each -> groups of 8: 16
+// windows 18.9 -> 11.4 us, 64 41.6 -> 16.2, 256 (43,000 blocks) 143 -> 43 us
+// (groups of 4, 16, 32: 58, 39, 42 us).
 #define LDM_SKY_WGS 1024
+#define LDM_SKY_GROUP 8
 static_assert(LDM_AX_CHUNK == LDM_SKY_BLOCK, "a partial block is one scan chunk");
 #define LDM_TW_LO_BITS 10  // four-step twiddle split W_L^e = hi[e>>10] * lo[e&1023]
 #define LDM_NFOLD_MAX 100000

@@ -145,6 +145,7 @@ struct Req {
   int n_share = 1;     // workgroups per pass B row block, each taking a share of the pairs
   bool share_in_y = false;  // the shares' partial spectra lie in Y (LdmJob::share_at)
   int n_axp = 0;       // axis partials (items of k_axis)
+  int sky_group = 1;   // candidate blocks per k_axis workgroup that the launch calls for
   bool sky_whole = false;  // width extremes from the whole list's Pareto sets in k_finalize (no k_axis items)
   size_t off_ldm = 0, off_y = 0, off_b = 0, off_b2 = 0, off_rows = 0, off_axp = 0, off_wrap = 0;
   size_t off_share = 0, off_img = 0, off_mom = 0, off_free = 0;  // partial spectra; half: correction values, tile moments, unused from here
@@ -929,6 +930,12 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   int shrink = 0;
   while (tiles << shrink < (long long)FILL_TILES_PER_CU * n_cu && shrink < 8) ++shrink;
   for (int i = 0; i < n; ++i) reqs[i].tile_shrink = shrink;
+  // (blocks of whole-list windows counted too: they have no axis items, but
+  // the group only goes up to LDM_SKY_GROUP)
+  long long sky = 0;
+  for (int i = 0; i < n; ++i) sky += (reqs[i].i1 - reqs[i].i0) / LDM_SKY_BLOCK;
+  for (int i = 0; i < n; ++i)
+    reqs[i].sky_group = (int)std::max(1ll, std::min<long long>(LDM_SKY_GROUP, (sky + LDM_SKY_WGS - 1) / LDM_SKY_WGS));
   // Half-length transforms pay where the launch's passes are more than a chain
   // of latencies: below HALF_MIN_POINTS (pairs times planned length) the
   // shorter passes take as long as the whole ones and the correction is extra.
@@ -1137,7 +1144,7 @@ LdmItemPlan item_plan(const radis_ldm_db& db, Req& R) {
     P.lo_e = fb0 * LDM_SKY_BLOCK;
     P.n_lo = chunks(P.lo_a, P.lo_e);
     // at most about LDM_SKY_WGS workgroups (each partial costs the reduction a read)
-    P.G = (fb1 - fb0 + LDM_SKY_WGS - 1) / LDM_SKY_WGS;
+    P.G = std::max<int64_t>(R.sky_group, (fb1 - fb0 + LDM_SKY_WGS - 1) / LDM_SKY_WGS);
     P.g0 = fb0;
     P.fb1 = fb1;
     P.n_g = (int)((fb1 - fb0 + P.G - 1) / P.G);

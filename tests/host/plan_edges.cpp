@@ -3,6 +3,7 @@
 //               the planning itself, alone and beside requests that plan
 //   shares_in_y pass B's partial spectra in Y: no share's overlaps what another
 //               reads or writes
+//   axis_groups width candidate blocks per workgroup from the whole launch's
 //   scratch     the no-allocation entry point's array holds what it held with
 //               the plain splits' tables
 //   bytes       the admission figure: at most one transform's buffers and a
@@ -87,6 +88,39 @@ void shares_in_y() {
       }
     }
   CHECK(split > 300, "%d split", split);
+}
+
+// Axis items: a block each where a launch has few, in groups of up to
+// LDM_SKY_GROUP where it has many, whatever number of requests they belong to.
+void axis_groups() {
+  for (int64_t n : {300000, 5000000, 100000000})
+    for (int count : {1, 4, 32, 256}) {
+      radis_ldm_db db;
+      db.n = n;
+      db.has_sky = true;
+      std::vector<Req> reqs;
+      int64_t blocks = 0;
+      for (int i = 0; i < count; ++i) {
+        Req R = request(20001, 16);
+        R.i0 = 1 + n / 40 * (i % 13);
+        R.i1 = n - 1 - n / 50 * (i % 17);
+        blocks += R.i1 / LDM_SKY_BLOCK - (R.i0 + LDM_SKY_BLOCK - 1) / LDM_SKY_BLOCK;
+        reqs.push_back(R);
+      }
+      CHECK(choose_split_b(reqs.data(), count, 256, true) == 0, "%s", g_err);
+      int64_t items = 0;
+      size_t total = 0;
+      for (Req& R : reqs) {
+        CHECK(layout_request(R, total) == 0, "%s", g_err);
+        const LdmItemPlan P = item_plan(db, R);
+        CHECK(P.n_g <= LDM_SKY_WGS && (int64_t)P.n_g * P.G >= P.fb1 - P.g0 && (int64_t)(P.n_g - 1) * P.G < P.fb1 - P.g0, "groups cover the window");
+        items += P.n_g;
+      }
+      // (each request's last group may be short)
+      CHECK(items <= LDM_SKY_WGS + blocks / LDM_SKY_GROUP + count, "%d windows of %lld lines: %lld items for %lld blocks", count,
+            (long long)n, (long long)items, (long long)blocks);
+      if (blocks <= LDM_SKY_WGS) CHECK(items == blocks, "a block each: %lld of %lld", (long long)items, (long long)blocks);
+    }
 }
 
 // LDM, Y, a partial spectrum (two where pass B is split over two shares: four
@@ -223,7 +257,7 @@ void scratch() {
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

@@ -43,3 +43,7 @@ def test_partial_spectra_in_y(section):
 
 def test_scratch_array_holds_every_split(section):
     section("scratch")
+
+
+def test_axis_groups_from_the_launch(section):
+    section("axis_groups")
