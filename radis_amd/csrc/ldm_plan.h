@@ -35,6 +35,8 @@ const double ATM_PER_BAR = 1.01325;          // lbl/broadening.py:1063
 const int STAT_BLOCK = 4096;             // lines per host-side statistics block
 const int FILL_LDS_TARGET = 44 * 1024;   // preferred LDS bytes of one fill tile (FP64 cells; 3 tiles per CU)
 const int FILL_LDS_MAX = 60 * 1024;      // hard limit (plus ~2.2 KB of static axis tables, < 64 KB)
+const int FILL_LDS_STATIC = 2304;       // its static axis tables
+const int LDS_PER_CU = 160 * 1024;
 const int MIN_TILE_W = 16, MAX_TILE_W = 4096;
 const int FILL_NARROW_W = 64;          // least width a tile is halved to for launches of few
 const int FILL_GROUP_TILE_W = 32;      // tile width of fills in row groups
@@ -140,6 +142,7 @@ struct Req {
   int64_t tL = 0;
   int tn1 = 0, tn2 = 0, bX[3] = {0, 0, 0};
   int cell_tiles = 0, n_cell = 0;  // half: fill tiles per cell of the image correction, cells
+  double half_loss = 0;  // half: what the launch loses by it (half_loss_ns)
   double wg_hi = 0;    // bound of the Gaussian FWHM (cm-1)
   int split_b = 1;     // 2: pass B's pairs are split over several workgroups per row block
   int n_share = 1;     // workgroups per pass B row block, each taking a share of the pairs
@@ -828,6 +831,32 @@ bool half_ok(const Req& R, int tile_w) {
 // k_finalize +0.6; 47 M, N_G = 12: -57 us of 534).
 constexpr long long SPARSE_G_POINTS = 1 << 22;
 
+// Image items of a request with n_cell cells: (cell, part of the nodes).
+int image_parts(int n_cell) { return std::max(1, (n_cell * IMG_NODES + IMG_TARGETS - 1) / IMG_TARGETS); }
+int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
+
+// What a half-length request costs a launch that fills the chip beyond the whole
+// length with tiles of `whole_w` points, in nanoseconds (negative: it gains).  The
+// passes save 2.4 per 1000 points of Y.  The image items take 8.4 + 0.45 N_L each,
+// and their number goes with the square of N_v / gap; tiles narrowed for the gap
+// 2.9 each; the moments 0.7 per 1000 LDM cells, and 2.4 per 1000 lines where
+// their LDS leaves two fill workgroups a CU instead of three.  Fitted to 333
+// launches (8,300 to 500,001 points, 12 to 294 rows, 1 to 200 requests), which
+// took half / whole us: 200 x 12,000 points (8 cells) 342 / 397; 200 x 15,541 (47
+// cells, 16-point tiles) 1228 / 417; 64 x 17,000 (13 cells) 224 / 231; 64 x 46,900
+// (53 cells) 634 / 471; 16 x 63,800 (95 cells) 344 / 187; 345 rows x 600,001 points
+// 1441 / 1755 with 50 M lines, 2821 / 2773 with 200 M.
+double half_loss_ns(const Req& R, int whole_w) {
+  const double V = (double)R.nv + 1, pairs = (R.m_cap + 1) / 2, nl = std::min(R.m_cap / 2, LDM_MAX_AX);
+  const size_t tile = fill_tile_bytes(R.m_cap, R.tile_w) + FILL_LDS_STATIC;
+  const size_t with = tile + (size_t)tile_moment_lds(R.m_cap, R.tile_w);
+  const double tiles = R.n_tiles - std::ceil(V / whole_w);
+  double t = -2.4e-3 * pairs * (double)R.plan.L + (8.4 + 0.45 * nl) * image_items(R.n_cell) + 2.9 * std::max(0.0, tiles) +
+             0.7e-3 * R.m_cap * V;
+  if (LDS_PER_CU / tile >= 3 && LDS_PER_CU / with < 3) t += 2.4e-3 * (double)(R.i1 - R.i0);
+  return t;
+}
+
 // Tile width, row groups and the transform a request runs (Req::half, tL,
 // tn1, tn2), from its plan, its row capacity and its conditions.
 int plan_exec(Req& R) {
@@ -860,6 +889,8 @@ int plan_exec(Req& R) {
   R.tn1 = R.plan.n1;
   R.tn2 = R.plan.n2;
   R.cell_tiles = R.n_cell = 0;
+  R.half_loss = 0;
+  const int whole_w = R.tile_w;
   const bool halves = R.plan.n1 >= 512 || R.plan.n2 >= 128;
   if (R.may_half && R.plan.fc && R.plan.wrap_k > 0 && R.fill_groups == 1 && halves) {
     int w = R.tile_w;
@@ -879,6 +910,7 @@ int plan_exec(Req& R) {
     }
   }
   R.n_tiles = (int)((V + R.tile_w - 1) / R.tile_w);
+  if (R.half) R.half_loss = half_loss_ns(R, whole_w);
   R.sparse_g = (long long)((R.m_cap + 1) / 2) * R.tL >= SPARSE_G_POINTS;
   if (R.plan.fc) {
     R.bX[0] = floor_log2(R.narrow_a ? FC_COLS_A_NARROW : fc_cols_a(R.tn1));
@@ -891,10 +923,6 @@ int plan_exec(Req& R) {
   }
   return 0;
 }
-
-// Image items of a request with n_cell cells: (cell, part of the nodes).
-int image_parts(int n_cell) { return std::max(1, (n_cell * IMG_NODES + IMG_TARGETS - 1) / IMG_TARGETS); }
-int image_items(int n_cell) { return n_cell * image_parts(n_cell); }
 
 // Workgroups per pass B row block (Req::n_share) for requests reqs[0..n)
 // that run together.  A compiled pass B workgroup walks every pair of its
@@ -911,7 +939,7 @@ constexpr int FC_B_SPLIT_MIN_PAIRS = 2;
 // lean: up to which its workspace may grow by more than the one further partial
 // spectrum)
 constexpr int64_t FC_B_SPLIT_WHOLE_Y = 64 << 20;
-constexpr double HALF_MIN_POINTS = 1 << 19;
+constexpr double HALF_MIN_POINTS = 1 << 19, HALF_LOSS_NS = 6000, HALF_N1_NS = 20000, HALF_N2_NS = 8000;
 // wide column blocks below which the narrow ones run: a CU each (n1 = 256), or
 // half of that (384, 512: 768-thread tiles of three passes; between 128 and 256
 // wide blocks of 384 they took 14.5 -> 17.9 us); pass C: a CU each, or a fourth (the batch's 320 class
@@ -942,12 +970,39 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   double points = 0;
   for (int i = 0; i < n; ++i) points += (double)((reqs[i].m_cap + 1) / 2) * (double)reqs[i].plan.L;
   for (int i = 0; i < n; ++i) reqs[i].may_half = points >= HALF_MIN_POINTS;
+  // ... and where it costs the launch less than it saves: for every request that
+  // can (0), for those that gain by themselves (1), or for none (2).  Mixing the
+  // two lengths adds sizes of compiled passes, each a launch of pass B, or of
+  // passes A and C, that ends in a tail of its own: 32 windows of a 2 M-line list
+  // took 449 us all half, 470 with 21 half (five n1 instead of three), 517 whole;
+  // 256 windows of a 5 M-line list 3288, 3072 and 3530 (fill and passes).  The
+  // first form is preferred by HALF_LOSS_NS: a launch that leaves the chip idle
+  // hides as much (a lone 19,500 points x 84 rows: 5 us more by the sum, 72 us
+  // half, 80 whole).
+  double t[3] = {-HALF_LOSS_NS, 0, 0};
+  unsigned n1s[3] = {0, 0, 0}, n2s[3] = {0, 0, 0};
+  for (int i = 0; i < n; ++i) {
+    Req& R = reqs[i];
+    // a request that cannot be laid out has nothing to count
+    const int rc = plan_exec(R);
+    if (rc) return rc;
+    if (!R.plan.fc) continue;
+    for (int k = 0; k < 3; ++k) {
+      const bool half = R.half && (k == 0 || (k == 1 && R.half_loss <= 0));
+      if (half) t[k] += R.half_loss;
+      n1s[k] |= 1u << ((half ? R.tn1 : R.plan.n1) >> 6);
+      n2s[k] |= 1u << floor_log2(half ? R.tn2 : R.plan.n2);
+    }
+  }
+  for (int k = 0; k < 3; ++k) t[k] += HALF_N1_NS * __builtin_popcount(n1s[k]) + HALF_N2_NS * __builtin_popcount(n2s[k]);
+  const int form = t[0] <= t[1] && t[0] <= t[2] ? 0 : t[1] <= t[2] ? 1 : 2;
+  for (int i = 0; i < n; ++i)
+    reqs[i].may_half = reqs[i].may_half && (form == 0 || (form == 1 && reqs[i].half_loss <= 0));
   std::map<int, long long> cols_a, cols_c;  // compiled n1 -> wide column blocks of passes A and C
   std::map<int, long long> blocks, images;  // compiled pass B class (N2) -> row blocks, image items of the launch
   for (int i = 0; i < n; ++i) {
     Req& R = reqs[i];
     R.narrow_a = R.narrow_c = false;
-    // a request that cannot be laid out has no split to count
     const int rc = plan_exec(R);
     if (rc) return rc;
     if (!R.plan.fc) continue;

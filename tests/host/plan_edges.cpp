@@ -4,6 +4,7 @@
 //   shares_in_y pass B's partial spectra in Y: no share's overlaps what another
 //               reads or writes
 //   axis_groups width candidate blocks per workgroup from the whole launch's
+//   half_cost   half-length transforms where they cost the launch less
 //   scratch     the no-allocation entry point's array holds what it held with
 //               the plain splits' tables
 //   bytes       the admission figure: at most one transform's buffers and a
@@ -121,6 +122,41 @@ void axis_groups() {
             (long long)n, (long long)items, (long long)blocks);
       if (blocks <= LDM_SKY_WGS) CHECK(items == blocks, "a block each: %lld of %lld", (long long)items, (long long)blocks);
     }
+}
+
+// Which launches run at half length: measured ones (times on both sides are at
+// half_loss_ns).
+void half_cost() {
+  const struct { int count; int64_t nv; int m_cap; int64_t lines; bool half; } cases[] = {
+      {200, 12000, 18, 48000, true},    {200, 15541, 18, 62000, false}, {64, 15541, 38, 62000, false},
+      {64, 17000, 38, 68000, true},     {64, 46900, 18, 190000, false}, {16, 63800, 18, 250000, false},
+      {4, 63800, 12, 250000, false},    {16, 40001, 38, 160000, true},  {64, 120417, 18, 480000, true},
+      {1, 200001, 12, 5000, true},      {1, 500001, 27, 5000000, true}, {1, 19500, 84, 78000, true},
+      {1, 600001, 144, 100000000, true}, {1, 600001, 345, 50000000, true}, {1, 600001, 345, 200000000, false}};
+  for (const auto& c : cases) {
+    std::vector<Req> reqs(c.count, request(c.nv, c.m_cap));
+    for (Req& R : reqs) R.i1 = c.lines;
+    CHECK(choose_split_b(reqs.data(), c.count, 256, true) == 0, "%s", g_err);
+    for (const Req& R : reqs) CHECK(R.half == c.half, "%d x %lld points, %d rows", c.count, (long long)c.nv, c.m_cap);
+  }
+  // many windows of random sizes mix both lengths, a few keep one
+  for (int count : {32, 256}) {
+    std::vector<Req> reqs;
+    int halves = 0, can = 0;
+    for (int i = 0; i < count; ++i) {
+      reqs.push_back(request(14000 + 86000 * (int64_t)(i * 37 % 256) / 256, 14 + i % 8));
+      Req R = reqs.back();
+      R.may_half = true;
+      CHECK(plan_exec(R) == 0, "%s", g_err);
+      can += R.half;
+    }
+    CHECK(choose_split_b(reqs.data(), count, 256, true) == 0, "%s", g_err);
+    for (const Req& R : reqs) {
+      halves += R.half;
+      if (count == 256) CHECK(!R.half || R.half_loss <= 0, "a request that costs more than it saves");
+    }
+    CHECK(count == 32 ? halves == can : halves > count / 3 && halves < can, "%d of %d half, %d can", halves, count, can);
+  }
 }
 
 // LDM, Y, a partial spectrum (two where pass B is split over two shares: four
@@ -257,7 +293,7 @@ void scratch() {
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"half_cost", half_cost}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

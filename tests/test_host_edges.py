@@ -47,3 +47,7 @@ def test_scratch_array_holds_every_split(section):
 
 def test_axis_groups_from_the_launch(section):
     section("axis_groups")
+
+
+def test_half_length_by_its_cost(section):
+    section("half_cost")
