@@ -1025,8 +1025,14 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
     // array their partial spectra have buffers of their own; batches are lean,
     // with the spectra in Y: requests are admitted by request_bytes, and three
     // further spectra were up to a fifth of a small request's workspace.
-    const long long room = std::max<long long>(0, (long long)FC_B_SPLIT_WGS_PER_CU * n_cu - images[R.tn2]);
-    int ns = (int)std::min<long long>(room / blocks[R.tn2], pairs / FC_B_SPLIT_MIN_PAIRS);
+    // image items take places first; they are short, so where they would leave
+    // no room for a second share only a workgroup per CU of them counts (4 x 46,900
+    // points x 84 rows, 848 items: one share 83.7 us, four 49.0; 255,001 points,
+    // 546 items, room for three: 19.6, four 22.4)
+    const long long places = (long long)FC_B_SPLIT_WGS_PER_CU * n_cu;
+    long long room = std::max(0ll, places - images[R.tn2]) / blocks[R.tn2];
+    if (room < 2) room = (places - std::min<long long>(images[R.tn2], n_cu)) / blocks[R.tn2];
+    int ns = (int)std::min<long long>(room, pairs / FC_B_SPLIT_MIN_PAIRS);
     const bool room_whole = (int64_t)pairs * R.plan.L * 8 <= FC_B_SPLIT_WHOLE_Y;
     ns = std::min(ns, R.half || room_whole ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);
     if (R.half && ns > 2) ns = std::min(ns, pairs - 1 - pairs / 8);  // they share Y's unused half with the moments

@@ -5,6 +5,7 @@
 //               reads or writes
 //   axis_groups width candidate blocks per workgroup from the whole launch's
 //   half_cost   half-length transforms where they cost the launch less
+//   image_room  pass B's shares beside many image items
 //   scratch     the no-allocation entry point's array holds what it held with
 //               the plain splits' tables
 //   bytes       the admission figure: at most one transform's buffers and a
@@ -159,6 +160,16 @@ void half_cost() {
   }
 }
 
+// Pass B's shares beside many image items: the rows' pairs are still split.
+void image_room() {
+  for (int m_cap : {38, 84}) {
+    std::vector<Req> reqs(4, request(46900, m_cap));
+    for (Req& R : reqs) R.i1 = 190000;
+    CHECK(choose_split_b(reqs.data(), 4, 256, true) == 0, "%s", g_err);
+    for (const Req& R : reqs) CHECK(R.n_share >= 2, "%d rows, half %d: %d shares, %d image items", m_cap, (int)R.half, R.n_share, R.half ? image_items(R.n_cell) : 0);
+  }
+}
+
 // LDM, Y, a partial spectrum (two where pass B is split over two shares: four
 // pairs or more, and twice the row blocks fit four workgroups per CU), rows,
 // axis partials, correction table, fill items at the full tile width, tables.
@@ -293,7 +304,7 @@ void scratch() {
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"half_cost", half_cost}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"half_cost", half_cost}, {"image_room", image_room}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

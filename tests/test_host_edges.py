@@ -51,3 +51,7 @@ def test_axis_groups_from_the_launch(section):
 
 def test_half_length_by_its_cost(section):
     section("half_cost")
+
+
+def test_shares_beside_image_items(section):
+    section("image_room")
