@@ -1297,20 +1297,28 @@ int radis_ldm_slit_convolve(const float* in, int64_t n, const float* slit, int32
   const char *a0 = (const char*)in, *a1 = a0 + n * 4, *b0 = (const char*)out, *b1 = b0 + n * 4;
   const char *s0 = (const char*)slit, *s1 = s0 + (int64_t)k * 4;
   if ((a0 < b1 && b0 < a1) || (s0 < b1 && b0 < s1)) return fail(RADIS_LDM_EINVAL, "output overlaps the input or the slit");
-  // outputs per lane: the more the fewer LDS reads per product, but a workgroup
-  // for every CU comes first
-  const auto launch_slit = [&](auto tile, auto kernel) -> int {
-    using Tile = decltype(tile);
-    const int64_t grid = (n + Tile::OUT - 1) / Tile::OUT;
+  // Few taps on a long grid: the direct sum (SlitTile<8, 4> -> k_slit_short: 500,000
+  // points, 9 taps 3.9 -> 3.3 us; 2 M points, 9 taps 9.2 -> 5.3, 33 taps 11.1 -> 9.1; 8 M
+  // points, 51 taps 45.1, 44.7 with the tile).  Else the
+  // outputs per lane: the more the fewer LDS reads per product, but a workgroup for
+  // every CU comes first, and 16 pay from about 400 taps on (2 M points, 201
+  // taps: 26.6 us, with 8 22.0; 801 taps: 60.5, 64.4).
+  const auto launch_slit = [&](auto kernel, int threads, int64_t outputs) -> int {
+    const int64_t grid = (n + outputs - 1) / outputs;
     if (grid > INT32_MAX) return fail(RADIS_LDM_ERANGE, "grid too long");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(Tile::T), 0, (hipStream_t)stream, in, (long long)n, slit, k,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, in, (long long)n, slit, k,
                        scale, out);
     return 0;
   };
   int rc;
-  if (n >= 256 * SlitTile<16, 4>::OUT) rc = launch_slit(SlitTile<16, 4>{}, k_slit_conv<16, 4>);
-  else if (n >= 256 * SlitTile<8, 4>::OUT) rc = launch_slit(SlitTile<8, 4>{}, k_slit_conv<8, 4>);
-  else rc = launch_slit(SlitTile<4, 8>{}, k_slit_conv<4, 8>);
+  if (n >= 256 * SLIT_SHORT_OUT && k <= (n >= 1024 * SLIT_SHORT_OUT ? SLIT_SHORT : 12))
+    rc = launch_slit(k_slit_short, 256, SLIT_SHORT_OUT);
+  else if (n >= 256 * SlitTile<16, 4>::OUT && k >= 400)
+    rc = launch_slit(k_slit_conv<16, 4>, SlitTile<16, 4>::T, SlitTile<16, 4>::OUT);
+  else if (n >= 256 * SlitTile<8, 4>::OUT)
+    rc = launch_slit(k_slit_conv<8, 4>, SlitTile<8, 4>::T, SlitTile<8, 4>::OUT);
+  else
+    rc = launch_slit(k_slit_conv<4, 8>, SlitTile<4, 8>::T, SlitTile<4, 8>::OUT);
   if (rc) return rc;
   HIPCHK(hipGetLastError());
   return 0;

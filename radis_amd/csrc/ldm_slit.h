@@ -19,7 +19,7 @@
 // transposed in LDS (element e at row e % R, column e / R), so the lanes'
 // reads are consecutive; the taps are read as broadcasts.  The waves of a
 // workgroup take the same 64 R outputs and a share of the taps each, and add
-// their sums at the end.
+// their sums at the end.  (Few taps on a long grid: k_slit_short below.)
 #pragma once
 
 #define SLIT_KCH 2048  // slit taps per LDS chunk
@@ -107,5 +107,39 @@ __global__ __launch_bounds__(64 * NW) void k_slit_conv(const float* __restrict__
 #pragma unroll
     for (int w = 1; w < NW; ++w) s += p[w * R * 65];
     out[o0 + e] = (float)(s * scale);
+  }
+}
+
+// Slits of up to SLIT_SHORT taps on long grids: bound by the bytes, which the
+// tiles above pass through LDS twice more (the waves' sums).  A workgroup takes
+// SLIT_SHORT_OUT consecutive outputs, a lane one of each quarter: consecutive
+// inputs per read, the taps as broadcasts.  8 M points, 9 taps 35.1 (SlitTile<8, 4>)
+// -> 17.4 us (the copy alone is 14), 21 taps 40.9 -> 23.2, 33 taps 40.4 -> 28.1.
+#define SLIT_SHORT 48
+#define SLIT_SHORT_OUT 1024
+
+__global__ __launch_bounds__(256) void k_slit_short(const float* __restrict__ in, long long n,
+                                                    const float* __restrict__ slit, int k, double scale,
+                                                    float* __restrict__ out) {
+  __shared__ float s_x[SLIT_SHORT_OUT + SLIT_SHORT];
+  __shared__ double s_h[SLIT_SHORT];
+  const long long o0 = (long long)blockIdx.x * SLIT_SHORT_OUT;
+  const long long x0 = o0 + (k - 1) / 2 - (k - 1);  // in[] index of the first output's first input
+  if ((int)threadIdx.x < k) s_h[threadIdx.x] = (double)slit[k - 1 - threadIdx.x];
+  for (int e = threadIdx.x; e < SLIT_SHORT_OUT + k - 1; e += 256) {
+    const long long q = x0 + e;
+    s_x[e] = (q >= 0 && q < n) ? in[q] : 0.0f;
+  }
+  __syncthreads();
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int m = 0; m < k; ++m) {
+    const double h = s_h[m];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = __builtin_fma(h, (double)s_x[threadIdx.x + 256 * r + m], acc[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const long long o = o0 + threadIdx.x + 256 * r;
+    if (o < n) out[o] = (float)(acc[r] * scale);
   }
 }

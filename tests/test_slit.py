@@ -142,3 +142,37 @@ def test_gpu_slit_every_tile_is_the_exact_sum_rounded_once(n, k):
         hit = np.zeros(n, dtype=bool)
         hit[max(0, p - c):p - c + k] = True  # out[i] holds in[p] where 0 <= i + c - p < k
         assert not np.any(np.isfinite(g2[hit])) and np.array_equal(g2[~hit], got[~hit])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [262143, 262144, 1048575, 1048576, 1049601])
+@pytest.mark.parametrize("k", [1, 2, 11, 12, 13, 47, 48, 49, 399, 400])
+def test_gpu_slit_short_and_long_slits_on_long_grids(n, k):
+    """Either side of the rule for the direct sum and for the tile of 16
+    outputs: the exact sum rounded once (half an FP32 ulp is 6e-8; 1e-7
+    asserted), also beside a NaN and an infinity."""
+    import torch
+
+    rng = np.random.default_rng(n * 3 + k)
+    I = (10.0 ** rng.uniform(-10.0, 0.0, n)).astype(np.float32)
+    s = rng.random(k) + 0.1
+    x = torch.as_tensor(I, device="cuda")
+    got = slit.convolve_device(x, s, 0.25, mode="same").double().cpu().numpy()
+    c = (k - 1) // 2
+    ref = 0.25 * np.convolve(I.astype(np.float64), s.astype(np.float32).astype(np.float64))[c:c + n] if k <= 49 else None
+    if ref is not None:
+        assert np.max(np.abs(got - ref) / ref) <= 1e-7
+    else:
+        pad = np.concatenate([np.zeros(k), I.astype(np.float64), np.zeros(k)])
+        s32 = s.astype(np.float32).astype(np.float64)
+        for i in np.unique(np.concatenate([rng.integers(0, n, 300), np.arange(20), np.arange(n - 20, n)])):
+            want = 0.25 * np.dot(s32, pad[k + i + c - k + 1:k + i + c + 1][::-1])
+            assert abs(got[i] - want) <= 1e-7 * want, (i, got[i], want)
+    p = int(rng.integers(0, n))
+    for bad in (float("nan"), float("inf")):
+        y = x.clone()
+        y[p] = bad
+        g2 = slit.convolve_device(y, s, 0.25, mode="same").double().cpu().numpy()
+        hit = np.zeros(n, dtype=bool)
+        hit[max(0, p - c):p - c + k] = True
+        assert not np.any(np.isfinite(g2[hit])) and np.array_equal(g2[~hit], got[~hit])
