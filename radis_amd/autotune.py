@@ -2,16 +2,16 @@
 
 The FFT schedule is the split L = n1 * n2 together with the pass kernels:
 compile-time-sized passes (fixed radix plans, for n1 in 2^a*{1,3,5} and n2 in
-2^a) or run-time-sized ones (any 7-smooth split).  The fill kernel and the
-FFT passes are separate kernels, so the two choices are tuned one after the
-other on their own stage times: the tile width on the fill time with the
-planner's FFT, then the FFT schedule on the time of the three FFT passes with
-the chosen tile.  Each candidate's time is the median over a few timed runs
-(per-kernel HIP events).
+2^a) or run-time-sized ones (any 7-smooth split).  The two choices are tuned
+one after the other, the tile width with the planner's FFT, then the FFT
+schedule with the chosen tile, each on the time of every stage: the tile width
+decides with the FFT length whether the passes run at half of it, and the tile
+bounds are found in the axis launch.  Each candidate's time is the median over a
+few timed runs (per-kernel HIP events).
 
 Results are cached in a JSON file keyed by the planner's default FFT length
-and LDM row capacity (and the LDM steps), so requests of the same size class
-share one tuning: ``$RADIS_AMD_TUNE_CACHE`` or
+and LDM row capacity, the LDM steps, the LDM weights and SCHEDULES, so requests
+of the same size class share one tuning: ``$RADIS_AMD_TUNE_CACHE`` or
 ``~/.cache/radis_amd/autotune.json``.  ``engine.make_request`` applies a
 cached entry unless the caller fixes the schedule.
 """
@@ -54,7 +54,13 @@ def wrap_floor(need):
     return L
 
 
-FILL_STAGES = ("tile_bounds", "fill")
+# part of the cache keys: entries timed on kernels whose schedules mean something
+# else are not applied (2: half-length passes, tile bounds in the axis launch)
+SCHEDULES = 2
+# what the whole step's time varies by between runs (a split off the planner's for
+# less was up to 3 % slower when used)
+MARGIN = 0.03
+FILL_STAGES = ("fill",)
 FFT_STAGES = ("fft_a", "fft_b", "fft_c")
 
 
@@ -111,13 +117,18 @@ def _untuned(req):
 
 
 def _key_info(db, req):
+    from . import _native
+
     _, info = db.request_bytes(_untuned(req))
-    return f"L={int(info.fft_len)}/mcap={int(info.m_cap)}/dxG={req.dxG:.6g}/dxL={req.dxL:.6g}", info
+    weights = "min-RMS" if int(req.flags) & _native.MIN_RMS else "simple"
+    return (f"v{SCHEDULES}/L={int(info.fft_len)}/mcap={int(info.m_cap)}/dxG={req.dxG:.6g}/dxL={req.dxL:.6g}/"
+            f"{weights}"), info
 
 
 def key_of(db, req):
     """Size class of a request: the planner's FFT length and LDM row
-    capacity for it (no overrides), and the LDM steps."""
+    capacity for it (no overrides), the LDM steps and weights (min-RMS ones
+    never run at half length)."""
     return _key_info(db, req)[0]
 
 
@@ -205,9 +216,10 @@ def tile_candidates(m_cap):
     return [w for w in TILE_WIDTHS if m_cap * (w + fill_pad(w)) * 8 <= FILL_LDS_MAX]
 
 
-def _time(db, req, stages, reps):
-    """Median over ``reps`` timed runs of the summed ``stages`` (ms) and the
-    planned info, or (None, None) if the schedule does not plan."""
+def _time(db, req, reps):
+    """Median times (ms) over ``reps`` timed runs as (every stage, FILL_STAGES,
+    FFT_STAGES) and the planned info, or (None, None) if the schedule does not
+    plan."""
     import statistics
 
     from . import _native, engine
@@ -225,10 +237,20 @@ def _time(db, req, stages, reps):
         for _ in range(reps):
             b.run(outs)
             st = b.stage_ms()
-            ts.append(sum(st[s] for s in stages))
-        return statistics.median(ts), b.info(0)
+            ts.append([sum(st.values()), sum(st[s] for s in FILL_STAGES), sum(st[s] for s in FFT_STAGES)])
+        return tuple(statistics.median(t) for t in zip(*ts)), b.info(0)
     finally:
         b.close()
+
+
+def _best(timed, default):
+    """The (times, schedule) of least total time; the planner's ``default``
+    schedule unless another is faster by more than MARGIN."""
+    best = min(timed)
+    for ms, sched in timed:
+        if sched == default and ms[0] <= (1.0 + MARGIN) * best[0][0]:
+            return ms, sched
+    return best
 
 
 def tune(db, req, reps=5, verbose=False):
@@ -241,12 +263,13 @@ def tune(db, req, reps=5, verbose=False):
     for w in tile_candidates(m_cap):
         r = copy.copy(base)
         r.tile_w = w
-        ms, _ = _time(db, r, FILL_STAGES, reps)
+        ms, _ = _time(db, r, reps)
         if ms is not None:
             fills.append((ms, w))
             if verbose:
-                print(f"  tile_w={w:4d}: fill {ms:.4f} ms", flush=True)
-    fill_ms, tile_w = min(fills) if fills else (float("nan"), int(info.tile_w))
+                print(f"  tile_w={w:4d}: {ms[0]:.4f} ms, fill {ms[1]:.4f}", flush=True)
+    default = int(info.tile_w)
+    (_, fill_ms, _), tile_w = _best(fills, default) if fills else ((0.0, float("nan"), 0.0), default)
     # 2) FFT schedule with that tile
     ffts = []
     for L, n1, generic in fft_candidates(nv):
@@ -254,16 +277,18 @@ def tune(db, req, reps=5, verbose=False):
         r.tile_w, r.fft_len, r.fft_n1 = tile_w, L, n1
         if generic:
             r.flags = int(r.flags) | _generic_flag()
-        ms, inf = _time(db, r, FFT_STAGES, reps)
+        ms, inf = _time(db, r, reps)
         if ms is None or (not generic and not inf.compiled_fft):
             continue
-        ffts.append((ms, L, n1, generic))
+        ffts.append((ms, (L, n1, generic)))
         if verbose:
-            print(f"  L={L:8d} n1={n1:5d} {'generic ' if generic else 'compiled'}: fft {ms:.4f} ms", flush=True)
+            print(f"  L={L:8d} n1={n1:5d} {'generic ' if generic else 'compiled'}: {ms[0]:.4f} ms, fft {ms[2]:.4f}",
+                  flush=True)
+    default = (int(info.fft_len), int(info.n1), not bool(info.compiled_fft))
     if ffts:
-        fft_ms, L, n1, generic = min(ffts)
+        (_, fill_ms, fft_ms), (L, n1, generic) = _best(ffts, default)
     else:
-        fft_ms, L, n1, generic = float("nan"), int(info.fft_len), int(info.n1), not bool(info.compiled_fft)
+        fft_ms, (L, n1, generic) = float("nan"), default
     entry = {"fft_len": int(L), "fft_n1": int(n1), "generic": bool(generic), "tile_w": int(tile_w),
              "fill_ms": fill_ms, "fft_ms": fft_ms, "candidates": len(fills) + len(ffts)}
     c = _load()
