@@ -68,16 +68,9 @@ def log(msg):
     print(f"[bench {time.strftime('%H:%M:%S')}] {msg}", file=sys.stderr, flush=True)
 
 
-def transform_len(info):
-    """Length the FFT passes run at: compiled passes take half of the planned
-    length unless it is the spectrum's own period (2 N_v)."""
-    L, n1, n2 = int(info.fft_len), int(info.n1), int(info.n2)
-    half = info.compiled_fft and L != 2 * int(info.n_v) and (n1 >= 512 or n2 >= 128)
-    return L // 2 if half else L
-
-
-def stage_bytes(n_lines, info, db):
-    """Algorithmic HBM bytes per launch of each kernel of one request.
+def stage_bytes(n_lines, info, db, L):
+    """Algorithmic HBM bytes per launch of each kernel of one request whose
+    passes run at length L (SpectrumBatch.pass_length).
 
     axis        : 12 B per scanned line (g_air, g_self, n_air f32) [+4 n_self] [+9 nu0 f64 + iso u8 with several
                   isotopologues]; the lines of whole blocks are replaced by their width candidates, 16 B each
@@ -89,13 +82,12 @@ def stage_bytes(n_lines, info, db):
     fft_a       : 4*R*(N_v+1) LDM read + 8*P*L packed-row spectra write
     fft_b       : 8*P*L read + 8*L write
     fft_c       : 8*L read + 4*N_v abscoeff write
-    with L the length the passes run at (transform_len) and R the rows that
-    move per column: M, or from P L = 2^22 on (rows of G-axis nodes beyond a
-    tile's reach are skipped) at least the two nodes its lines fall between.
+    with R the rows that move per column: M, or from P L = 2^22 on (rows of
+    G-axis nodes beyond a tile's reach are skipped) at least the two nodes its
+    lines fall between.
     """
     M = int(info.n_g * info.n_l)
     P = (M + 1) // 2
-    L = transform_len(info)
     V = int(info.n_v) + 1
     R = min(M, 2 * int(info.n_l)) if P * L >= 1 << 22 else M
     ns = 4 if db.has_nself else 0
@@ -285,6 +277,7 @@ def bench_single(args, workload):
     if inf.status:
         raise RuntimeError(f"device status {inf.status}")
     n_win = int(inf.line_end - inf.line_begin)
+    pass_len = batch.pass_length(0)[0]
     # 1) the timed steps: eager launches (or graph replays with --graph), no
     #    per-kernel events
     log(f"{workload}: timing {args.steps} steps")
@@ -318,7 +311,7 @@ def bench_single(args, workload):
         for _ in range(args.warmup):
             replay()
         other = {"graph_ms_per_step": round(timed_loop(replay, args.steps) * 1e3, 4)}
-    bytes_ = stage_bytes(n_win, inf, db)
+    bytes_ = stage_bytes(n_win, inf, db, pass_len)
     alg = step_alg_bytes(n_win, inf, db)
     dom = max(stages, key=stages.get)
     achieved = bytes_[dom] / (stages[dom] * 1e-3) / 1e9

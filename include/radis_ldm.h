@@ -130,11 +130,15 @@ typedef struct {
  * L = 2*N_v (radis/lbl/broadening.py:1900-1902, 2340-2346).  Without this
  * flag a transform longer than 2*N_v has its circular images corrected
  * (image-correction items in the fill launch), so the output is the L = 2*N_v
- * result whatever fft_len is.  The compiled passes then run at fft_len / 2,
- * a period just above N_v, and its images are corrected from a coarse
- * description (the result is the same L = 2*N_v one to FP32 rounding); an
+ * result whatever fft_len is; an
  * explicit fft_len must then be 2*N_v itself or leave a gap the correction
- * can span (about 0.5 % of L). */
+ * can span (about 0.5 % of L).
+ * Compiled passes of such a transform may run at fft_len / 2, a period just
+ * above N_v whose images are corrected from a coarse description; which
+ * requests do is the planner's choice by cost (radis_ldm_batch_pass_length).
+ * Never with this flag, fft_len = 2*N_v or RADIS_LDM_MIN_RMS, nor where the
+ * LDM is filled in row groups or the Gaussian (at 10,000 K or Tgas) reaches
+ * 1/64 of the gap fft_len / 2 - N_v. */
 #define RADIS_LDM_PERIOD_L 64
 
 /* Planned sizes of a request (filled by radis_ldm_batch_create / _info). */
@@ -226,6 +230,10 @@ int radis_ldm_batch_graph_replay(radis_ldm_batch *b, void *stream);
  * (gpu.py:372-374). */
 int radis_ldm_batch_info(radis_ldm_batch *b, int i, radis_ldm_request_info *info, void *stream);
 int radis_ldm_batch_workspace_bytes(const radis_ldm_batch *b, int64_t *bytes);
+/* Length that request i's FFT passes run at in the present layout: fft_len or
+ * half of it (RADIS_LDM_PERIOD_L above); shares (NULL, or host memory): the
+ * workgroups that pass B splits a row block's pairs over. */
+int radis_ldm_batch_pass_length(const radis_ldm_batch *b, int i, int64_t *length, int32_t *shares);
 void radis_ldm_batch_destroy(radis_ldm_batch *b);
 
 /* Device time per stage (axis, finalize, tile_bounds, fill, fft_a, fft_b,

@@ -164,6 +164,7 @@ _PROTOTYPES = {
     "radis_ldm_batch_graph_replay": (c_int, [c_void_p, c_void_p]),
     "radis_ldm_batch_info": (c_int, [c_void_p, c_int, POINTER(RequestInfo), c_void_p]),
     "radis_ldm_batch_workspace_bytes": (c_int, [c_void_p, POINTER(c_int64)]),
+    "radis_ldm_batch_pass_length": (c_int, [c_void_p, c_int, POINTER(c_int64), POINTER(c_int32)]),
     "radis_ldm_batch_destroy": (None, [c_void_p]),
     "radis_ldm_batch_enable_timing": (c_int, [c_void_p, c_int]),
     "radis_ldm_batch_stage_ms": (c_int, [c_void_p, POINTER(c_float)]),

@@ -1133,6 +1133,13 @@ int radis_ldm_batch_workspace_bytes(const radis_ldm_batch* b, int64_t* bytes) {
   return 0;
 }
 
+int radis_ldm_batch_pass_length(const radis_ldm_batch* b, int i, int64_t* length, int32_t* shares) {
+  if (!b || !length || i < 0 || i >= b->n) return fail(RADIS_LDM_EINVAL, "bad arguments");
+  *length = b->reqs[i].tL;
+  if (shares) *shares = b->reqs[i].n_share;
+  return 0;
+}
+
 int radis_ldm_batch_enable_timing(radis_ldm_batch* b, int enable) {
   if (!b) return fail(RADIS_LDM_EINVAL, "null batch");
   // the kernels' events exist from the first timed run on (32 of them created and

@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from ctypes import POINTER, byref, c_float, c_int64, c_uint8, c_void_p
+from ctypes import POINTER, byref, c_float, c_int32, c_int64, c_uint8, c_void_p
 
 import numpy as np
 
@@ -348,6 +348,14 @@ class SpectrumBatch:
         v = c_int64()
         check(self._lib.radis_ldm_batch_workspace_bytes(self._h, byref(v)))
         return int(v.value)
+
+    def pass_length(self, i):
+        """(length, shares): the length that request i's FFT passes run at,
+        its planned fft_len or half of it, and the workgroups that pass B
+        splits a row block's pairs over."""
+        n, s = c_int64(), c_int32()
+        check(self._lib.radis_ldm_batch_pass_length(self._h, int(i), byref(n), byref(s)))
+        return int(n.value), int(s.value)
 
     # -- conditions -------------------------------------------------------------
     # request fields fixed by the plan: the schedule and the flags that pick
