@@ -87,7 +87,8 @@ def test_a_budget_of_request_bytes_is_enough(nv):
         b = engine.SpectrumBatch(db, [req])
         got = b.results(b.run())[0]
         length, shares = b.pass_length(0)
-        assert shares > 2 and (length == b.info(0).fft_len or not kw)
+        # (run-time-sized passes walk every pair in one workgroup)
+        assert (shares > 2 if b.info(0).compiled_fft else shares == 1) and (length == b.info(0).fft_len or not kw)
         L = int(b.info(0).fft_len) if kw else None
         assert oracle.rel_peak_error(got, oracle.eq_abscoeff(lines.as_dict(), wmin, wmax, ws, T, p, 0.3, dx, dx, L=L)) <= TOL
         b.close()
