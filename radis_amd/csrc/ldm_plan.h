@@ -12,7 +12,6 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <thread>
 #include <vector>
 
@@ -115,6 +114,10 @@ struct FftPlan {
 // Sizes with compile-time-sized passes: n1 (passes A and C) and n2 (pass B).
 const int FC_N1[] = {256, 320, 384, 512, 640, 768, 1024};
 const int FC_N2[] = {64, 128, 256, 512, 1024, 2048};
+// tables by compiled size: n1 up to 1024 in steps of 64, the logarithm of n2 (half
+// lengths: n1 from 256, n2 from 32 up)
+const int FC_N1_SIZES = 17, FC_N2_SIZES = 12;
+int fc_n1_index(int n1) { return n1 >> 6; }
 // A compiled split is preferred while its length is within this factor of
 // the smallest generic (7-smooth) length: its passes run ~3x faster.
 const double FC_SLACK = 1.35;
@@ -990,7 +993,7 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
     for (int k = 0; k < 3; ++k) {
       const bool half = R.half && (k == 0 || (k == 1 && R.half_loss <= 0));
       if (half) t[k] += R.half_loss;
-      n1s[k] |= 1u << ((half ? R.tn1 : R.plan.n1) >> 6);
+      n1s[k] |= 1u << fc_n1_index(half ? R.tn1 : R.plan.n1);
       n2s[k] |= 1u << floor_log2(half ? R.tn2 : R.plan.n2);
     }
   }
@@ -998,26 +1001,29 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
   const int form = t[0] <= t[1] && t[0] <= t[2] ? 0 : t[1] <= t[2] ? 1 : 2;
   for (int i = 0; i < n; ++i)
     reqs[i].may_half = reqs[i].may_half && (form == 0 || (form == 1 && reqs[i].half_loss <= 0));
-  std::map<int, long long> cols_a, cols_c;  // compiled n1 -> wide column blocks of passes A and C
-  std::map<int, long long> blocks, images;  // compiled pass B class (N2) -> row blocks, image items of the launch
+  // by compiled size (fixed storage: planning allocates nothing): wide column
+  // blocks of passes A and C, row blocks of pass B and image items of the launch
+  long long cols_a[FC_N1_SIZES] = {}, cols_c[FC_N1_SIZES] = {}, blocks[FC_N2_SIZES] = {}, images[FC_N2_SIZES] = {};
   for (int i = 0; i < n; ++i) {
     Req& R = reqs[i];
     R.narrow_a = R.narrow_c = false;
     const int rc = plan_exec(R);
     if (rc) return rc;
     if (!R.plan.fc) continue;
-    cols_a[R.tn1] += (long long)((R.m_cap + 1) / 2) * (R.tn2 >> R.bX[0]);
-    cols_c[R.tn1] += R.tn2 >> R.bX[2];
-    blocks[R.tn2] += R.tn1 >> R.bX[1];
-    images[R.tn2] += image_items(R.n_cell);
+    const int a = fc_n1_index(R.tn1), b = floor_log2(R.tn2);
+    cols_a[a] += (long long)((R.m_cap + 1) / 2) * (R.tn2 >> R.bX[0]);
+    cols_c[a] += R.tn2 >> R.bX[2];
+    blocks[b] += R.tn1 >> R.bX[1];
+    images[b] += image_items(R.n_cell);
   }
   for (int i = 0; i < n; ++i) {
     Req& R = reqs[i];
     R.split_b = R.n_share = 1;
     R.share_in_y = false;
     if (!R.plan.fc) continue;
-    R.narrow_a = fc_narrow_a(R.tn1) && cols_a[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_A_NARROW_DIV);
-    R.narrow_c = fc_narrow_c(R.tn1) && cols_c[R.tn1] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_C_NARROW_DIV);
+    const int a = fc_n1_index(R.tn1), b = floor_log2(R.tn2);
+    R.narrow_a = fc_narrow_a(R.tn1) && cols_a[a] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_A_NARROW_DIV);
+    R.narrow_c = fc_narrow_c(R.tn1) && cols_c[a] < (long long)n_cu / (R.tn1 == 256 ? 1 : FC_C_NARROW_DIV);
     const int pairs = (R.m_cap + 1) / 2, rb = R.tn1 >> R.bX[1];
     // whole length: two shares, or more where Y is small (a share's chain of pairs
     // is what a lone small request waits for: 20,001 points, twelve pairs in two
@@ -1030,8 +1036,8 @@ int choose_split_b(Req* reqs, int n, int n_cu, bool lean = false) {
     // points x 84 rows, 848 items: one share 83.7 us, four 49.0; 255,001 points,
     // 546 items, room for three: 19.6, four 22.4)
     const long long places = (long long)FC_B_SPLIT_WGS_PER_CU * n_cu;
-    long long room = std::max(0ll, places - images[R.tn2]) / blocks[R.tn2];
-    if (room < 2) room = (places - std::min<long long>(images[R.tn2], n_cu)) / blocks[R.tn2];
+    long long room = std::max(0ll, places - images[b]) / blocks[b];
+    if (room < 2) room = (places - std::min<long long>(images[b], n_cu)) / blocks[b];
     int ns = (int)std::min<long long>(room, pairs / FC_B_SPLIT_MIN_PAIRS);
     const bool room_whole = (int64_t)pairs * R.plan.L * 8 <= FC_B_SPLIT_WHOLE_Y;
     ns = std::min(ns, R.half || room_whole ? std::min(FC_B_SPLIT_MAX, 2 * R.plan.n1 / rb) : 2);

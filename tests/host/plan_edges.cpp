@@ -6,15 +6,27 @@
 //   axis_groups width candidate blocks per workgroup from the whole launch's
 //   half_cost   half-length transforms where they cost the launch less
 //   image_room  pass B's shares beside many image items
+//   no_allocation  planning a lone request allocates nothing
 //   scratch     the no-allocation entry point's array holds what it held with
 //               the plain splits' tables
 //   bytes       the admission figure: at most one transform's buffers and a
 //               second partial spectrum, and no less than what batches of such
 //               requests lay out
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <new>
 
 #include "ldm_plan.h"
+
+long g_news = 0;  // allocations through operator new
+void* operator new(size_t n) {
+  ++g_news;
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -170,6 +182,38 @@ void image_room() {
   }
 }
 
+// What the no-allocation entry point plans with, plan to scratch layout.
+void no_allocation() {
+  radis_ldm_db db;
+  db.n = 5000000;
+  db.has_sky = true;
+  for (int64_t nv : {4000, 20001, 150001, 600001})
+    for (int m_cap : {1, 18, 144, 700})
+      for (int flags : {0, RADIS_LDM_MIN_RMS, RADIS_LDM_GENERIC_FFT}) {
+        const long before = g_news;
+        Req R;
+        R.r.Tgas = 1000.0;
+        R.r.flags = flags;
+        R.nv = nv;
+        R.delta_w = 0.002;
+        R.wg_hi = 0.01;
+        R.i0 = 1;
+        R.i1 = db.n;
+        R.m_cap = R.m_need = m_cap;
+        int64_t b = 0;
+        size_t work = 0;
+        NoallocLayout S;
+        int rc = plan_fft(nv, 0, R.plan, 0, !(flags & RADIS_LDM_GENERIC_FFT), false);
+        if (!rc) rc = choose_split_b(&R, 1, 256);
+        if (!rc) rc = layout_request(R, work);
+        const LdmItemPlan P = item_plan(db, R);
+        if (!rc) noalloc_layout(R, P, plan_items(P) + P.n_img, work, S);
+        if (!rc) rc = request_bytes(R, 256, b);
+        CHECK(rc == 0, "%s", g_err);
+        CHECK(g_news == before, "nv %lld, %d rows: %ld allocations", (long long)nv, m_cap, g_news - before);
+      }
+}
+
 // LDM, Y, a partial spectrum (two where pass B is split over two shares: four
 // pairs or more, and twice the row blocks fit four workgroups per CU), rows,
 // axis partials, correction table, fill items at the full tile width, tables.
@@ -304,7 +348,7 @@ void scratch() {
 }  // namespace
 
 int main(int argc, char** argv) {
-  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"half_cost", half_cost}, {"image_room", image_room}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
+  const struct { const char* name; void (*run)(); } sections[] = {{"wide_tile", wide_tile}, {"axis_groups", axis_groups}, {"half_cost", half_cost}, {"image_room", image_room}, {"no_allocation", no_allocation}, {"bytes", bytes}, {"scratch", scratch}, {"shares_in_y", shares_in_y}};
   for (const auto& s : sections)
     if (argc == 2 && !std::strcmp(argv[1], s.name)) {
       s.run();

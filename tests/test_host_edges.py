@@ -55,3 +55,7 @@ def test_half_length_by_its_cost(section):
 
 def test_shares_beside_image_items(section):
     section("image_room")
+
+
+def test_planning_a_lone_request_allocates_nothing(section):
+    section("no_allocation")
