@@ -260,17 +260,16 @@ int build_layout(radis_ldm_batch* b) {
   }
   // --- twiddle tables, deduplicated by size
   std::map<int, size_t> sub_off;
-  std::map<int64_t, size_t> l_off;
+  std::map<std::pair<int64_t, bool>, size_t> l_off;  // (length, FP64)
   size_t twsz = 0;
   sub_off[LDM_WRAP_LC] = twsz;  // the image correction's transform
   twsz = align_up(twsz + (size_t)LDM_WRAP_LC * 8, 256);
   for (Req& R : b->reqs) {
     for (int N : {R.tn1, R.tn2})
       if (!sub_off.count(N)) { sub_off[N] = twsz; twsz = align_up(twsz + (size_t)N * 8, 256); }
-    if (!l_off.count(R.tL)) {
-      l_off[R.tL] = twsz;
-      const size_t nhi = (size_t)((R.tL + 1023) >> LDM_TW_LO_BITS);
-      twsz = align_up(twsz + (nhi + 1024) * 8, 256);
+    if (!l_off.count({R.tL, R.plan.fc})) {
+      l_off[{R.tL, R.plan.fc}] = twsz;
+      twsz = align_up(twsz + twl_bytes(R), 256);
     }
   }
   if (b->ctx->budget > 0 && b->ctx->in_use + (int64_t)(total + twsz) > b->ctx->budget)
@@ -288,9 +287,9 @@ int build_layout(radis_ldm_batch* b) {
   // point builds its tables the same way)
   std::vector<LdmTwiddles> tabs;
   for (auto& kv : sub_off)
-    tabs.push_back({(float2*)((char*)b->twmem + kv.second), nullptr, nullptr, kv.first, 0, 0});
+    tabs.push_back({(float2*)((char*)b->twmem + kv.second), nullptr, nullptr, kv.first, 0, 0, false});
   for (auto& kv : l_off)
-    tabs.push_back({nullptr, nullptr, (float2*)((char*)b->twmem + kv.second), 0, 0, (long long)kv.first});
+    tabs.push_back({nullptr, nullptr, (char*)b->twmem + kv.second, 0, 0, (long long)kv.first.first, kv.first.second});
   for (size_t at = 0; at < tabs.size(); at += LDM_TW_TABLES) {
     const size_t n = std::min<size_t>(LDM_TW_TABLES, tabs.size() - at);
     LdmTwiddleSet set{};
@@ -307,8 +306,7 @@ int build_layout(radis_ldm_batch* b) {
     char* base = (char*)b->twmem;
     R.tw1 = (const float2*)(base + sub_off[R.tn1]);
     R.tw2 = (const float2*)(base + sub_off[R.tn2]);
-    R.twl_hi = (const float2*)(base + l_off[R.tL]);
-    R.twl_lo = R.twl_hi + (size_t)((R.tL + 1023) >> LDM_TW_LO_BITS);
+    set_twl(R, base + l_off[{R.tL, R.plan.fc}]);
     R.tw_wrap = (const float2*)(base + sub_off[LDM_WRAP_LC]);
   }
   // --- work items (FFT passes grouped by kernel variant), per request in
@@ -1230,21 +1228,18 @@ int radis_ldm_run_noalloc(radis_ldm_ctx* ctx, const radis_ldm_db* db, const radi
   if (S.bytes > (size_t)RADIS_LDM_NOALLOC_BYTES + SCRATCH_TABLES)
     return fail(RADIS_LDM_ERANGE, "request needs %zu bytes of scratch, above the %lld of radis_ldm_run_noalloc "
                                   "(use a batch)", S.bytes, (long long)RADIS_LDM_NOALLOC_BYTES);
-  const long long nhi = (R.tL + 1023) >> LDM_TW_LO_BITS;
   char* const base = ctx->scratch;
   float2* tw1 = (float2*)(base + S.tw1);
   float2* tw2 = (float2*)(base + S.tw2);
-  float2* twl = (float2*)(base + S.twl);
   R.tw1 = tw1;
   R.tw2 = tw2;
-  R.twl_hi = twl;
-  R.twl_lo = twl + nhi;
+  set_twl(R, base + S.twl);
   R.tw_wrap = (float2*)(base + S.twc);
   LdmJob J;
   fill_job(*db, R, base + S.work, out_dev, J);
   hipStream_t s = (hipStream_t)stream;
-  const LdmTwiddles wrap{(float2*)(base + S.twc), nullptr, nullptr, LDM_WRAP_LC, 0, 0};
-  const LdmTwiddles tw{tw1, tw2, twl, R.tn1, R.tn2, (long long)R.tL};
+  const LdmTwiddles wrap{(float2*)(base + S.twc), nullptr, nullptr, LDM_WRAP_LC, 0, 0, false};
+  const LdmTwiddles tw{tw1, tw2, base + S.twl, R.tn1, R.tn2, (long long)R.tL, R.plan.fc};
   const long long n_set = n_items + wrap.total() + tw.total();  // one element per thread: below 2^31 in the scratch array
   hipLaunchKernelGGL(k_setup, dim3((unsigned)(1 + (n_set + 255) / 256)), dim3(256), 0, s, J, (LdmJob*)(base + S.job), P,
                      (int4*)(base + S.items), n_items, wrap, tw);

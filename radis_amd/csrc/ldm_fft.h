@@ -32,12 +32,17 @@ __device__ __forceinline__ gptr<T> glb(T* p) {
 // a native 2-vector: the float2 class's own copy and assignment operators
 // take generic pointers)
 typedef float gf2 __attribute__((ext_vector_type(2)));
+typedef double gd2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float gld(const float* p, unsigned byte_off) {
   return *(gptr<const float>)((const char*)p + byte_off);
 }
 __device__ __forceinline__ float2 gld(const float2* p, unsigned byte_off) {
   const gf2 v = *(gptr<const gf2>)((const char*)p + byte_off);
   return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ double2 gld(const double2* p, unsigned byte_off) {
+  const gd2 v = *(gptr<const gd2>)((const char*)p + byte_off);
+  return make_double2(v.x, v.y);
 }
 __device__ __forceinline__ int gld(const int* p, unsigned byte_off) {
   return *(gptr<const int>)((const char*)p + byte_off);

@@ -18,6 +18,7 @@
 #include "ldm_fft.h"
 #include "ldm_image.h"
 #include "ldm_kernels.h"
+#include "ldm_twiddle.h"
 
 constexpr int fc_odd(int n) { return n % 3 == 0 ? 3 : (n % 5 == 0 ? 5 : 1); }
 constexpr int fc_log2(int n) { return n <= 1 ? 0 : 1 + fc_log2(n >> 1); }
@@ -280,29 +281,11 @@ __device__ __forceinline__ void fc_load_tw_stages(float2* __restrict__ s_tw, con
   }
 }
 
-// Twiddles W_L^(m * (j0 + s*DS + q*DQ)) of one thread's last-stage outputs
-// (s < IT thread passes, q < R legs; m fixed per thread) as
-// base * A^s * C^q from three table values, so an output costs one complex
-// product instead of two table gathers.  The powers of C are products at most
-// log2(R) deep (a chain of R - 1 took as many operations and 15 roundings at
-// R = 16).  Every exponent is below L.
-template <int IT, int R>
-struct TwProg {
-  float2 ws[IT], wq[R];
-  __device__ __forceinline__ void init(const LdmJob& J, long long m, long long j0, long long DS, long long DQ) {
-    set(twiddle_L(J, m * j0), twiddle_L(J, m * DS), twiddle_L(J, m * DQ));
-  }
-  // from the three table values W^(m j0), W^(m DS), W^(m DQ)
-  __device__ __forceinline__ void set(float2 base, float2 A, float2 C) {
-    ws[0] = base;
-#pragma unroll
-    for (int s = 1; s < IT; ++s) ws[s] = cmul(ws[s - 1], A);
-    wq[0] = make_float2(1.0f, 0.0f);
-#pragma unroll
-    for (int q = 1; q < R; ++q) wq[q] = q == 1 ? C : cmul(wq[q / 2], wq[q - q / 2]);
-  }
-  __device__ __forceinline__ float2 operator()(int s, int q) const { return cmul(ws[s], wq[q]); }
-};
+// the table halves of W_L^e (e < L) of the compiled passes
+__device__ __forceinline__ void twiddle_halves(const LdmJob& J, unsigned e, double2 (&h)[2]) {
+  h[0] = gld(J.twd_hi, 16u * (e >> LDM_TW_LO_BITS));
+  h[1] = gld(J.twd_lo, 16u * (e & ((1u << LDM_TW_LO_BITS) - 1)));
+}
 
 // ---------------------------------------------------------------------------
 // Pass A with N1 fixed (see k_fft_a): B = fc_cols_a(N1) columns per workgroup.
@@ -337,6 +320,14 @@ __global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob
   // has consumed them, so they are in flight during the LDS stages and the
   // stores.
   float2 v[SH::IT0][SH::R0];
+  // The twiddle progression's factors W^(m DS) and W^(m DQ) of the tile's B
+  // columns, in LDS by the first 2 B threads: 144 rows of 600,001 points took 111
+  // us with six 16-byte gathers per thread (107 from FP32 tables), so 104.
+  // Not in narrow tiles, which take one block each, nor in transforms of two
+  // stages, without a barrier between the write and the use.
+  constexpr bool AC = T >= FC_T_A && fc_nstages(N1) > 2;
+  static_assert(2 * B <= T, "a thread per column and factor");
+  __shared__ double2 s_ac[AC ? 2 * B : 1];
   // issue the loads of block idx into v; false (for the whole workgroup)
   // when the block has no work
   auto fetch = [&](int idx) -> bool {
@@ -401,30 +392,34 @@ __global__ __launch_bounds__(T, T >= FC_T_A ? 4 : 2) void k_fft_a_c(const LdmJob
     const int N2 = J.tn2, n2_0 = it.z * B;
     float2* Y = J.ybuf + (long long)it.y * J.tL;
     // output k1 of this thread's last-stage element (s, q): j0 + s*(T/B) + q*NS;
-    // the table halves of the progression's three factors load now and are
-    // multiplied out just before the last stage
-    float2 twr[3][2];
-    {
-      const unsigned m = n2_0 + (threadIdx.x & (B - 1));
-      const unsigned ex[3] = {m * (threadIdx.x >> LB), m * (T >> LB), m * NSL};  // < L <= 2^21
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        twr[t][0] = gld(J.twl_hi, 8u * (ex[t] >> LDM_TW_LO_BITS));
-        twr[t][1] = gld(J.twl_lo, 8u * (ex[t] & ((1u << LDM_TW_LO_BITS) - 1)));
-      }
+    // the table halves of its base (and factors) load now and are multiplied out
+    // just before the last stage
+    const int b = threadIdx.x & (B - 1);
+    const unsigned m = n2_0 + b;
+    double2 twr[AC ? 1 : 3][2], twc[2];
+    twiddle_halves(J, m * (threadIdx.x >> LB), twr[0]);  // < L <= 2^21
+    if constexpr (AC) {
+      if (threadIdx.x < 2 * B) twiddle_halves(J, m * (threadIdx.x < B ? T >> LB : NSL), twc);
+    } else {
+      twiddle_halves(J, m * (T >> LB), twr[1]);
+      twiddle_halves(J, m * NSL, twr[2]);
     }
     TwProg<SH::ITL, SH::RL> tw;
     auto before_last = [&] {
-      tw.set(cmul(twr[0][0], twr[0][1]), cmul(twr[1][0], twr[1][1]), cmul(twr[2][0], twr[2][1]));
+      if constexpr (AC) tw.set(cmul64(twr[0][0], twr[0][1]), s_ac[b], s_ac[B + b]);
+      else tw.set(cmul64(twr[0][0], twr[0][1]), cmul64(twr[1][0], twr[1][1]), cmul64(twr[2][0], twr[2][1]));
     };
     auto ld = [&](int s, int q, int) -> float2 { return v[s][q]; };
     auto st = [&](int s, int q, int e, float2 z) {
       const unsigned k1 = (unsigned)e >> LB, n2 = n2_0 + (e & (B - 1));
       // byte offsets are below 8 L <= 2^24
-      gst(Y, 8u * (k1 * (unsigned)N2 + n2), cmul(z, tw(s, q)));
+      gst(Y, 8u * (k1 * (unsigned)N2 + n2), cmul(z, cmul(tw.ws[s], tw.wq[q])));
     };
     bool next = false;
-    auto prefetch = [&] { next = fetch(idx + gridDim.x); };
+    auto prefetch = [&] {
+      if (AC && threadIdx.x < 2 * B) s_ac[threadIdx.x] = cmul64(twc[0], twc[1]);
+      next = fetch(idx + gridDim.x);
+    };
     // first stage from v, last stage straight to Y with the W_L twiddle
     fc_fft_io<N1, B, T, true, true, true, true>(buf, s_tw, ld, st, prefetch, before_last);
     live = next;
@@ -689,10 +684,17 @@ __global__ __launch_bounds__(FC_T_B, N2 >= 256 ? 4 : 2) void k_fft_b_c(const Ldm
   float2* Bo = J.bbuf + J.share_at[share] + (long long)k1_0 * N2;
   // output n2 of this thread's last-stage element (s, q): j0 + s*(T/B) + q*NS, row k1 fixed
   TwProg<SH::ITL, SH::RL> tw;
-  tw.init(J, k1_0 + (threadIdx.x & (B - 1)), threadIdx.x >> LB, T >> LB, NSL);
+  {
+    const unsigned m = k1_0 + (threadIdx.x & (B - 1));
+    double2 h[3][2];
+    twiddle_halves(J, m * (threadIdx.x >> LB), h[0]);  // < L <= 2^21
+    twiddle_halves(J, m * (T >> LB), h[1]);
+    twiddle_halves(J, m * NSL, h[2]);
+    tw.set(cmul64(h[0][0], h[0][1]), cmul64(h[1][0], h[1][1]), cmul64(h[2][0], h[2][1]));
+  }
   auto st_out = [&](int s, int q, int e, float2 z) {
     const int b = e & (B - 1), n2 = e >> LB;
-    gst(Bo, 8u * (unsigned)(b * N2 + n2), cmulc(z, tw(s, q)));
+    gst(Bo, 8u * (unsigned)(b * N2 + n2), cmulc(z, cmul(tw.ws[s], tw.wq[q])));
   };
   FcNone none;
   auto nop = [] {};

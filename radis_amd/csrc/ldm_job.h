@@ -285,6 +285,7 @@ struct LdmJob {
   unsigned long long wl_min_bits, wl_max_bits, wg_min_bits, wg_max_bits;
   int status;
   int sparse_g;                  // 1: rows of G-axis nodes beyond a tile's reach are neither written nor read (LdmAxes::tlo)
+  const double2 *twd_hi, *twd_lo;  // twl_hi and twl_lo in FP64 (compiled passes; those are then null)
 };
 
 // Device-computed LDM axes of one request (written by k_finalize).

@@ -156,6 +156,7 @@ struct Req {
   size_t off_ldm = 0, off_y = 0, off_b = 0, off_b2 = 0, off_rows = 0, off_axp = 0, off_wrap = 0;
   size_t off_share = 0, off_img = 0, off_mom = 0, off_free = 0;  // partial spectra; half: correction values, tile moments, unused from here
   const float2 *tw1 = nullptr, *tw2 = nullptr, *twl_hi = nullptr, *twl_lo = nullptr, *tw_wrap = nullptr;
+  const double2 *twd_hi = nullptr, *twd_lo = nullptr;
 };
 
 // Host arrays of a line list that go to the device with its columns: the
@@ -803,6 +804,8 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.tw2 = R.tw2;
   J.twl_hi = R.twl_hi;
   J.twl_lo = R.twl_lo;
+  J.twd_hi = R.twd_hi;
+  J.twd_lo = R.twd_lo;
   J.tw_wrap = R.tw_wrap;
   J.wl_min_bits = ~0ull;
   J.wl_max_bits = 0ull;
@@ -1175,6 +1178,22 @@ __host__ __device__ inline int4 plan_item(const LdmItemPlan& P, int i) {
 
 namespace {
 
+// The two-level W_L table (set_twl): FP64 for the compiled passes, FP32 for the
+// run-time-sized ones, whose lengths go to 2^23.
+long long twl_hi_len(const Req& R) { return (R.tL + (1 << LDM_TW_LO_BITS) - 1) >> LDM_TW_LO_BITS; }
+size_t twl_bytes(const Req& R) { return (size_t)(twl_hi_len(R) + (1 << LDM_TW_LO_BITS)) * (R.plan.fc ? 16 : 8); }
+void set_twl(Req& R, const void* table) {
+  R.twl_hi = R.twl_lo = nullptr;
+  R.twd_hi = R.twd_lo = nullptr;
+  if (R.plan.fc) {
+    R.twd_hi = (const double2*)table;
+    R.twd_lo = R.twd_hi + twl_hi_len(R);
+  } else {
+    R.twl_hi = (const float2*)table;
+    R.twl_lo = R.twl_hi + twl_hi_len(R);
+  }
+}
+
 // Bytes that a batch of this one request allocates, at most; in a batch of
 // several it takes no more: more points there only favour the half length, more
 // row blocks fewer shares.
@@ -1187,7 +1206,8 @@ int request_bytes(Req& R, int n_cu, int64_t& bytes) {
   if (rc) return rc;
   // work items and job table (16 B per item, a few per tile and block)
   bytes = (int64_t)total + (int64_t)R.wide_tiles * R.fill_groups * 16;
-  // twiddle tables, plus alignment slack
+  // twiddle tables, plus slack for alignment, the image correction's table and the
+  // second half of FP64 ones (at most 24 KB)
   bytes += (int64_t)(R.plan.n1 + R.plan.n2 + 1024 + (R.plan.L >> LDM_TW_LO_BITS) + 1) * 8 + 64 * 1024;
   return 0;
 }
@@ -1269,7 +1289,7 @@ int plan_one(const radis_ldm_db& db, const radis_ldm_request& rq, Req& R) {
 // requests add to the tables: narrow fill tiles, pass A blocks and several pass B
 // shares (at most a few items per CU each, 16 B), a width item per candidate block
 // (LDM_SKY_WGS of them) and the tile ranges of the axes: up to 19 KB counted over
-// 10^6 plans.
+// 10^6 plans; and for the FP64 half of the W_L table, up to 24 KB.
 #define SCRATCH_TABLES (64 << 10)
 struct NoallocLayout {
   size_t job, axes, res, items, tw1, tw2, twl, twc, work, bytes;
@@ -1291,7 +1311,7 @@ void noalloc_layout(const Req& R, const LdmItemPlan& P, int n_items, size_t work
   S.items = items_in_work ? 0 : take(items_bytes);
   S.tw1 = take((size_t)R.plan.n1 * 8);
   S.tw2 = take((size_t)R.plan.n2 * 8);
-  S.twl = take((size_t)(((R.tL + 1023) >> LDM_TW_LO_BITS) + 1024) * 8);
+  S.twl = take(twl_bytes(R));
   S.twc = take((size_t)LDM_WRAP_LC * 8);
   S.work = take(work);
   if (items_in_work) S.items = S.work + R.off_free;

@@ -8,18 +8,20 @@
 // Element i of the twiddle tables of one size set: W_n1^e (e < n1), W_n2^e
 // (e < n2) and the two-level W_L table: hi[q] = W_L^((q * 1024) mod L),
 // q < ceil(L / 1024), then lo[e] = W_L^e, e < 1024.  W_N^e = exp(-2 pi i e / N),
-// evaluated as sincospi(-2 e / N) in FP64 and rounded to FP32.  Null tables are
-// skipped.
+// evaluated as sincospi(-2 e / N) in FP64 and rounded to FP32 (the W_L table of
+// the compiled passes stays FP64: twl64).  Null tables are skipped.
 struct LdmTwiddles {
-  float2 *tw1, *tw2, *twl;
+  float2 *tw1, *tw2;
+  void* twl;
   int n1, n2;
   long long L;
+  bool twl64;
   __host__ __device__ long long nhi() const { return (L + (1 << LDM_TW_LO_BITS) - 1) >> LDM_TW_LO_BITS; }
   __host__ __device__ long long total() const {
     return (tw1 ? n1 : 0) + (tw2 ? n2 : 0) + (twl ? nhi() + (1 << LDM_TW_LO_BITS) : 0);
   }
   __device__ void put(long long k) const {
-    float2* dst;
+    float2* dst = nullptr;
     double e, N;
     if (tw1 && k < n1) {
       dst = tw1 + k; e = (double)k; N = (double)n1;
@@ -29,14 +31,15 @@ struct LdmTwiddles {
         dst = tw2 + k; e = (double)k; N = (double)n2;
       } else {
         if (tw2) k -= n2;
-        dst = twl + k;
+        if (!twl64) dst = (float2*)twl + k;
         N = (double)L;
         e = k < nhi() ? (double)((k << LDM_TW_LO_BITS) % L) : (double)(k - nhi());
       }
     }
     double sn, cs;
     sincospi(-2.0 * e / N, &sn, &cs);
-    *dst = make_float2((float)cs, (float)sn);
+    if (dst) *dst = make_float2((float)cs, (float)sn);
+    else ((double2*)twl)[k] = make_double2(cs, sn);
   }
 };
 

@@ -266,7 +266,7 @@ void bytes() {
               int64_t tw = LDM_WRAP_LC * 8;
               for (Req& Q : reqs) {
                 CHECK(layout_request(Q, total) == 0, "%s", g_err);
-                tw += ((int64_t)Q.tn1 + Q.tn2 + 1024 + (Q.tL + 1023) / 1024) * 8 + 3 * 256;
+                tw += ((int64_t)Q.tn1 + Q.tn2) * 8 + (int64_t)twl_bytes(Q) + 3 * 256;
               }
               CHECK((int64_t)total + tw <= sum, "nv %lld, %d rows, %d requests: %lld B of %lld", (long long)nv, m_cap, n,
                     (long long)total + tw, (long long)sum);
