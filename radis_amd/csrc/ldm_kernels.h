@@ -973,31 +973,40 @@ __device__ __forceinline__ void line_terms(const LineConst& C, const LineRaw& r,
 // sits on the common path (only atomics), so atomics retire in the background.
 // ---------------------------------------------------------------------------
 
-// GROUPED: the LDM is taller than one tile's LDS (J.fill_groups > 1 for some
-// request of the launch); item y = tile * fill_groups + g, and the workgroup
-// keeps rows [g * fill_rows, g * fill_rows + MR) only: each of its 8 atomics
-// checks its corner's row.  A request with fill_groups = 1 has one group of
-// every row.  HALF: some request of the launch runs half-length transforms.
 // The G-axis nodes [l0, l1] whose rows a tile's lines can reach (LdmAxes::tlo,
 // thi; every node in the grid's first tile and its last two).  With one isotopologue
 // the Gaussian width goes with nu0, so a tile meets two or three of the nodes
 // whatever N_G is: writing and reading the other rows' zeros was five sixths of
 // the LDM's traffic at N_G = 12, a third at N_G = 3.
+// The ranges load before the tile's lines: loads return in order, and ballots behind
+// those waited for every line in flight (500,002 points x 27 rows in 32-point tiles:
+// 83.8 us, 74.3 with every row written, so 77.8; 600,001 x 144 rows 190.4 -> 183.5).
 struct GNodes {
   int l0, l1;
-  __device__ __forceinline__ GNodes(const LdmJob& J, const LdmAxes& A, int ng, int tile) : l0(0), l1(ng - 1) {
-    if (!J.sparse_g || ng <= 2 || tile == 0 || tile >= J.n_tiles - 2) return;  // uniform
-    const int lane = threadIdx.x & 63;
+  bool some;  // uniform: not every node
+  int2 r0, r1;
+  __device__ __forceinline__ GNodes(const LdmJob& J, const LdmAxes& A, int ng, int tile)
+      : l0(0), l1(ng - 1), some(J.sparse_g && ng > 2 && tile != 0 && tile < J.n_tiles - 2) {
+    if (!some) return;
+    const int l = threadIdx.x & 63;
+    r0 = make_int2(A.tlo[min(l, ng - 1)], A.thi[min(l, ng - 1)]);
+    if (ng > 64) r1 = make_int2(A.tlo[min(l + 64, ng - 1)], A.thi[min(l + 64, ng - 1)]);
+  }
+  __device__ __forceinline__ void find(int ng, int tile) {
+    if (!some) return;
+    const int l = threadIdx.x & 63;
     l0 = l1 = -1;
-    for (int base = 0; base < ng; base += 64) {
-      const int l = base + lane;
-      const bool in = l < ng;
-      const unsigned long long lo = __ballot(in && A.tlo[in ? l : 0] <= tile), hi = __ballot(in && A.thi[in ? l : 0] >= tile);
+    auto half = [&](int base, int2 r) {
+      const bool in = base + l < ng;
+      const unsigned long long lo = __ballot(in && r.x <= tile), hi = __ballot(in && r.y >= tile);
       if (lo) l1 = base + 63 - __builtin_clzll(lo);
       if (l0 < 0 && hi) l0 = base + __builtin_ctzll(hi);
-    }
+    };
+    half(0, r0);
+    if (ng > 64) half(64, r1);
   }
 };
+static_assert(LDM_MAX_AX == 128, "two nodes per lane");
 // The columns of a pair of rows that the fill wrote: [0, w0), [a, a + len) and
 // [w1, V).  Without a branch, so that a thread's loads stay in flight together.
 static_assert(LDM_AX_PAIRS == 256, "k_finalize: a thread per pair");
@@ -1025,6 +1034,11 @@ struct PairColumns {
   }
 };
 
+// GROUPED: the LDM is taller than one tile's LDS (J.fill_groups > 1 for some
+// request of the launch); item y = tile * fill_groups + g, and the workgroup
+// keeps rows [g * fill_rows, g * fill_rows + MR) only: each of its 8 atomics
+// checks its corner's row.  A request with fill_groups = 1 has one group of
+// every row.  HALF: some request of the launch runs half-length transforms.
 template <bool NONEQ, bool PLAIN, bool GROUPED, bool HALF>
 __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, const int4 it, const LdmDb& db,
                                           double* acc) {
@@ -1038,6 +1052,8 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
   const long long k_lo = (long long)tile * W;
   long long k_hi = k_lo + W;
   if (k_hi > J.v) k_hi = J.v;
+  // the G-axis nodes this tile's lines can reach: the flush writes their rows
+  GNodes act(J, A, ng, tile);
   const LineConst C(J, A, db);
   const LineCols cols(db);
   const unsigned lo = (unsigned)(J.i0 + it.z), hi = (unsigned)(J.i0 + it.w);  // written by tile_bounds
@@ -1072,8 +1088,7 @@ __device__ __forceinline__ void fill_tile(const LdmJob& J, const LdmAxes& A, con
     for (int e = threadIdx.x; e < n2; e += blockDim.x) a2[e] = make_double2(0.0, 0.0);
     if ((n & 1) && threadIdx.x == 0) acc[n - 1] = 0.0;
   }
-  // the G-axis nodes this tile's lines can reach: the flush writes their rows
-  const GNodes act(J, A, ng, tile);
+  act.find(ng, tile);
   lds_barrier();
   const int wlen = (int)(k_hi - k_lo);
   const int sg = nl * Wp;
