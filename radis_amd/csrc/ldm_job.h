@@ -243,7 +243,7 @@ struct LdmJob {
   int n_share, split_b;
   unsigned share_inv;            // 2^16 / n_share: share s takes the pairs from P s share_inv >> 16
   long long share_at[FC_B_SPLIT_MAX];  // (share_in_y: written by k_finalize)
-  int share_in_y;                // 1: bbuf is Y
+  int share_in_y;                // shares whose spectra lie in Y (bbuf is Y), or 0
   // half-length transforms: per cell IMG_NODES values of the correction
   double* img_u;                 // [n_cell][IMG_NODES]
   int cell_tiles, n_cell;        // fill tiles per cell, cells

@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void k_finalize(LdmJob* __restrict__ jobs, Ldm
   if (J.half)  // the image correction is accumulated by the pass B launch
     for (int e = threadIdx.x; e < J.n_cell * IMG_NODES; e += blockDim.x) J.img_u[e] = 0.0;
   const double nu_a = ends ? db.nu0[i0] : 0.0, nu_b = ends ? db.nu0[i1 - 1] : 0.0;
-  const int n_share = J.share_in_y ? J.n_share : 0;
+  const int n_share = J.share_in_y;
   // Q(Tref)/Q(T) of the slots with a partition-function spline (the fill
   // reads these after this kernel): calc_linestrength_eq's Qref/Q,
   // radis/lbl/base.py:2605-2697

@@ -772,7 +772,7 @@ void fill_job(const radis_ldm_db& db, const Req& R, char* work, float* out, LdmJ
   J.ybuf = (float2*)(work + R.off_y);
   J.bbuf = (float2*)(work + R.off_share);
   J.share_inv = 65536u / (unsigned)R.n_share;
-  J.share_in_y = R.share_in_y ? 1 : 0;
+  J.share_in_y = R.share_in_y ? R.n_share : 0;
   const long long share_stride = R.half || R.n_share > 2 || R.share_in_y ? R.tL : (long long)(R.off_b2 - R.off_b) / 8;
   for (int i = 0; i < R.n_share; ++i) J.share_at[i] = i * share_stride;
   J.mom = R.half ? (float*)(work + R.off_mom) : nullptr;
