@@ -64,7 +64,7 @@ static_assert(LDM_AX_CHUNK == LDM_SKY_BLOCK, "a partial block is one scan chunk"
 #define FC_CAP_B 2048  // complex elements of a pass B tile
 #define FC_T_B 256
 #define FC_B_SPLIT_MAX 4  // most workgroups per pass B row block
-#define FC_C_SUM (1 << 20)  // pass C launch-class flag: B is the sum of two pass B shares
+#define FC_C_SUM (1 << 20)  // pass C launch-class flag: B is the sum of pass B's shares
 #define FC_B_ROWS_LDS 512  // rows whose lineshape coefficients pass B stages in LDS (more: read from global memory)
 // Half-length transforms (ldm_image.h): the compiled passes run at half the
 // planned length L, and the circular images that a period of L/2 < 2 N_v
